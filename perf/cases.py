@@ -114,6 +114,7 @@ def prepare(case, seed):
         scf = SCF(S, precision=case["precision"])
         scf.initial_potential()
         rho = scf.rho * (1.0 + 0.05 * np.cos(np.linspace(0.0, 20.0 + seed % 7, S.nn)))
+        rho *= scf.rho.sum() / rho.sum()        # a density step keeps the electron count
         return {"case": case, "scf": scf, "rho": rho, "ebs": -7.0, "eent": -0.3}
     sq = SpectralQuadrature(S, precision=case["precision"])
     if case["kind"] in ("forces", "adjoint", "tangent"):
