@@ -24,12 +24,10 @@ void cheb_step(sqg_ctx *c, int B, T *x, T *y, T *out, bool first)
     launch_zmarch<T, MODE_CHEB>(c, B, Z, -1, 0.0);
 }
 
-int batch_images(sqg_ctx *c, int B)
+int batch_images(sqg_ctx *c, const std::vector<int> &nodes)
 {
-    const int *dn = c->node_list.as<int>();
     HIPCHK(hipMemsetAsync(c->flags.p, 0, 16 * sizeof(int), c->st));
-    (void)dn;
-    return node_images(c, B);
+    return node_images(c, nodes.data(), (int)nodes.size());
 }
 
 // Sign of rho_pc and d rho_pc/d lambda per node at the last lambda_f
@@ -83,7 +81,8 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     std::vector<int> nodes(B);
     for (int i = 0; i < B; ++i) nodes[i] = z0 * n * n + i;
     HIPCHK(hipMemcpyAsync(c->node_list.p, nodes.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));
-    batch_images(c, B);
+    st = batch_images(c, nodes);
+    if (st) return st;
     HIPCHK(c->adj.ensure((size_t)P.nvec * vl * sizeof(T)));
     T *base = c->adj.as<T>();
     auto pair = [&](int j, int w) { return base + (size_t)(2 * j + w) * vl; };
@@ -158,19 +157,18 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     return ovf ? SQG_E_OVERFLOW : SQG_OK;
 }
 
-// d rho along dV (adj_in) for the B nodes starting at node s0, into adj_out.
+// d rho along dV (adj_in) for the given nodes, into adj_out.
 template <typename T>
-int tangent_batch(sqg_ctx *c, int s0, int B)
+int tangent_batch(sqg_ctx *c, const std::vector<int> &nodes)
 {
-    const int K2 = c->p.npl / 2, q4 = c->p.npl / 4;
+    const int B = (int)nodes.size(), K2 = c->p.npl / 2, q4 = c->p.npl / 4;
     const size_t M3 = c->M3, vl = (size_t)B * M3;
     const int cidx = (c->p.nloc * c->M + c->p.nloc) * c->M + c->p.nloc;
     int st = ensure_batch(c, B);
     if (st) return st;
-    std::vector<int> nodes(B);
-    for (int i = 0; i < B; ++i) nodes[i] = s0 + i;
     HIPCHK(hipMemcpyAsync(c->node_list.p, nodes.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));
-    batch_images(c, B);
+    st = batch_images(c, nodes);
+    if (st) return st;
     HIPCHK(c->adj.ensure(6 * vl * sizeof(T)));
     HIPCHK(c->adj_rec.ensure((size_t)B * (K2 + 1) * 3 * sizeof(double)));
     T *tr[3], *dr[3];

@@ -78,7 +78,8 @@ struct sqg_ctx {
     // batch buffers
     int Bcap = 0;
     DBuf X, Y, X2, Y2, NLv, s, node_list, list, list_cnt, flags;   // X2, Y2: Lanczos ping-pong
-    DBuf glist, glist_cnt;         // group image lists (NG slots per group)
+    DBuf gst, glist, glist_cnt;    // first slot of each group, group image lists
+    int ng = 0;                    // groups of the current batch
     int gl_max = 0;                // longest group list of the current batch
     int projr_R = 0;               // k_projr register slots for the batch (0: k_projs instead)
     DBuf lred, aa, bb, dq, eq, lmin, lmax, lmin_prev, lmax_prev, lchg, cnt, done, ca, ib, bprev;
@@ -152,20 +153,49 @@ Geo make_geo(const sqg_ctx *c, const int *dnodes, const int *ddone)
 // half of the cube's rows (two workgroups per node cube).
 int zmarch_threads(int M) { return (zhalf_rows(M, 0) * M + 63) / 64 * 64; }
 
-// Visiting order of the FD nodes: 4x4x2 bricks, so that workgroups that run
-// at the same time (consecutive batch slots) march overlapping cubes and
-// share Veff, projector tables and ELL entries in the caches.
+// Visiting order of the FD nodes: bricks of up to 4x4x2 nodes, so that
+// workgroups that run at the same time (consecutive batch slots) march
+// overlapping cubes and share Veff, projector tables and ELL entries in the
+// caches.  Each axis is cut into near-equal runs (of up to 4, 2 and 2 nodes in
+// x, y and z; a brick is two y runs), so a grid side that 4 does not divide
+// has no thin last brick.  The nodes of one (x run, y run, z) are consecutive:
+// the up to 4x2x1 block that one projection workgroup takes.
+struct NodeOrder {
+    int n;
+    std::vector<int> rx, ry, rz;   // run of each coordinate
+    explicit NodeOrder(int n_) : n(n_), rx(runs(n_, 4)), ry(runs(n_, 2)), rz(runs(n_, 2)) {}
+    static std::vector<int> runs(int n, int len)
+    {
+        const int m = (n + len - 1) / len;
+        std::vector<int> r(n);
+        for (int c = 0; c < m; ++c)
+            for (int i = (int)((long)c * n / m); i < (int)((long)(c + 1) * n / m); ++i) r[i] = c;
+        return r;
+    }
+    // sort key: brick z, y, x; then z, the brick's y run, y, x
+    unsigned long key(int node) const
+    {
+        const int x = node % n, y = (node / n) % n, z = node / (n * n);
+        const unsigned long m = (unsigned long)n + 1;
+        unsigned long k = rz[z];
+        for (unsigned long f : {(unsigned long)(ry[y] / 2), (unsigned long)rx[x], (unsigned long)z}) k = k * m + f;
+        return (k * 2 + (ry[y] & 1)) * (m * m) + (unsigned long)y * m + x;
+    }
+    void sort(std::vector<int> &nodes) const
+    {
+        std::vector<std::pair<unsigned long, int>> k(nodes.size());
+        for (size_t i = 0; i < nodes.size(); ++i) k[i] = {key(nodes[i]), nodes[i]};
+        if (std::is_sorted(k.begin(), k.end())) return;
+        std::sort(k.begin(), k.end());
+        for (size_t i = 0; i < nodes.size(); ++i) nodes[i] = k[i].second;
+    }
+};
+
 std::vector<int> node_order(int n)
 {
-    const int bx = 4, by = 4, bz = 2;
-    std::vector<int> seq;
-    seq.reserve((size_t)n * n * n);
-    for (int z0 = 0; z0 < n; z0 += bz)
-        for (int y0 = 0; y0 < n; y0 += by)
-            for (int x0 = 0; x0 < n; x0 += bx)
-                for (int z = z0; z < std::min(z0 + bz, n); ++z)
-                    for (int y = y0; y < std::min(y0 + by, n); ++y)
-                        for (int x = x0; x < std::min(x0 + bx, n); ++x) seq.push_back((z * n + y) * n + x);
+    std::vector<int> seq((size_t)n * n * n);
+    for (size_t i = 0; i < seq.size(); ++i) seq[i] = (int)i;
+    NodeOrder(n).sort(seq);
     return seq;
 }
 
@@ -184,8 +214,6 @@ int ensure_batch(sqg_ctx *c, int B)
     HIPCHK(c->node_list.ensure((size_t)B * sizeof(int)));
     HIPCHK(c->list.ensure((size_t)B * LCAP * sizeof(int)));
     HIPCHK(c->list_cnt.ensure((size_t)B * sizeof(int)));
-    HIPCHK(c->glist.ensure((size_t)((B + NG - 1) / NG) * GLCAP * sizeof(int)));
-    HIPCHK(c->glist_cnt.ensure((size_t)((B + NG - 1) / NG) * sizeof(int)));
     HIPCHK(c->flags.ensure(16 * sizeof(int)));
     HIPCHK(c->lred.ensure((size_t)B * ZHALF * 4 * sizeof(double)));
     for (DBuf *d : {&c->aa, &c->bb, &c->dq, &c->eq}) HIPCHK(d->ensure((size_t)B * S * sizeof(double)));
@@ -258,6 +286,7 @@ PArgs<T> pargs(sqg_ctx *c, const int *dn, const int *dd, const T *V)
     A.n_ip = std::max(c->n_ip, 1);
     A.list = c->list.as<int>();
     A.list_cnt = c->list_cnt.as<int>();
+    A.gst = c->gst.as<int>();
     A.glist = c->glist.as<int>();
     A.glist_cnt = c->glist_cnt.as<int>();
     A.img_type = c->img_type.as<int>();
@@ -297,24 +326,74 @@ ProjrShape projr_shape(const sqg_ctx *c, size_t ts)
     return {8, 0, ts == 4 ? 2 : 1, mfma};
 }
 
-// k_projr's slab capacity per plane and member: the union plane of a 4x2
-// (NM = 8) or 2x2 (NM = 4) block of cubes, or one cube, with rows padded to a
-// pitch congruent to the box side modulo 32 (as k_projr pads them).
-int projr_pu(const sqg_ctx *c, const ProjrShape &ps)
+// LDS values per plane and member of a staged block of ux x uy points: rows
+// padded to a pitch congruent to the box side modulo 32 (as k_projr and
+// k_projm pad them), k_projm's member stride congruent to 8.
+int projr_slab(const sqg_ctx *c, const ProjrShape &ps, int ux, int uy)
 {
     int wbox = 0;
     for (int t = 0; t < c->n_typ; ++t)
         if (c->h_nproj[t] > 0) wbox = 2 * c->h_nlocc[t] + 1;
-    auto upitch = [&](int u) { return u + (((wbox - u) % 32) + 32) % 32; };
-    auto slab = [&](int u) { return ps.mfma ? u + (((8 - u) % 32) + 32) % 32 : u; };
-    const int ux = ps.nm == 8 ? c->M + 3 : c->M + 1, uy = c->M + 1;
-    return std::max(slab(upitch(ux) * uy), slab(upitch(c->M) * c->M));
+    const int u = (ux + (((wbox - ux) % 32) + 32) % 32) * uy;
+    return ps.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
 }
 
-// Image lists of the B nodes in node_list (per node and per group of NG
-// slots); sets gl_max and projr_R.  Overflow goes to flags[0].
-int node_images(sqg_ctx *c, int B)
+// k_projr's slab capacity: the union plane of a 4x2 block of cubes or one cube.
+int projr_pu(const sqg_ctx *c, const ProjrShape &ps)
 {
+    return std::max(projr_slab(c, ps, c->M + 3, c->M + 1), projr_slab(c, ps, c->M, c->M));
+}
+
+// k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
+int projs_pu(const sqg_ctx *c) { return (c->M + 3) * (c->M + 3); }
+
+// Cuts B slots into groups of up to NG consecutive ones whose cubes the
+// staged projection kernels can walk together: the union plane fits the slab
+// capacity of every kernel that may run on the batch, and the cubes are at
+// most one plane apart in z.  A run ends where the next node is too far away
+// (a brick's edge, a gap in the caller's list): walking such members one
+// after the other in one workgroup, as unions that do not fit would need, is
+// several times slower: with runs of 8 slots cut anywhere, a density step on a
+// 15^3 LiH grid (25^3 cubes) took 534 ms and on a 10^3 Al grid (17^3) 44.6 ms,
+// against 155 and 15.2 ms.
+std::vector<int> make_groups(const sqg_ctx *c, const int *nodes, int B)
+{
+    const int n = c->p.n, M = c->M;
+    const ProjrShape shapes[2] = {projr_shape(c, c->split() ? 4 : c->real_size()), projr_shape(c, 8)};
+    const int nsh = c->split() ? 2 : 1;
+    auto fits = [&](int dx, int dy, int dz) {
+        if (dz > 1 || (M + dx) * (M + dy) > projs_pu(c)) return false;
+        for (int i = 0; i < nsh; ++i)
+            if (shapes[i].nm && projr_slab(c, shapes[i], M + dx, M + dy) > projr_pu(c, shapes[i])) return false;
+        return true;
+    };
+    std::vector<int> gst{0};
+    int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+    for (int b = 0; b < B; ++b) {
+        const int r[3] = {nodes[b] % n, (nodes[b] / n) % n, nodes[b] / (n * n)};
+        const int cnt = b - gst.back();
+        int l[3], h[3];
+        for (int d = 0; d < 3; ++d) {
+            l[d] = cnt ? std::min(lo[d], r[d]) : r[d];
+            h[d] = cnt ? std::max(hi[d], r[d]) : r[d];
+        }
+        if (cnt && (cnt == NG || !fits(h[0] - l[0], h[1] - l[1], h[2] - l[2]))) {
+            gst.push_back(b);
+            for (int d = 0; d < 3; ++d) l[d] = h[d] = r[d];
+        }
+        for (int d = 0; d < 3; ++d) { lo[d] = l[d]; hi[d] = h[d]; }
+    }
+    gst.push_back(B);
+    return gst;
+}
+
+// Image lists of the B nodes in node_list (per node and per group) on the
+// groups gst; sets ng, gl_max and projr_R.  Overflow goes to flags[0].
+int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst)
+{
+    const int ng = (int)gst.size() - 1;
+    c->ng = ng;
+    HIPCHK(hipMemcpyAsync(c->gst.p, gst.data(), gst.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
     LArgs L{};
     L.g = make_geo(c, c->node_list.as<int>(), nullptr);
     L.n_img = c->n_img;
@@ -325,6 +404,8 @@ int node_images(sqg_ctx *c, int B)
     L.list = c->list.as<int>();
     L.list_cnt = c->list_cnt.as<int>();
     L.overflow = c->flags.as<int>();
+    L.gst = c->gst.as<int>();
+    L.ng = ng;
     L.glist = c->glist.as<int>();
     L.glist_cnt = c->glist_cnt.as<int>();
     // the projection shapes of the phases that will run on these lists (both
@@ -333,19 +414,18 @@ int node_images(sqg_ctx *c, int B)
     const int nsh = c->split() ? 2 : 1;
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)1, 0);
     hipLaunchKernelGGL(k_node_images, dim3((B + 127) / 128), dim3(128), 0, c->st, L, B);
-    const int ng = (B + NG - 1) / NG;
     bool any_nm = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
         const ProjrShape &ps = shapes[i];
         LArgs Li = L;
         if (ps.nm) {
             Li.pr_bad = c->flags.as<int>() + 4;
-            Li.pr_nw = PROJR_NT / 64; Li.pr_sz = ps.sz; Li.pr_pu = projr_pu(c, ps); Li.pr_mfma = ps.mfma;
+            Li.pr_nw = PROJR_NT / 64; Li.pr_sz = ps.sz;
             any_nm = true;
             any_mfma |= ps.mfma != 0;
         }
         // a second launch rebuilds the same group lists and adds its slot plan
-        if (i == 0 || ps.nm) hipLaunchKernelGGL(k_group_images, dim3((ng + 63) / 64), dim3(64), 0, c->st, Li, B);
+        if (i == 0 || ps.nm) hipLaunchKernelGGL(k_group_images, dim3((ng + 63) / 64), dim3(64), 0, c->st, Li);
     }
     std::vector<int> gc(ng + 1);
     HIPCHK(hipMemcpyAsync(gc.data(), c->glist_cnt.p, (size_t)ng * sizeof(int), hipMemcpyDeviceToHost, c->st));
@@ -365,6 +445,16 @@ int node_images(sqg_ctx *c, int B)
     return SQG_OK;
 }
 
+// Groups and image lists of the B nodes in node_list (nodes: their host copy).
+int node_images(sqg_ctx *c, const int *nodes, int B)
+{
+    const std::vector<int> gst = make_groups(c, nodes, B);
+    HIPCHK(c->gst.ensure(gst.size() * sizeof(int)));
+    HIPCHK(c->glist.ensure((gst.size() - 1) * GLCAP * sizeof(int)));
+    HIPCHK(c->glist_cnt.ensure((gst.size() - 1) * sizeof(int)));
+    return image_lists(c, B, gst);
+}
+
 // LDS bytes of one k_nlapplyg workgroup (loc table, row offsets, NG values per row)
 size_t nlapplyg_lds(const sqg_ctx *c)
 {
@@ -379,12 +469,11 @@ void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
     if (shg <= 160 * 1024) {
         NGArgs<T> N{};
         N.g = A.g; N.nl = A.nl; N.nlv = A.nlv;
-        N.glist = c->glist.as<int>(); N.glist_cnt = c->glist_cnt.as<int>();
+        N.gst = c->gst.as<int>(); N.glist = c->glist.as<int>(); N.glist_cnt = c->glist_cnt.as<int>();
         N.img_type = c->img_type.as<int>(); N.nproj = c->nproj.as<int>(); N.ip_base = c->ip_base.as<int>();
-        N.B = B;
         auto fn = N.nl.ip16 ? k_nlapplyg<T, true> : k_nlapplyg<T, false>;
         if (shg > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shg);
-        hipLaunchKernelGGL(fn, dim3((B + NG - 1) / NG), dim3(512), shg, c->st, N);
+        hipLaunchKernelGGL(fn, dim3(c->ng), dim3(512), shg, c->st, N);
         return;
     }
     const size_t shm = (size_t)std::max(c->n_ip, 1) * sizeof(double);
@@ -393,57 +482,55 @@ void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
     hipLaunchKernelGGL(fn, dim3(B), dim3(512), shm, c->st, A);
 }
 
-template <typename T, int MAXP, int FORMED, int SZ, int NT, int NPU, int NM>
-void projs_go(sqg_ctx *c, dim3 grid, size_t shm, const PArgs<T> &P)
+template <typename T, int MAXP, int FORMED, int SZ, int NT, int NPU>
+void projs_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 {
-    auto fn = k_projs<T, MAXP, FORMED, SZ, NT, NPU, NM>;
+    auto fn = k_projs<T, MAXP, FORMED, SZ, NT, NPU>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(grid.x * (NG / NM)), dim3(NT), shm, c->st, P);
+    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(NT), shm, c->st, P);
 }
 
-template <typename T, int FORMED, int SZ, int NM>
-void projs_np(sqg_ctx *c, dim3 grid, size_t shs, const PArgs<T> &P, int npu)
+template <typename T, int FORMED, int SZ>
+void projs_np(sqg_ctx *c, size_t shs, const PArgs<T> &P, int npu)
 {
     constexpr int NT = 512;
-    if (npu == 1) projs_go<T, 1, FORMED, SZ, NT, 1, NM>(c, grid, shs, P);
-    else if (npu == 3) projs_go<T, 4, FORMED, SZ, NT, 3, NM>(c, grid, shs, P);
-    else projs_go<T, 4, FORMED, SZ, NT, 4, NM>(c, grid, shs, P);
+    if (npu == 1) projs_go<T, 1, FORMED, SZ, NT, 1>(c, shs, P);
+    else if (npu == 3) projs_go<T, 4, FORMED, SZ, NT, 3>(c, shs, P);
+    else projs_go<T, 4, FORMED, SZ, NT, 4>(c, shs, P);
 }
 
-// Staged projections (k_projs, all NG members of a group per workgroup):
-// planes per slab (sz) and the largest union plane (pu) staged at once.
-// Returns false when not even a single cube plane fits in LDS.
+// Staged projections (k_projs, all members of a group per workgroup) with the
+// deepest slab (planes staged at once) that fits the LDS.  Returns false when
+// not even a single union plane fits.
 template <typename T, int FORMED>
-bool launch_projs(sqg_ctx *c, dim3 grid, PArgs<T> &P, int mp)
+bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
 {
     constexpr int D = sizeof(T) == 4 ? 4 : 2;   // deep slab (planes)
     const size_t sa = ((size_t)std::max(c->gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16;
     // projector values are loaded and summed for npu of the mp slots
     const int npu = mp == 1 ? 1 : c->max_nproj == 3 ? 3 : 4;
-    for (int pu : {(c->M + 3) * (c->M + 3), c->M2}) {
-        for (int sz : {D, D / 2}) {
-            const size_t shs = sa + (size_t)pu * NG * sizeof(T) * sz;
-            if (shs > 160 * 1024) continue;
-            P.pu = pu;
-            if (sz == 4) projs_np<T, FORMED, 4, NG>(c, grid, shs, P, npu);
-            else if (sz == 2) projs_np<T, FORMED, 2, NG>(c, grid, shs, P, npu);
-            else projs_np<T, FORMED, 1, NG>(c, grid, shs, P, npu);
-            return true;
-        }
+    P.pu = projs_pu(c);
+    for (int sz : {D, D / 2, 1}) {
+        const size_t shs = sa + (size_t)P.pu * NG * sizeof(T) * sz;
+        if (shs > 160 * 1024) continue;
+        if (sz == 4) projs_np<T, FORMED, 4>(c, shs, P, npu);
+        else if (sz == 2) projs_np<T, FORMED, 2>(c, shs, P, npu);
+        else projs_np<T, FORMED, 1>(c, shs, P, npu);
+        return true;
     }
     return false;
 }
 
-template <typename T, int FORMED, int SZ, int NM, int R>
-void projr_go(sqg_ctx *c, dim3 grid, size_t shm, const PArgs<T> &P)
+template <typename T, int FORMED, int SZ, int R>
+void projr_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 {
-    auto fn = k_projr<T, FORMED, SZ, PROJR_NT, NM, R, PROJR_RPI>;
+    auto fn = k_projr<T, FORMED, SZ, PROJR_NT, R, PROJR_RPI>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(grid.x * (NG / NM)), dim3(PROJR_NT), shm, c->st, P);
+    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(PROJR_NT), shm, c->st, P);
 }
 
 template <typename T, int FORMED>
-bool launch_projr(sqg_ctx *c, dim3 grid, PArgs<T> &P)
+bool launch_projr(sqg_ctx *c, PArgs<T> &P)
 {
     const ProjrShape ps = projr_shape(c, sizeof(T));
     const size_t sa = ((size_t)std::max(c->gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16;
@@ -457,14 +544,14 @@ bool launch_projr(sqg_ctx *c, dim3 grid, PArgs<T> &P)
         if (ps.mfma) {
             auto fn = k_projm<T, FORMED, SZ, PROJR_NT, PROJM_SLOTS>;
             if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-            hipLaunchKernelGGL(fn, grid, dim3(PROJR_NT), shm, c->st, P);
+            hipLaunchKernelGGL(fn, dim3(c->ng), dim3(PROJR_NT), shm, c->st, P);
             return true;
         }
     }
     if (ps.mfma) return false;
-    if (c->projr_R == 5) projr_go<T, FORMED, SZ, 8, 5>(c, grid, shm, P);
-    else if (c->projr_R == 10) projr_go<T, FORMED, SZ, 8, 10>(c, grid, shm, P);
-    else projr_go<T, FORMED, SZ, 8, 16>(c, grid, shm, P);
+    if (c->projr_R == 5) projr_go<T, FORMED, SZ, 5>(c, shm, P);
+    else if (c->projr_R == 10) projr_go<T, FORMED, SZ, 10>(c, shm, P);
+    else projr_go<T, FORMED, SZ, 16>(c, shm, P);
     return true;
 }
 
@@ -481,13 +568,10 @@ void launch_proj(sqg_ctx *c, int B, const PArgs<T> &A, int which = -1, double al
     }
     if (c->n_ip > 0) {
         PArgs<T> P = A;
-        P.B = B;
-        const dim3 grid((B + NG - 1) / NG);
-        if (c->projr_R && launch_projr<T, FORMED>(c, grid, P)) goto apply;
-        // staged projections (k_projs) with the deepest slab whose planes
-        // (a union of a 4x4 footprint, else a single cube plane) fit in LDS
+        const dim3 grid(c->ng);
+        if (c->projr_R && launch_projr<T, FORMED>(c, P)) goto apply;
         const int mp = c->max_nproj <= 1 ? 1 : c->max_nproj <= 4 ? 4 : 0;
-        if (mp && launch_projs<T, FORMED>(c, grid, P, mp)) goto apply;
+        if (mp && launch_projs<T, FORMED>(c, P, mp)) goto apply;
         if (c->max_nproj <= 1)
             hipLaunchKernelGGL((k_projg<T, 1, FORMED>), grid, dim3(256), 0, c->st, P);
         else if (c->max_nproj <= 4)
@@ -649,14 +733,14 @@ int lanczos_batch(sqg_ctx *c, int B, long *passes_out)
 // Without lanczos the bounds of the last density step are reused.
 // TL: the stored type of the Lanczos passes, T: of the Chebyshev steps.
 template <typename TL, typename T>
-int run_batch(sqg_ctx *c, int B, long *passes_out, bool lanczos)
+int run_batch(sqg_ctx *c, const int *nodes, int B, long *passes_out, bool lanczos)
 {
     const int *dn = c->node_list.as<int>();
     int *flags = c->flags.as<int>();
     HIPCHK(hipMemsetAsync(flags, 0, 16 * sizeof(int), c->st));
     // image lists
     {
-        const int st = node_images(c, B);
+        const int st = node_images(c, nodes, B);
         if (st) return st;
     }
     const size_t vlen = (size_t)B * c->M3;
@@ -787,7 +871,7 @@ int moments_for_nodes(sqg_ctx *c, const int *nodes, int count, long *passes, int
         int st = ensure_batch(c, B);
         if (st) return st;
         HIPCHK(hipMemcpyAsync(c->node_list.p, nodes + done_n, (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));
-        st = run_batch<TL, T>(c, B, passes, lanczos);
+        st = run_batch<TL, T>(c, nodes + done_n, B, passes, lanczos);
         if (st) return st;
         if (lanczos)
             hipLaunchKernelGGL(k_scatter_batch, dim3((B + 127) / 128), dim3(128), 0, c->st, B,
@@ -801,8 +885,12 @@ int moments_for_nodes(sqg_ctx *c, const int *nodes, int count, long *passes, int
     return SQG_OK;
 }
 
-int moments_dispatch(sqg_ctx *c, const int *nodes, int count, long *passes, int cap = 0, bool lanczos = true)
+int moments_dispatch(sqg_ctx *c, const int *list, int count, long *passes, int cap = 0, bool lanczos = true)
 {
+    // results are kept by node, so the list is visited in brick order
+    std::vector<int> order(list, list + count);
+    NodeOrder(c->p.n).sort(order);
+    const int *nodes = order.data();
     if (cap <= 0) cap = choose_batch(c, count);
     if (c->p.precision == SQG_MIXED) return moments_for_nodes<float, float>(c, nodes, count, passes, cap, lanczos);
     if (c->split()) return moments_for_nodes<float, double>(c, nodes, count, passes, cap, lanczos);
@@ -916,7 +1004,7 @@ int forces_batch(sqg_ctx *c, int B, const int *hnodes, std::vector<double> &rec)
     int *flags = c->flags.as<int>();
     HIPCHK(hipMemsetAsync(flags, 0, 16 * sizeof(int), c->st));
     {
-        const int st = node_images(c, B);
+        const int st = node_images(c, hnodes, B);
         if (st) return st;
     }
     const size_t vlen = (size_t)B * c->M3;
@@ -1373,7 +1461,7 @@ int sqg_hsub_apply_batch(sqg_ctx *c, const double *veff, const int *nodes, int n
     HIPCHK(hipMemcpy(tmp.p, v, len * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(hipMemsetAsync(c->flags.p, 0, 16 * sizeof(int), c->st));
     const int *dn = c->node_list.as<int>();
-    st = node_images(c, nb);
+    st = node_images(c, nodes, nb);
     if (st) return st;
     auto run = [&](auto tag) -> int {
         using T = decltype(tag);
@@ -1402,9 +1490,9 @@ int sqg_hsub_apply_batch(sqg_ctx *c, const double *veff, const int *nodes, int n
 // own allocations; nothing here allocates or frees).
 struct ScratchView {
     sqg_ctx *c;
-    DBuf *bufs[11];
-    void *saved_p[11];
-    size_t saved_b[11];
+    DBuf *bufs[12];
+    void *saved_p[12];
+    size_t saved_b[12];
     int n = 0;
     size_t off = 0;
     explicit ScratchView(sqg_ctx *c_) : c(c_) {}
@@ -1421,12 +1509,12 @@ struct ScratchView {
     }
 };
 
-// Scratch bytes the allocation-free H v of nb nodes needs (per-call buffers
-// rounded to 256 bytes each).
-size_t noalloc_bytes(const sqg_ctx *c, int nb)
+// Scratch bytes the allocation-free H v of nb nodes in ng groups needs
+// (per-call buffers rounded to 256 bytes each, without the group table).
+size_t noalloc_bytes(const sqg_ctx *c, int nb, size_t ng)
 {
     auto r = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t rs = c->real_size(), len = (size_t)nb * c->M3, ng = (size_t)(nb + NG - 1) / NG;
+    const size_t rs = c->real_size(), len = (size_t)nb * c->M3;
     size_t t = r(nb * sizeof(int)) + r((size_t)nb * LCAP * sizeof(int)) + r(nb * sizeof(int)) +
                r(ng * GLCAP * sizeof(int)) + r(ng * sizeof(int)) + r(16 * sizeof(int)) +
                r((size_t)nb * std::max(c->n_ip, 1) * sizeof(double)) + r(len * rs);
@@ -1434,23 +1522,24 @@ size_t noalloc_bytes(const sqg_ctx *c, int nb)
     return t;
 }
 
-
-int sqg_hsub_apply_batch_noalloc(sqg_ctx *c, const double *d_veff, const int *nodes, int nb, const double *d_v,
-                                 double *d_hv)
+// H v of nb nodes in the scratch array.  Nodes too far apart to share groups
+// need more list space than full groups do: such a batch runs as two halves.
+static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int nb, const double *d_v, double *d_hv)
 {
-    if (!c || !d_veff || !nodes || nb < 0 || !d_v || !d_hv) return SQG_E_ARG;
-    if (!c->geom) return SQG_E_NOGEOM;
-    if (!c->scratch_ptr) return SQG_E_HIP;
-    for (int i = 0; i < nb; ++i)
-        if (nodes[i] < 0 || nodes[i] >= c->nn) return SQG_E_ARG;
-    if (nb == 0) return SQG_OK;
-    if (noalloc_bytes(c, nb) > (size_t)SQG_NOALLOC_SCRATCH_BYTES) return SQG_E_OVERFLOW;
-    HIPCHK(hipSetDevice(c->p.device));
-    const size_t len = (size_t)nb * c->M3, rs = c->real_size(), ng = (size_t)(nb + NG - 1) / NG;
+    const std::vector<int> gst = make_groups(c, nodes, nb);
+    const size_t len = (size_t)nb * c->M3, rs = c->real_size(), ng = gst.size() - 1;
+    if (noalloc_bytes(c, nb, ng) + (gst.size() * sizeof(int) + 255) / 256 * 256 > (size_t)SQG_NOALLOC_SCRATCH_BYTES) {
+        if (nb == 1) return SQG_E_OVERFLOW;
+        const int h = nb / 2;
+        const int st = noalloc_piece(c, d_veff, nodes, h, d_v, d_hv);
+        if (st) return st;
+        return noalloc_piece(c, d_veff, nodes + h, nb - h, d_v + (size_t)h * c->M3, d_hv + (size_t)h * c->M3);
+    }
     ScratchView V(c);
     V.put(c->node_list, nb * sizeof(int));
     V.put(c->list, (size_t)nb * LCAP * sizeof(int));
     V.put(c->list_cnt, nb * sizeof(int));
+    V.put(c->gst, gst.size() * sizeof(int));
     V.put(c->glist, ng * GLCAP * sizeof(int));
     V.put(c->glist_cnt, ng * sizeof(int));
     V.put(c->flags, 16 * sizeof(int));
@@ -1465,7 +1554,7 @@ int sqg_hsub_apply_batch_noalloc(sqg_ctx *c, const double *d_veff, const int *no
     // flags start at zero (a fill kernel, not a memset node)
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>(), (size_t)16, 0);
     HIPCHK(hipMemcpyAsync(c->node_list.p, nodes, nb * sizeof(int), hipMemcpyHostToDevice, c->st));
-    int st = node_images(c, nb);
+    int st = image_lists(c, nb, gst);
     if (st) return st;
     const int *dn = c->node_list.as<int>();
     auto run = [&](auto tag) {
@@ -1495,6 +1584,21 @@ int sqg_hsub_apply_batch_noalloc(sqg_ctx *c, const double *d_veff, const int *no
     HIPCHK(hipMemcpyAsync(ovf4, c->flags.p, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     return (ovf4[0] | ovf4[2] | ovf4[3]) ? SQG_E_OVERFLOW : SQG_OK;
+}
+
+int sqg_hsub_apply_batch_noalloc(sqg_ctx *c, const double *d_veff, const int *nodes, int nb, const double *d_v,
+                                 double *d_hv)
+{
+    if (!c || !d_veff || !nodes || nb < 0 || !d_v || !d_hv) return SQG_E_ARG;
+    if (!c->geom) return SQG_E_NOGEOM;
+    if (!c->scratch_ptr) return SQG_E_HIP;
+    for (int i = 0; i < nb; ++i)
+        if (nodes[i] < 0 || nodes[i] >= c->nn) return SQG_E_ARG;
+    if (nb == 0) return SQG_OK;
+    // the limit callers see: nb nodes in full groups
+    if (noalloc_bytes(c, nb, (size_t)(nb + NG - 1) / NG) > (size_t)SQG_NOALLOC_SCRATCH_BYTES) return SQG_E_OVERFLOW;
+    HIPCHK(hipSetDevice(c->p.device));
+    return noalloc_piece(c, d_veff, nodes, nb, d_v, d_hv);
 }
 
 int sqg_forces_nonlocal(sqg_ctx *c, double *f)
@@ -1654,9 +1758,10 @@ int sqg_tangent_veff(sqg_ctx *c, const double *dV, int fixed_n, double *drho)
     const int cap = std::min(choose_batch_adj(c, nn, 6 * (size_t)c->M3 * c->real_size() +
                                                      (size_t)(c->p.npl / 2 + 1) * 3 * sizeof(double)),
                              65535);
+    const std::vector<int> all = node_order(c->p.n);
     for (int s0 = 0; s0 < nn; s0 += cap) {
-        const int B = std::min(cap, nn - s0);
-        st = c->p.precision == SQG_MIXED ? tangent_batch<float>(c, s0, B) : tangent_batch<double>(c, s0, B);
+        const std::vector<int> nodes(all.begin() + s0, all.begin() + std::min(s0 + cap, nn));
+        st = c->p.precision == SQG_MIXED ? tangent_batch<float>(c, nodes) : tangent_batch<double>(c, nodes);
         if (st) return st;
     }
     HIPCHK(hipMemcpy(drho, c->adj_out.p, (size_t)nn * sizeof(double), hipMemcpyDeviceToHost));

@@ -4,7 +4,7 @@
 //   vectors   X, Y      [B][M^3]  M = 2 nloc + 1, each node cube z-major (z, y, x)
 //   projections s       [B][n_ip] FP64, one value per image-projector
 //   image lists         [B][LCAP] image ids whose rc-cube meets the node cube
-//   group image lists   [ceil(B/NG)][GLCAP] the same for NG consecutive slots
+//   group image lists   [groups][GLCAP] the same for a group of up to NG consecutive slots
 //   Veff                [n^3] periodic grid (x fastest), read through wrapped indices
 //   projector ELL       over the extended grid (n + 2 nloc)^3: per point the
 //                       (image-projector id, U value) pairs that cover it
@@ -579,76 +579,18 @@ struct PArgs {
     const int *nlocc, *nproj;     // per type
     const double *inv_denom;      // [type][16]
     const double *ca, *ib;        // LANCZOS: projects v = (V - ca V2) * ib
-    const int *glist, *glist_cnt; // group image lists (k_projg, k_projs)
-    int B;                        // slots in the batch (k_projg, k_projs)
-    int pu;                       // k_projs: largest union plane (points) staged at once
+    const int *gst;               // [groups + 1] first slot of each group
+    const int *glist, *glist_cnt; // group image lists
+    int pu;                       // staged kernels: LDS values per plane and member
 };
 
-// s[b][ip] = <U_ip, v_b>/Denom over the intersection of the image's rc-cube
-// and node b's cube (nonlocal.cpp:149-171).  One wave per image.  With
-// FORMED, v is the Lanczos vector formed from the two stored vectors with the
-// same rounding as the z-march forms it, so that the projections always
-// belong to the vector being multiplied (a recursion on projections would
-// amplify rounding by |alpha/beta| per pass).
-template <typename T, int MAXP, int FORMED>
-__global__ void __launch_bounds__(256) k_proj(PArgs<T> A)
-{
-    const Geo &G = A.g;
-    const int b = blockIdx.x;
-    if (G.done && G.done[b]) return;
-    const int node = G.node_list[b];
-    const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2;
-    const int ni = node % n, nj = (node / n) % n, nk = node / (n * n);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwave = blockDim.x >> 6;
-    const int cnt = A.list_cnt[b];
-    const T *__restrict__ V = A.V + (size_t)b * G.M3;
-    const T *__restrict__ V2 = FORMED ? A.V2 + (size_t)b * G.M3 : nullptr;
-    double *sb = A.s + (size_t)b * A.n_ip;
-    T cab = 0, ibb = 1;
-    if (FORMED) { cab = (T)A.ca[b]; ibb = (T)A.ib[b]; }
-    for (int li = wave; li < cnt; li += nwave) {
-        const int J = A.list[(size_t)b * LCAP + li];
-        const int t = A.img_type[J];
-        const int nc = A.nlocc[t], np = A.nproj[t], w = 2 * nc + 1;
-        const int cx = A.img_nn[3 * J], cy = A.img_nn[3 * J + 1], cz = A.img_nn[3 * J + 2];
-        const int lox = max(cx - nc, ni - nloc), hix = min(cx + nc, ni + nloc);
-        const int loy = max(cy - nc, nj - nloc), hiy = min(cy + nc, nj + nloc);
-        const int loz = max(cz - nc, nk - nloc), hiz = min(cz + nc, nk + nloc);
-        const int bx = hix - lox + 1, by = hiy - loy + 1;
-        const int area = bx * by;
-        const int w2 = w * w, w3 = w2 * w;
-        const T *U = A.udv + A.udv_off[J];
-        double acc[MAXP];
-#pragma unroll
-        for (int i = 0; i < MAXP; ++i) acc[i] = 0.0;
-        for (int a = lane; a < area; a += 64) {
-            const int iy = a / bx, ix = a - iy * bx;
-            const int gx = lox + ix, gy = loy + iy;
-            const int cidx = (gy - nj + nloc) * M + (gx - ni + nloc);
-            const int ridx = (gy - cy + nc) * w + (gx - cx + nc);
-            for (int gz = loz; gz <= hiz; ++gz) {
-                const size_t o = (size_t)(gz - nk + nloc) * M2 + cidx;
-                double v;
-                if (FORMED) v = (double)((V[o] - cab * V2[o]) * ibb);
-                else v = (double)V[o];
-                const int q = (gz - cz + nc) * w2 + ridx;
-#pragma unroll
-                for (int i = 0; i < MAXP; ++i)
-                    if (i < np) acc[i] += v * (double)U[(size_t)i * w3 + q];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < MAXP; ++i) {
-            if (i < np) {
-                const double r = wave_sum(acc[i]);
-                if (lane == 0) sb[A.ip_base[J] + i] = r * A.inv_denom[16 * t + i];
-            }
-        }
-    }
-}
-
-// The projections of k_proj for the NG consecutive slots of a group at once:
-// one wave per image of the group list reads each U value once for the
+// Projections s[b][ip] = <U_ip, v_b>/Denom over the intersection of the
+// image's rc-cube and node b's cube (nonlocal.cpp:149-171), for the slots of a
+// group at once.  With FORMED, v is the Lanczos vector formed from the two
+// stored vectors with the same rounding as the z-march forms it, so that the
+// projections always belong to the vector being multiplied (a recursion on
+// projections would amplify rounding by |alpha/beta| per pass).
+// One wave per image of the group list reads each U value once for the
 // group (the cubes of neighbouring nodes overlap in all but a few planes)
 // and accumulates it against every member's vector.  Lane l always takes
 // the points of the image's rc-box whose xy index in the box is l mod 64,
@@ -663,7 +605,7 @@ __global__ void __launch_bounds__(256) k_projg(PArgs<T> A)
     constexpr unsigned TS = sizeof(T);
     const Geo &G = A.g;
     const int q = blockIdx.x;
-    const int b0 = q * NG, gn = min(NG, A.B - b0);
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwave = blockDim.x >> 6;
     int ni[NG], nj[NG], nk[NG];
@@ -843,8 +785,7 @@ __device__ __forceinline__ double wave_sums(double (&v)[NV], int lane)
 // Slabs hold SZ planes whose first global z is a multiple of SZ.  Lane l takes the box points
 // whose xy index in the image box is l mod 64; the plane's partial sums are
 // combined by wave_sums and added plane after plane, so a member's totals
-// depend only on its own cube.  A group whose union plane exceeds pu points
-// is walked one member at a time, in the same order.
+// depend only on its own cube.
 
 // Image data that k_projs reads per image and plane, cached in LDS per group
 struct ImgMeta {
@@ -866,13 +807,10 @@ __device__ __forceinline__ int first_cz_at_least(const ImgMeta *im, int cnt, int
     return lo;
 }
 
-template <typename T, int MAXP, int FORMED, int SZ, int NT, int NPU, int NM>
+template <typename T, int MAXP, int FORMED, int SZ, int NT, int NPU>
 __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 {
-    // NM members per workgroup: all NG slots of the group, or a 2x2 block of
-    // its 4x2 slots (two workgroups per group, half the LDS each)
-    static_assert(NM == NG || NM == 4, "k_projs: NM is NG or 4");
-    constexpr int SUBS = NG / NM;
+    constexpr int NM = NG;
     constexpr int NV = NM * MAXP;
     constexpr int LV = NV == 32 ? 5 : NV == 16 ? 4 : NV == 8 ? 3 : NV == 4 ? 2 : 0;
     static_assert(LV > 0, "k_projs: NM * MAXP must be 4, 8, 16 or 32");
@@ -883,30 +821,26 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
     constexpr int RPI = SZ >= 4 ? 2 : 3;   // rounds of 64 box points per U load batch
     constexpr int PPT = SZ >= 4 ? 2 : 3;   // staged points per thread per load batch
     const Geo &G = A.g;
-    const int q = blockIdx.x / SUBS, hsub = blockIdx.x % SUBS;
-    const int b0 = q * NG, gn = min(NG, A.B - b0);
+    const int q = blockIdx.x;
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwave = blockDim.x >> 6;
-    int ni[NM], nj[NM], nk[NM], gs[NM];   // gs: the member's slot in the group
+    int ni[NM], nj[NM], nk[NM];
     bool on[NM];
     T cab[NM], ibb[NM];
     int nact = 0;
     unsigned onmask = 0;
-    int x0 = 1 << 30, x1 = -(1 << 30), y0 = 1 << 30, y1 = -(1 << 30);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        gs[m] = NM == NG ? m : (m & 1) + 2 * hsub + 4 * (m >> 1);
-        on[m] = gs[m] < gn && !(G.done && G.done[b0 + gs[m]]);
-        const int node = G.node_list[b0 + min(gs[m], gn - 1)];
+        on[m] = m < gn && !(G.done && G.done[b0 + m]);
+        const int node = G.node_list[b0 + min(m, gn - 1)];
         ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
         cab[m] = 0; ibb[m] = 1;
         if (on[m]) {
             ++nact;
             onmask |= 1u << m;
-            if (FORMED) { cab[m] = (T)A.ca[b0 + gs[m]]; ibb[m] = (T)A.ib[b0 + gs[m]]; }
-            x0 = min(x0, ni[m]); x1 = max(x1, ni[m]);
-            y0 = min(y0, nj[m]); y1 = max(y1, nj[m]);
+            if (FORMED) { cab[m] = (T)A.ca[b0 + m]; ibb[m] = (T)A.ib[b0 + m]; }
         }
     }
     const int cnt = A.glist_cnt[q];
@@ -931,147 +865,139 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 #pragma unroll
         for (int m = 0; m < NM; ++m)
             if ((onmask >> m) & 1u)
-                for (int i = 0; i < e.np; ++i) A.s[(size_t)(b0 + gs[m]) * A.n_ip + e.ipb + i] = 0.0;
+                for (int i = 0; i < e.np; ++i) A.s[(size_t)(b0 + m) * A.n_ip + e.ipb + i] = 0.0;
     }
     const size_t gb = (size_t)gn * M3 * TS;
     const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3, gb);
     const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3, gb);
-    const bool together = (x1 - x0 + M) * (y1 - y0 + M) <= A.pu;
-#pragma unroll 1
-    for (int sub = 0; sub < (together ? 1 : NM); ++sub) {
-        // members staged in this walk, and the union of their cubes
-        bool in_sub[NM];
-        int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
+    // union of the members' cubes
+    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            in_sub[m] = on[m] && (together || m == sub);
-            if (in_sub[m]) {
-                ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-                uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-                uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+    for (int m = 0; m < NM; ++m) {
+        if (on[m]) {
+            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
+            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
+            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+        }
+    }
+    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, up = ux * uy, sp = SZ * up;
+    // slabs of SZ planes whose first global z is a multiple of SZ (the same
+    // slab boundaries for every grouping of the nodes)
+    const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
+#pragma unroll 1
+    for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
+        // the previous slab is consumed, and this wave's atomics (and the
+        // zeroing stores) have been performed in L2 (vmcnt 0) before any
+        // wave adds the next slab's totals
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        // the images that can cross the slab form one range of the z-sorted list
+        if (tid == 0) {
+            sh_lo = first_cz_at_least(im, cnt, gzs - sh_ncmax);
+            sh_hi = first_cz_at_least(im, cnt, gzs + SZ + sh_ncmax);
+        }
+        // stage the slab ([plane][point][member]): every load of the
+        // thread's points issued before the first store
+#pragma unroll 1
+        for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
+            T xv[PPT][NM], yv[PPT][NM];
+#pragma unroll
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                const int sl = p / up, pq = p - sl * up;
+                const int yy = pq / ux, xx = pq - yy * ux;
+                const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
+                    const bool ok = p < sp && on[m] && (unsigned)lx < (unsigned)M &&
+                                    (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
+                    const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
+                    xv[r][m] = bload<T>(rX, o);
+                    yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                if (p < sp) {
+#pragma unroll
+                    for (int m = 0; m < NM; ++m)
+                        pl[(size_t)p * NM + m] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
+                }
             }
         }
-        if (ux1 < ux0) continue;
-        const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, up = ux * uy, sp = SZ * up;
-        // slabs of SZ planes whose first global z is a multiple of SZ (the same
-        // slab boundaries for every grouping of the nodes)
-        const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
+        __syncthreads();
+        const int li_lo = __builtin_amdgcn_readfirstlane(sh_lo), li_hi = __builtin_amdgcn_readfirstlane(sh_hi);
 #pragma unroll 1
-        for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
-            // the previous slab is consumed, and this wave's atomics (and the
-            // zeroing stores) have been performed in L2 (vmcnt 0) before any
-            // wave adds the next slab's totals
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            // the images that can cross the slab form one range of the z-sorted list
-            if (tid == 0) {
-                sh_lo = first_cz_at_least(im, cnt, gzs - sh_ncmax);
-                sh_hi = first_cz_at_least(im, cnt, gzs + SZ + sh_ncmax);
-            }
-            // stage the slab ([plane][point][member]): every load of the
-            // thread's points issued before the first store
+        for (int li = li_lo + wave; li < li_hi; li += nwave) {
+            // the image's data is wave-uniform: keep it in scalar registers
+            const ImgMeta &e = im[li];
+            const int w = __builtin_amdgcn_readfirstlane(e.w), oz = __builtin_amdgcn_readfirstlane(e.oz);
+            const int bz0 = gzs - oz;   // box z of the slab's first plane
+            if (bz0 + SZ <= 0 || bz0 >= w) continue;
+            const int ox = __builtin_amdgcn_readfirstlane(e.ox), oy = __builtin_amdgcn_readfirstlane(e.oy);
+            const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
+            const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
+            if (rlo > rhi || clo > chi) continue;
+            const int np = __builtin_amdgcn_readfirstlane(e.np), w2 = w * w, w3 = w2 * w;
+            const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(e.uoff >> 32)) << 32) |
+                                     (unsigned)__builtin_amdgcn_readfirstlane((int)e.uoff));
+            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + uoff, (size_t)np * w3 * TS);
+            // the value this lane adds at the end: member kw / MAXP, projector kw % MAXP
+            const int kw = lane >> (6 - LV), mw = kw / MAXP, iw = kw - mw * MAXP;
+            const bool writer = (lane & ((64 >> LV) - 1)) == 0 && ((onmask >> mw) & 1u) && iw < np;
+            const int t = __builtin_amdgcn_readfirstlane(e.t), ipb = __builtin_amdgcn_readfirstlane(e.ipb);
+            const double idn = writer ? A.inv_denom[16 * t + iw] : 0.0;
+            double acc[NV];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) acc[k] = 0.0;
+            const int a_hi = (rhi + 1) * w;
+            // a / w through the float reciprocal: exact, since (a + 1/2)/w
+            // stays at least 1/(2w) away from an integer (a < w^2, w < 1000)
+            const float rw = 1.0f / (float)w;
+            // RPI rounds of 64 box points at a time, their U loads issued together
 #pragma unroll 1
-            for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
-                T xv[PPT][NM], yv[PPT][NM];
+            for (int c0 = (rlo * w) & ~63; c0 < a_hi; c0 += 64 * RPI) {
+                T u[RPI][SZ][NPU];
+                int pp[RPI];
+                bool in[RPI];
 #pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
-                    const int sl = p / up, pq = p - sl * up;
-                    const int yy = pq / ux, xx = pq - yy * ux;
-                    const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+                for (int r = 0; r < RPI; ++r) {
+                    const int a = c0 + 64 * r + lane;
+                    const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
+                    in[r] = a < a_hi && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) {
-                        const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
-                        const bool ok = p < sp && in_sub[m] && (unsigned)lx < (unsigned)M &&
-                                        (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
-                        const unsigned o = ok ? (unsigned)(gs[m] * M3 + lz * M2 + ly * M + lx) * TS : OOB;
-                        xv[r][m] = bload<T>(rX, o);
-                        yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                    for (int z = 0; z < SZ; ++z) {
+                        const bool okz = in[r] && (unsigned)(bz0 + z) < (unsigned)w;
+#pragma unroll
+                        for (int i = 0; i < NPU; ++i)
+                            u[r][z][i] = bload<T>(rU, (okz && i < np) ? (unsigned)(i * w3 + (bz0 + z) * w2 + a) * TS : OOB);
                     }
+                    pp[r] = in[r] ? (oy + by - uy0) * ux + (ox + bx - ux0) : 0;
                 }
 #pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
-                    if (p < sp) {
+                for (int r = 0; r < RPI; ++r) {
 #pragma unroll
-                        for (int m = 0; m < NM; ++m)
-                            pl[(size_t)p * NM + m] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
-                    }
-                }
-            }
-            __syncthreads();
-            const int li_lo = __builtin_amdgcn_readfirstlane(sh_lo), li_hi = __builtin_amdgcn_readfirstlane(sh_hi);
-#pragma unroll 1
-            for (int li = li_lo + wave; li < li_hi; li += nwave) {
-                // the image's data is wave-uniform: keep it in scalar registers
-                const ImgMeta &e = im[li];
-                const int w = __builtin_amdgcn_readfirstlane(e.w), oz = __builtin_amdgcn_readfirstlane(e.oz);
-                const int bz0 = gzs - oz;   // box z of the slab's first plane
-                if (bz0 + SZ <= 0 || bz0 >= w) continue;
-                const int ox = __builtin_amdgcn_readfirstlane(e.ox), oy = __builtin_amdgcn_readfirstlane(e.oy);
-                const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
-                const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
-                if (rlo > rhi || clo > chi) continue;
-                const int np = __builtin_amdgcn_readfirstlane(e.np), w2 = w * w, w3 = w2 * w;
-                const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(e.uoff >> 32)) << 32) |
-                                         (unsigned)__builtin_amdgcn_readfirstlane((int)e.uoff));
-                const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + uoff, (size_t)np * w3 * TS);
-                // the value this lane adds at the end: member kw / MAXP, projector kw % MAXP
-                const int kw = lane >> (6 - LV), mw = kw / MAXP, iw = kw - mw * MAXP;
-                const bool writer = (lane & ((64 >> LV) - 1)) == 0 && ((onmask >> mw) & 1u) && iw < np;
-                const int t = __builtin_amdgcn_readfirstlane(e.t), ipb = __builtin_amdgcn_readfirstlane(e.ipb);
-                const double idn = writer ? A.inv_denom[16 * t + iw] : 0.0;
-                double acc[NV];
+                    for (int z = 0; z < SZ; ++z) {
+                        const T *pv = pl + ((size_t)z * up + pp[r]) * NM;
+                        T v[NM];
 #pragma unroll
-                for (int k = 0; k < NV; ++k) acc[k] = 0.0;
-                const int a_hi = (rhi + 1) * w;
-                // a / w through the float reciprocal: exact, since (a + 1/2)/w
-                // stays at least 1/(2w) away from an integer (a < w^2, w < 1000)
-                const float rw = 1.0f / (float)w;
-                // RPI rounds of 64 box points at a time, their U loads issued together
-#pragma unroll 1
-                for (int c0 = (rlo * w) & ~63; c0 < a_hi; c0 += 64 * RPI) {
-                    T u[RPI][SZ][NPU];
-                    int pp[RPI];
-                    bool in[RPI];
+                        for (int m = 0; m < NM; ++m) v[m] = pv[m];
+                        if (in[r]) {
 #pragma unroll
-                    for (int r = 0; r < RPI; ++r) {
-                        const int a = c0 + 64 * r + lane;
-                        const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
-                        in[r] = a < a_hi && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
+                            for (int m = 0; m < NM; ++m)
 #pragma unroll
-                        for (int z = 0; z < SZ; ++z) {
-                            const bool okz = in[r] && (unsigned)(bz0 + z) < (unsigned)w;
-#pragma unroll
-                            for (int i = 0; i < NPU; ++i)
-                                u[r][z][i] = bload<T>(rU, (okz && i < np) ? (unsigned)(i * w3 + (bz0 + z) * w2 + a) * TS : OOB);
-                        }
-                        pp[r] = in[r] ? (oy + by - uy0) * ux + (ox + bx - ux0) : 0;
-                    }
-#pragma unroll
-                    for (int r = 0; r < RPI; ++r) {
-#pragma unroll
-                        for (int z = 0; z < SZ; ++z) {
-                            const T *pv = pl + ((size_t)z * up + pp[r]) * NM;
-                            T v[NM];
-#pragma unroll
-                            for (int m = 0; m < NM; ++m) v[m] = pv[m];
-                            if (in[r]) {
-#pragma unroll
-                                for (int m = 0; m < NM; ++m)
-#pragma unroll
-                                    for (int i = 0; i < NPU; ++i)
-                                        acc[m * MAXP + i] += (double)v[m] * (double)u[r][z][i];
-                            }
+                                for (int i = 0; i < NPU; ++i)
+                                    acc[m * MAXP + i] += (double)v[m] * (double)u[r][z][i];
                         }
                     }
                 }
-                const double tot = wave_sums<NV>(acc, lane);
-                // one lane per value and slab; slabs are ordered by the fence
-                // and barrier above, so the additions happen in slab order
-                const int gw = NM == NG ? mw : (mw & 1) + 2 * hsub + 4 * (mw >> 1);   // gs[mw]
-                if (writer) unsafeAtomicAdd(A.s + (size_t)(b0 + gw) * A.n_ip + ipb + iw, tot * idn);
             }
+            const double tot = wave_sums<NV>(acc, lane);
+            // one lane per value and slab; slabs are ordered by the fence
+            // and barrier above, so the additions happen in slab order
+            if (writer) unsafeAtomicAdd(A.s + (size_t)(b0 + mw) * A.n_ip + ipb + iw, tot * idn);
         }
     }
 }
@@ -1091,46 +1017,37 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 // Requires one box size for every image of the list and R larger than the
 // slot distance of any two images of a wave alive at once (k_group_images
 // computes the R a batch needs; the host picks a compiled R at least that).
-template <typename T, int FORMED, int SZ, int NT, int NM, int R, int RPI>
+template <typename T, int FORMED, int SZ, int NT, int R, int RPI>
 __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
 {
-    static_assert(NM == NG || NM == 4, "k_projr: NM is NG or 4");
-    constexpr int SUBS = NG / NM;
+    constexpr int NM = NG;
     constexpr int NV = NM;                    // one projector per image (s channel)
-    constexpr int LV = NV == 8 ? 3 : 2;
+    constexpr int LV = 3;
+    static_assert(NV == 1 << LV, "k_projr: NG is 8");
     constexpr unsigned TS = sizeof(T);
     constexpr int PPT = 2;                    // staged points per thread per load batch
     const Geo &G = A.g;
-    const int q = blockIdx.x / SUBS, hsub = blockIdx.x % SUBS;
-    const int b0 = q * NG, gn = min(NG, A.B - b0);
+    const int q = blockIdx.x;
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int NW = NT / 64;
-    int ni[NM], nj[NM], nk[NM], gs[NM];
+    int ni[NM], nj[NM], nk[NM];
     bool on[NM];
     T cab[NM], ibb[NM];
     int nact = 0;
     unsigned onmask = 0;
-    // extent of every member of the group (frozen ones included), so that the
-    // choice between one walk and member-by-member walks is the same in every
-    // pass (k_group_images checks the slot plan of that choice)
-    int x0 = 1 << 30, x1 = -(1 << 30), y0 = 1 << 30, y1 = -(1 << 30);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        gs[m] = NM == NG ? m : (m & 1) + 2 * hsub + 4 * (m >> 1);
-        on[m] = gs[m] < gn && !(G.done && G.done[b0 + gs[m]]);
-        const int node = G.node_list[b0 + min(gs[m], gn - 1)];
+        on[m] = m < gn && !(G.done && G.done[b0 + m]);
+        const int node = G.node_list[b0 + min(m, gn - 1)];
         ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
         cab[m] = 0; ibb[m] = 1;
-        if (gs[m] < gn) {
-            x0 = min(x0, ni[m]); x1 = max(x1, ni[m]);
-            y0 = min(y0, nj[m]); y1 = max(y1, nj[m]);
-        }
         if (on[m]) {
             ++nact;
             onmask |= 1u << m;
-            if (FORMED) { cab[m] = (T)A.ca[b0 + gs[m]]; ibb[m] = (T)A.ib[b0 + gs[m]]; }
+            if (FORMED) { cab[m] = (T)A.ca[b0 + m]; ibb[m] = (T)A.ib[b0 + m]; }
         }
     }
     const int cnt = A.glist_cnt[q];
@@ -1154,170 +1071,160 @@ __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
     const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3, gb);
     // LDS rows of the slab are padded to a pitch congruent to the box side
     // modulo 32 values, so that the box rows one wave reads fall on disjoint
-    // banks; A.pu is the slab capacity per plane and member
+    // banks
     const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
     auto upitch_of = [&](int u) { return u + (((wbox - u) % 32) + 32) % 32; };
-    const bool together = upitch_of(x1 - x0 + M) * (y1 - y0 + M) <= A.pu;
     // the value this lane stores for a leaving image: member kw
     const int kw = lane >> (6 - LV);
     const bool wlane = (lane & ((64 >> LV) - 1)) == 0;
-    const int gw = NM == NG ? kw : (kw & 1) + 2 * hsub + 4 * (kw >> 1);   // gs[kw]
-    double *sw = A.s + (size_t)(b0 + gw) * A.n_ip;
-#pragma unroll 1
-    for (int sub = 0; sub < (together ? 1 : NM); ++sub) {
-        bool in_sub[NM];
-        unsigned submask = 0;
-        int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
+    double *sw = A.s + (size_t)(b0 + kw) * A.n_ip;
+    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            in_sub[m] = on[m] && (together || m == sub);
-            if (in_sub[m]) {
-                submask |= 1u << m;
-                ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-                uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-                uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+    for (int m = 0; m < NM; ++m) {
+        if (on[m]) {
+            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
+            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
+            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+        }
+    }
+    const bool writer = wlane && ((onmask >> kw) & 1u);
+    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), up = upx * uy;
+    const int np_ = ux * uy, sp = SZ * np_;   // staged points of a slab (unpadded)
+    const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
+    // per-wave slot state: images started (slotted or not), slotted
+    // images, live-slot mask, per-slot image data
+    int nstart = 0, nslot = 0;
+    unsigned live = 0;
+    int s_oz[R], s_ze[R], s_w[R], s_ipb[R], s_t[R];
+    long s_uoff[R];
+    int s_pp[R][RPI];                     // LDS point of the lane's box point, or -1
+    double acc[R][NM];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        s_oz[r] = s_ze[r] = s_w[r] = s_ipb[r] = s_t[r] = 0;
+        s_uoff[r] = 0;
+#pragma unroll
+        for (int k = 0; k < RPI; ++k) s_pp[r][k] = -1;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
+    }
+#pragma unroll 1
+    for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
+        // the previous slab is consumed before it is overwritten
+        __syncthreads();
+#pragma unroll 1
+        for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
+            T xv[PPT][NM], yv[PPT][NM];
+#pragma unroll
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                const int sl = p / np_, pq = p - sl * np_;
+                const int yy = pq / ux, xx = pq - yy * ux;
+                const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
+                    const bool ok = p < sp && on[m] && (unsigned)lx < (unsigned)M &&
+                                    (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
+                    const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
+                    xv[r][m] = bload<T>(rX, o);
+                    yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                }
             }
-        }
-        if (ux1 < ux0) continue;
-        const bool writer = wlane && ((submask >> kw) & 1u);
-        const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), up = upx * uy;
-        const int np_ = ux * uy, sp = SZ * np_;   // staged points of a slab (unpadded)
-        const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
-        // per-wave slot state: images started (slotted or not), slotted
-        // images, live-slot mask, per-slot image data
-        int nstart = 0, nslot = 0;
-        unsigned live = 0;
-        int s_oz[R], s_ze[R], s_w[R], s_ipb[R], s_t[R];
-        long s_uoff[R];
-        int s_pp[R][RPI];                     // LDS point of the lane's box point, or -1
-        double acc[R][NM];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            s_oz[r] = s_ze[r] = s_w[r] = s_ipb[r] = s_t[r] = 0;
-            s_uoff[r] = 0;
-#pragma unroll
-            for (int k = 0; k < RPI; ++k) s_pp[r][k] = -1;
-#pragma unroll
-            for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
-        }
-#pragma unroll 1
-        for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
-            // the previous slab is consumed before it is overwritten
-            __syncthreads();
-#pragma unroll 1
-            for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
-                T xv[PPT][NM], yv[PPT][NM];
-#pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                if (p < sp) {
+                    // member-major: [plane][member][row][padded column]
                     const int sl = p / np_, pq = p - sl * np_;
                     const int yy = pq / ux, xx = pq - yy * ux;
-                    const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+                    T *dst = pl + (size_t)sl * NM * up + yy * upx + xx;
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) {
-                        const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
-                        const bool ok = p < sp && in_sub[m] && (unsigned)lx < (unsigned)M &&
-                                        (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
-                        const unsigned o = ok ? (unsigned)(gs[m] * M3 + lz * M2 + ly * M + lx) * TS : OOB;
-                        xv[r][m] = bload<T>(rX, o);
-                        yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
-                    if (p < sp) {
-                        // member-major: [plane][member][row][padded column]
-                        const int sl = p / np_, pq = p - sl * np_;
-                        const int yy = pq / ux, xx = pq - yy * ux;
-                        T *dst = pl + (size_t)sl * NM * up + yy * upx + xx;
-#pragma unroll
-                        for (int m = 0; m < NM; ++m)
-                            dst[(size_t)m * up] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
-                    }
+                    for (int m = 0; m < NM; ++m)
+                        dst[(size_t)m * up] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
                 }
             }
-            __syncthreads();
-            const int zl = gzs + SZ - 1;   // last plane of the slab
-            // images of this wave that enter the union in this slab take their slot
+        }
+        __syncthreads();
+        const int zl = gzs + SZ - 1;   // last plane of the slab
+        // images of this wave that enter the union in this slab take their slot
 #pragma unroll 1
-            for (;;) {
-                const int li = wave + NW * nstart;
-                if (li >= cnt) break;
-                const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
-                const int w = __builtin_amdgcn_readfirstlane(im[li].w);
-                const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
-                const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
-                                  by0 + w - 1 < uy0 || by0 > uy1;
-                const int zs = max(oz, uz0);
-                if (!miss && zs > zl) break;
-                if (miss) {   // the box misses the union: the projection is zero
-                    const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
-                    if (writer) sw[ipb] = 0.0;
-                    ++nstart;
-                    continue;
-                }
-                const int slot = nslot % R;
-                ++nslot;
-                const int ox = __builtin_amdgcn_readfirstlane(im[li].ox), oy = __builtin_amdgcn_readfirstlane(im[li].oy);
-                const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
-                const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
-                const float rw = 1.0f / (float)w;
-                int pp[RPI];
-#pragma unroll
-                for (int k = 0; k < RPI; ++k) {
-                    const int a = 64 * k + lane;
-                    const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
-                    const bool in = a < w * w && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
-                    pp[k] = in ? (oy + by - uy0) * upx + (ox + bx - ux0) : -1;
-                }
-                const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb), t = __builtin_amdgcn_readfirstlane(im[li].t);
-                const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
-                                         (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if (r == slot) {
-                        s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_w[r] = w; s_ipb[r] = ipb; s_t[r] = t;
-                        s_uoff[r] = uoff;
-#pragma unroll
-                        for (int k = 0; k < RPI; ++k) s_pp[r][k] = pp[k];
-#pragma unroll
-                        for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
-                    }
-                }
-                live |= 1u << slot;
+        for (;;) {
+            const int li = wave + NW * nstart;
+            if (li >= cnt) break;
+            const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
+            const int w = __builtin_amdgcn_readfirstlane(im[li].w);
+            const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
+            const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
+                              by0 + w - 1 < uy0 || by0 > uy1;
+            const int zs = max(oz, uz0);
+            if (!miss && zs > zl) break;
+            if (miss) {   // the box misses the union: the projection is zero
+                const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
+                if (writer) sw[ipb] = 0.0;
                 ++nstart;
+                continue;
             }
-            // every live slot adds the slab's planes of its box
+            const int slot = nslot % R;
+            ++nslot;
+            const int ox = __builtin_amdgcn_readfirstlane(im[li].ox), oy = __builtin_amdgcn_readfirstlane(im[li].oy);
+            const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
+            const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
+            const float rw = 1.0f / (float)w;
+            int pp[RPI];
+#pragma unroll
+            for (int k = 0; k < RPI; ++k) {
+                const int a = 64 * k + lane;
+                const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
+                const bool in = a < w * w && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
+                pp[k] = in ? (oy + by - uy0) * upx + (ox + bx - ux0) : -1;
+            }
+            const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb), t = __builtin_amdgcn_readfirstlane(im[li].t);
+            const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
+                                     (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                if (!((live >> r) & 1u)) continue;
-                const int w = s_w[r], w2 = w * w;
-                const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
-                const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)w2 * w * TS);
-                for (int z = za; z <= zb; ++z) {
-                    const int bz = z - s_oz[r];
-                    T u[RPI];
+                if (r == slot) {
+                    s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_w[r] = w; s_ipb[r] = ipb; s_t[r] = t;
+                    s_uoff[r] = uoff;
 #pragma unroll
-                    for (int k = 0; k < RPI; ++k)
-                        u[k] = bload<T>(rU, s_pp[r][k] >= 0 ? (unsigned)(bz * w2 + 64 * k + lane) * TS : OOB);
+                    for (int k = 0; k < RPI; ++k) s_pp[r][k] = pp[k];
 #pragma unroll
-                    for (int k = 0; k < RPI; ++k) {
-                        const T *pv = pl + (size_t)(z - gzs) * NM * up + max(s_pp[r][k], 0);
-                        T v[NM];
+                    for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
+                }
+            }
+            live |= 1u << slot;
+            ++nstart;
+        }
+        // every live slot adds the slab's planes of its box
 #pragma unroll
-                        for (int m = 0; m < NM; ++m) v[m] = pv[(size_t)m * up];
-                        if (s_pp[r][k] >= 0) {
+        for (int r = 0; r < R; ++r) {
+            if (!((live >> r) & 1u)) continue;
+            const int w = s_w[r], w2 = w * w;
+            const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
+            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)w2 * w * TS);
+            for (int z = za; z <= zb; ++z) {
+                const int bz = z - s_oz[r];
+                T u[RPI];
 #pragma unroll
-                            for (int m = 0; m < NM; ++m) acc[r][m] += (double)v[m] * (double)u[k];
-                        }
+                for (int k = 0; k < RPI; ++k)
+                    u[k] = bload<T>(rU, s_pp[r][k] >= 0 ? (unsigned)(bz * w2 + 64 * k + lane) * TS : OOB);
+#pragma unroll
+                for (int k = 0; k < RPI; ++k) {
+                    const T *pv = pl + (size_t)(z - gzs) * NM * up + max(s_pp[r][k], 0);
+                    T v[NM];
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) v[m] = pv[(size_t)m * up];
+                    if (s_pp[r][k] >= 0) {
+#pragma unroll
+                        for (int m = 0; m < NM; ++m) acc[r][m] += (double)v[m] * (double)u[k];
                     }
                 }
-                if (s_ze[r] <= zl) {   // the image leaves the union in this slab
-                    const double tot = wave_sums<NV>(acc[r], lane);
-                    if (writer) sw[s_ipb[r]] = tot * A.inv_denom[16 * s_t[r]];
-                    live &= ~(1u << r);
-                }
+            }
+            if (s_ze[r] <= zl) {   // the image leaves the union in this slab
+                const double tot = wave_sums<NV>(acc[r], lane);
+                if (writer) sw[s_ipb[r]] = tot * A.inv_denom[16 * s_t[r]];
+                live &= ~(1u << r);
             }
         }
     }
@@ -1348,7 +1255,7 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
     constexpr int PPT = 2;
     const Geo &G = A.g;
     const int q = blockIdx.x;
-    const int b0 = q * NG, gn = min(NG, A.B - b0);
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1358,17 +1265,12 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
     T cab[NM], ibb[NM];
     int nact = 0;
     unsigned onmask = 0;
-    int x0 = 1 << 30, x1 = -(1 << 30), y0 = 1 << 30, y1 = -(1 << 30);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
         on[m] = m < gn && !(G.done && G.done[b0 + m]);
         const int node = G.node_list[b0 + min(m, gn - 1)];
         ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
         cab[m] = 0; ibb[m] = 1;
-        if (m < gn) {
-            x0 = min(x0, ni[m]); x1 = max(x1, ni[m]);
-            y0 = min(y0, nj[m]); y1 = max(y1, nj[m]);
-        }
         if (on[m]) {
             ++nact;
             onmask |= 1u << m;
@@ -1397,7 +1299,6 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
     const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
     auto upitch_of = [&](int u) { return u + (((wbox - u) % 32) + 32) % 32; };
     auto mstride_of = [&](int u) { return u + (((8 - u) % 32) + 32) % 32; };
-    const bool together = mstride_of(upitch_of(x1 - x0 + M) * (y1 - y0 + M)) <= A.pu;
     // lane roles in the MFMA: K index, block (member quad, point phase), row/column
     const int kk = lane >> 4, bb = (lane >> 2) & 3, ii = lane & 3;
     const int mA = 4 * (bb & 1) + ii;          // member of the lane's A value
@@ -1406,169 +1307,161 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
     const int mw = 4 * ((lane >> 2) & 1) + (lane >> 4), jw = lane & 3;
     const bool wl = (lane & 8) == 0;
     double *sw = A.s + (size_t)(b0 + mw) * A.n_ip;
-#pragma unroll 1
-    for (int sub = 0; sub < (together ? 1 : NM); ++sub) {
-        bool in_sub[NM];
-        unsigned submask = 0;
-        int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
+    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            in_sub[m] = on[m] && (together || m == sub);
-            if (in_sub[m]) {
-                submask |= 1u << m;
-                ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-                uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-                uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+    for (int m = 0; m < NM; ++m) {
+        if (on[m]) {
+            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
+            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
+            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+        }
+    }
+    const bool writer = wl && ((onmask >> mw) & 1u);
+    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), ms = mstride_of(upx * uy);
+    const int np_ = ux * uy, sp = SZ * np_;
+    const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
+    int nstart = 0, nslot = 0;
+    unsigned live = 0;
+    int s_oz[R], s_ze[R], s_ipb[R], s_t[R], s_np[R], s_ox[R], s_oy[R];
+    long s_uoff[R];
+    double cacc[R][2];   // per slot: the first and second MFMA of each box row
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        s_oz[r] = s_ze[r] = s_ipb[r] = s_t[r] = s_np[r] = s_ox[r] = s_oy[r] = 0;
+        s_uoff[r] = 0;
+        cacc[r][0] = cacc[r][1] = 0.0;
+    }
+#pragma unroll 1
+    for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
+        __syncthreads();
+#pragma unroll 1
+        for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
+            T xv[PPT][NM], yv[PPT][NM];
+#pragma unroll
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                const int sl = p / np_, pq = p - sl * np_;
+                const int yy = pq / ux, xx = pq - yy * ux;
+                const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
+                    const bool ok = p < sp && on[m] && (unsigned)lx < (unsigned)M &&
+                                    (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
+                    const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
+                    xv[r][m] = bload<T>(rX, o);
+                    yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                }
             }
-        }
-        if (ux1 < ux0) continue;
-        const bool writer = wl && ((submask >> mw) & 1u);
-        const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), ms = mstride_of(upx * uy);
-        const int np_ = ux * uy, sp = SZ * np_;
-        const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
-        int nstart = 0, nslot = 0;
-        unsigned live = 0;
-        int s_oz[R], s_ze[R], s_ipb[R], s_t[R], s_np[R], s_ox[R], s_oy[R];
-        long s_uoff[R];
-        double cacc[R][2];   // per slot: the first and second MFMA of each box row
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            s_oz[r] = s_ze[r] = s_ipb[r] = s_t[r] = s_np[r] = s_ox[r] = s_oy[r] = 0;
-            s_uoff[r] = 0;
-            cacc[r][0] = cacc[r][1] = 0.0;
-        }
-#pragma unroll 1
-        for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
-            __syncthreads();
-#pragma unroll 1
-            for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
-                T xv[PPT][NM], yv[PPT][NM];
-#pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
+            for (int r = 0; r < PPT; ++r) {
+                const int p = p0 + r * (int)blockDim.x + tid;
+                if (p < sp) {
                     const int sl = p / np_, pq = p - sl * np_;
                     const int yy = pq / ux, xx = pq - yy * ux;
-                    const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+                    T *dst = pl + (size_t)sl * NM * ms + yy * upx + xx;
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) {
-                        const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
-                        const bool ok = p < sp && in_sub[m] && (unsigned)lx < (unsigned)M &&
-                                        (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
-                        const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
-                        xv[r][m] = bload<T>(rX, o);
-                        yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < PPT; ++r) {
-                    const int p = p0 + r * (int)blockDim.x + tid;
-                    if (p < sp) {
-                        const int sl = p / np_, pq = p - sl * np_;
-                        const int yy = pq / ux, xx = pq - yy * ux;
-                        T *dst = pl + (size_t)sl * NM * ms + yy * upx + xx;
-#pragma unroll
-                        for (int m = 0; m < NM; ++m)
-                            dst[(size_t)m * ms] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
-                    }
+                    for (int m = 0; m < NM; ++m)
+                        dst[(size_t)m * ms] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
                 }
             }
-            __syncthreads();
-            const int zl = gzs + SZ - 1;
+        }
+        __syncthreads();
+        const int zl = gzs + SZ - 1;
 #pragma unroll 1
-            for (;;) {
-                const int li = wave + NW * nstart;
-                if (li >= cnt) break;
-                const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
-                const int w = wbox;
-                const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
-                const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
-                                  by0 + w - 1 < uy0 || by0 > uy1;
-                const int zs = max(oz, uz0);
-                if (!miss && zs > zl) break;
-                const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
-                const int np = __builtin_amdgcn_readfirstlane(im[li].np);
-                if (miss) {   // the box misses the union: the projections are zero
-                    if (writer && jw < np) sw[ipb + jw] = 0.0;
-                    ++nstart;
-                    continue;
-                }
-                const int slot = nslot % R;
-                ++nslot;
-                const int t = __builtin_amdgcn_readfirstlane(im[li].t);
-                const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
-                                         (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if (r == slot) {
-                        s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_ipb[r] = ipb; s_t[r] = t; s_np[r] = np;
-                        s_ox[r] = bx0; s_oy[r] = by0; s_uoff[r] = uoff;
-                        cacc[r][0] = cacc[r][1] = 0.0;
-                    }
-                }
-                live |= 1u << slot;
+        for (;;) {
+            const int li = wave + NW * nstart;
+            if (li >= cnt) break;
+            const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
+            const int w = wbox;
+            const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
+            const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
+                              by0 + w - 1 < uy0 || by0 > uy1;
+            const int zs = max(oz, uz0);
+            if (!miss && zs > zl) break;
+            const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
+            const int np = __builtin_amdgcn_readfirstlane(im[li].np);
+            if (miss) {   // the box misses the union: the projections are zero
+                if (writer && jw < np) sw[ipb + jw] = 0.0;
                 ++nstart;
+                continue;
             }
+            const int slot = nslot % R;
+            ++nslot;
+            const int t = __builtin_amdgcn_readfirstlane(im[li].t);
+            const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
+                                     (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                if (!((live >> r) & 1u)) continue;
-                const int w = wbox, w2 = w * w, w3 = w2 * w;
-                const int ox = s_ox[r], oy = s_oy[r];
-                const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
-                const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
-                const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
-                const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)s_np[r] * w3 * TS);
-                const bool colj = ii < s_np[r];
-                bool okx[2];
+                if (r == slot) {
+                    s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_ipb[r] = ipb; s_t[r] = t; s_np[r] = np;
+                    s_ox[r] = bx0; s_oy[r] = by0; s_uoff[r] = uoff;
+                    cacc[r][0] = cacc[r][1] = 0.0;
+                }
+            }
+            live |= 1u << slot;
+            ++nstart;
+        }
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) okx[hh] = bxl0 + 8 * hh >= clo && bxl0 + 8 * hh <= chi;
-                for (int z = za; z <= zb; ++z) {
-                    const int bz = z - s_oz[r];
-                    const T *pz = pl + (size_t)(z - gzs) * NM * ms + (size_t)mA * ms;
-                    // rows in chunks of RC, the next chunk's operands loaded
-                    // while the current chunk's MFMAs run
-                    constexpr int RC = 4;
-                    T an[RC][2], bn[RC][2];
-                    auto load_rows = [&](int by0) {
+        for (int r = 0; r < R; ++r) {
+            if (!((live >> r) & 1u)) continue;
+            const int w = wbox, w2 = w * w, w3 = w2 * w;
+            const int ox = s_ox[r], oy = s_oy[r];
+            const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
+            const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
+            const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
+            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)s_np[r] * w3 * TS);
+            const bool colj = ii < s_np[r];
+            bool okx[2];
 #pragma unroll
-                        for (int j = 0; j < RC; ++j) {
-                            const int by = by0 + j;
-                            const bool rowok = by <= rhi;
-                            const int lrow = (oy + by - uy0) * upx + (ox - ux0);
-                            const int urow = ii * w3 + bz * w2 + by * w;
+            for (int hh = 0; hh < 2; ++hh) okx[hh] = bxl0 + 8 * hh >= clo && bxl0 + 8 * hh <= chi;
+            for (int z = za; z <= zb; ++z) {
+                const int bz = z - s_oz[r];
+                const T *pz = pl + (size_t)(z - gzs) * NM * ms + (size_t)mA * ms;
+                // rows in chunks of RC, the next chunk's operands loaded
+                // while the current chunk's MFMAs run
+                constexpr int RC = 4;
+                T an[RC][2], bn[RC][2];
+                auto load_rows = [&](int by0) {
 #pragma unroll
-                            for (int hh = 0; hh < 2; ++hh) {
-                                const int bx = bxl0 + 8 * hh;
-                                const bool ok = rowok && okx[hh];
-                                an[j][hh] = ok ? pz[lrow + bx] : (T)0;
-                                bn[j][hh] = bload<T>(rU, (ok && colj) ? (unsigned)(urow + bx) * TS : OOB);
-                            }
+                    for (int j = 0; j < RC; ++j) {
+                        const int by = by0 + j;
+                        const bool rowok = by <= rhi;
+                        const int lrow = (oy + by - uy0) * upx + (ox - ux0);
+                        const int urow = ii * w3 + bz * w2 + by * w;
+#pragma unroll
+                        for (int hh = 0; hh < 2; ++hh) {
+                            const int bx = bxl0 + 8 * hh;
+                            const bool ok = rowok && okx[hh];
+                            an[j][hh] = ok ? pz[lrow + bx] : (T)0;
+                            bn[j][hh] = bload<T>(rU, (ok && colj) ? (unsigned)(urow + bx) * TS : OOB);
                         }
-                    };
-                    load_rows(rlo);
-                    for (int by0 = rlo; by0 <= rhi; by0 += RC) {
-                        T ac[RC][2], bc[RC][2];
+                    }
+                };
+                load_rows(rlo);
+                for (int by0 = rlo; by0 <= rhi; by0 += RC) {
+                    T ac[RC][2], bc[RC][2];
 #pragma unroll
-                        for (int j = 0; j < RC; ++j)
+                    for (int j = 0; j < RC; ++j)
 #pragma unroll
-                            for (int hh = 0; hh < 2; ++hh) { ac[j][hh] = an[j][hh]; bc[j][hh] = bn[j][hh]; }
-                        if (by0 + RC <= rhi) load_rows(by0 + RC);
+                        for (int hh = 0; hh < 2; ++hh) { ac[j][hh] = an[j][hh]; bc[j][hh] = bn[j][hh]; }
+                    if (by0 + RC <= rhi) load_rows(by0 + RC);
 #pragma unroll
-                        for (int j = 0; j < RC; ++j) {
-                            if (by0 + j <= rhi) {
+                    for (int j = 0; j < RC; ++j) {
+                        if (by0 + j <= rhi) {
 #pragma unroll
-                                for (int hh = 0; hh < 2; ++hh)
-                                    cacc[r][hh] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)ac[j][hh], (double)bc[j][hh],
-                                                                                     cacc[r][hh], 0, 0, 0);
-                            }
+                            for (int hh = 0; hh < 2; ++hh)
+                                cacc[r][hh] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)ac[j][hh], (double)bc[j][hh],
+                                                                                 cacc[r][hh], 0, 0, 0);
                         }
                     }
                 }
-                if (s_ze[r] <= zl) {   // the image leaves the union: add the partial sums and store
-                    const double c = cacc[r][0] + cacc[r][1];
-                    const double tot = c + __shfl_xor(c, 8, 64);
-                    if (writer && jw < s_np[r]) sw[s_ipb[r] + jw] = tot * A.inv_denom[16 * s_t[r] + jw];
-                    live &= ~(1u << r);
-                }
+            }
+            if (s_ze[r] <= zl) {   // the image leaves the union: add the partial sums and store
+                const double c = cacc[r][0] + cacc[r][1];
+                const double tot = c + __shfl_xor(c, 8, 64);
+                if (writer && jw < s_np[r]) sw[s_ipb[r] + jw] = tot * A.inv_denom[16 * s_t[r] + jw];
+                live &= ~(1u << r);
             }
         }
     }
@@ -1579,17 +1472,15 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
 // and applies them to every member's projections, which sit in LDS
 // compacted to the images of the group list (loc maps an image-projector id
 // to its row, sl holds NG values per row).  Each member's sum runs over the
-// point's entries in slot order, as in k_nlapply.  When the members' cubes
-// are far apart (a group that spans two bricks), each member's cube is
-// walked on its own instead of the union box.
+// point's entries in slot order, as in k_nlapply.
 template <typename T>
 struct NGArgs {
     Geo g;
     NL<T> nl;
     T *nlv;                       // [B][M^3] out
+    const int *gst;               // [groups + 1] first slot of each group
     const int *glist, *glist_cnt;
     const int *img_type, *nproj, *ip_base;
-    int B;
 };
 
 template <typename T, bool IP16>
@@ -1598,7 +1489,7 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     constexpr unsigned TS = sizeof(T);
     const Geo &G = A.g;
     const int q = blockIdx.x;
-    const int b0 = q * NG, gn = min(NG, A.B - b0);
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, M = G.M, M2 = G.M2, M3 = G.M3, E = G.E;
     int ni[NG], nj[NG], nk[NG];
     bool on[NG];
@@ -1680,31 +1571,18 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
         }
     };
     const int ux = ex1 - ex0 + 1, uy = ey1 - ey0 + 1, uz = ez1 - ez0 + 1;
-    if ((long)ux * uy * uz <= (long)nact * M3) {
-        const int uxy = ux * uy, tot = uxy * uz;
+    const int uxy = ux * uy, tot = uxy * uz;
 #pragma unroll 1
-        for (int p = threadIdx.x; p < tot; p += blockDim.x) {
-            const int z = p / uxy, r = p - z * uxy, y = r / ux, x = r - y * ux;
-            const int gx = ex0 + x, gy = ey0 + y, gz = ez0 + z;
-            double a[NG];
-            point(gx, gy, gz, a);
+    for (int p = threadIdx.x; p < tot; p += blockDim.x) {
+        const int z = p / uxy, r = p - z * uxy, y = r / ux, x = r - y * ux;
+        const int gx = ex0 + x, gy = ey0 + y, gz = ez0 + z;
+        double a[NG];
+        point(gx, gy, gz, a);
 #pragma unroll
-            for (int m = 0; m < NG; ++m) {
-                const unsigned lx = gx - ni[m], ly = gy - nj[m], lz = gz - nk[m];
-                if (on[m] && lx < (unsigned)M && ly < (unsigned)M && lz < (unsigned)M)
-                    out[(size_t)m * M3 + (lz * M2 + ly * M + lx)] = (T)a[m];
-            }
-        }
-    } else {
         for (int m = 0; m < NG; ++m) {
-            if (!on[m]) continue;
-#pragma unroll 1
-            for (int p = threadIdx.x; p < M3; p += blockDim.x) {
-                const int z = p / M2, r = p - z * M2, y = r / M, x = r - y * M;
-                double a[NG];
-                point(ni[m] + x, nj[m] + y, nk[m] + z, a);
-                out[(size_t)m * M3 + p] = (T)a[m];
-            }
+            const unsigned lx = gx - ni[m], ly = gy - nj[m], lz = gz - nk[m];
+            if (on[m] && lx < (unsigned)M && ly < (unsigned)M && lz < (unsigned)M)
+                out[(size_t)m * M3 + (lz * M2 + ly * M + lx)] = (T)a[m];
         }
     }
 }
@@ -1826,13 +1704,14 @@ struct LArgs {
     int n_img;
     const int *img_type, *img_nn, *nlocc, *nproj;
     int *list, *list_cnt, *overflow;
-    int *glist, *glist_cnt;       // [ceil(B/NG)][GLCAP], [ceil(B/NG)]
+    const int *gst;               // [ng + 1] first slot of each group
+    int ng;
+    int *glist, *glist_cnt;       // [ng][GLCAP], [ng]
     // register slots k_projr needs for any group of the batch (a maximum;
     // 99 when the list mixes box sizes) with pr_nw waves walking slabs of
-    // pr_sz planes, pr_pu the slab capacity per plane and member
+    // pr_sz planes
     int *pr_bad;
-    int pr_nw, pr_sz, pr_pu;
-    int pr_mfma;                  // k_projm's member stride (congruent to 8 modulo 32)
+    int pr_nw, pr_sz;
 };
 
 __global__ void k_node_images(LArgs A, int B)
@@ -1867,11 +1746,11 @@ __global__ void k_node_images(LArgs A, int B)
 
 // Images meeting any of the cubes of the NG consecutive slots of a group
 // (the union of their node lists), sorted by z like the node lists.
-__global__ void k_group_images(LArgs A, int B)
+__global__ void k_group_images(LArgs A)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (B + NG - 1) / NG) return;
-    const int b0 = q * NG, gn = min(NG, B - b0);
+    if (q >= A.ng) return;
+    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = A.g.n, nloc = A.g.nloc;
     int ni[NG], nj[NG], nk[NG];
 #pragma unroll
@@ -1906,32 +1785,21 @@ __global__ void k_group_images(LArgs A, int B)
         // the register slots k_projr needs (written as a maximum into
         // pr_bad; 99 when it does not apply): the k-th image of a wave that
         // meets the walk's union takes slot k mod R, so R must exceed k - j
-        // for every earlier one j still alive in the slab where k enters.  Over the union of the
-        // group's cubes when k_projr walks them together, else over each
-        // member's cube (a walk with fewer members clamps to a smaller
-        // z-range and only shortens lives).
+        // for every earlier one j still alive in the slab where k enters (a
+        // walk with fewer members clamps to a smaller z-range and only
+        // shortens lives).
         int need = 1;
         const int nc0 = A.nlocc[A.img_type[L[0]]];
         for (int i = 1; i < cnt; ++i)
             if (A.nlocc[A.img_type[L[i]]] != nc0) need = 99;
         const int w = 2 * nc0 + 1, SZ = A.pr_sz;
-        int x0 = 1 << 30, x1 = -(1 << 30), y0 = 1 << 30, y1 = -(1 << 30);
-        for (int m = 0; m < gn; ++m) {
-            x0 = min(x0, ni[m]); x1 = max(x1, ni[m]); y0 = min(y0, nj[m]); y1 = max(y1, nj[m]);
-        }
-        const int ux = x1 - x0 + 2 * nloc + 1;
-        const int upx = ux + (((w - ux) % 32) + 32) % 32;
-        int slab = upx * (y1 - y0 + 2 * nloc + 1);
-        if (A.pr_mfma) slab += (((8 - slab) % 32) + 32) % 32;
-        const bool together = slab <= A.pr_pu;
-        for (int walk = 0; walk < (together ? 1 : gn) && need < 99; ++walk) {
+        if (need < 99) {
             int uz0 = 1 << 30, uz1 = -(1 << 30), ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30);
-            for (int m = 0; m < gn; ++m)
-                if (together || m == walk) {
-                    uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
-                    ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-                    uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-                }
+            for (int m = 0; m < gn; ++m) {
+                uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
+                ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
+                uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
+            }
             const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
             for (int wv = 0; wv < A.pr_nw; ++wv) {
                 constexpr int WN = 32;   // live images looked back on

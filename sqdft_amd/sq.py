@@ -28,9 +28,10 @@ PRECISIONS = {"fp64": 0, "mixed": 1, "mixed_lanczos": 2}
 
 
 def node_order(n: int) -> np.ndarray:
-    """The order in which sqg_density visits the n^3 FD nodes and cuts them
-    into batches: 4x4x2 bricks of nodes (x fastest inside a brick, bricks x,
-    then y, then z), so that consecutive batch slots hold overlapping cubes."""
+    """The n^3 FD nodes in 4x4x2 bricks (x fastest inside a brick, bricks x,
+    then y, then z), so that consecutive ones hold overlapping cubes: the order
+    in which sqg_density visits them and cuts them into batches when 4 divides
+    n (otherwise it evens the bricks out)."""
     out = []
     for z0 in range(0, n, 2):
         for y0 in range(0, n, 4):

@@ -1,0 +1,44 @@
+"""Grouping of FD nodes for the projections: whatever list the nodes come in
+(brick order, shuffled, far apart, with repeats) and whatever grid side they
+are cut from, a node's bounds and moments are the same bits, and H v agrees
+with the FP64 oracle (1e-12 FP64; 2e-6 with FP32 storage, the bound of one
+FP32 rounding per value through H)."""
+import numpy as np
+import pytest
+
+import helpers as H
+from sqdft_amd.configs import smooth_veff
+from sqdft_amd.sq import SpectralQuadrature
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed", "mixed_lanczos"])
+@pytest.mark.parametrize("elem,n", [("al", 7), ("al", 9), ("lih", 13)])
+def test_moments_do_not_depend_on_the_list(elem, n, prec):
+    print(elem, n, prec, flush=True)
+    S = (H.small_al if elem == "al" else H.small_lih)(n_cell=n)[0]
+    veff = smooth_veff(S)
+    sq = SpectralQuadrature(S, precision=prec)
+    whole = sq.node_moments(veff, np.arange(S.nn))
+    rng = np.random.Generator(np.random.PCG64(n))
+    for nodes in (rng.permutation(S.nn)[: 3 * n], np.arange(0, S.nn, 2 * n + 1), np.array([5, 5, 0, S.nn - 1, 5])):
+        part = sq.node_moments(veff, nodes)
+        for k in ("chi", "zee", "mu", "iters"):
+            assert np.array_equal(part[k], whole[k][nodes]), k
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("elem", ["al", "lih"])
+def test_hsub_of_scattered_nodes(elem, prec, tol):
+    print(elem, prec, flush=True)
+    S, Rcut, T = (H.small_al if elem == "al" else H.small_lih)(n_cell=9)
+    veff, o = smooth_veff(S), H.oracle_for(S, Rcut, T)
+    rng = np.random.Generator(np.random.PCG64(3))
+    nodes = np.concatenate([np.arange(11), rng.integers(0, S.nn, 6), [4, 4]])
+    sq = SpectralQuadrature(S, precision=prec)
+    v = rng.standard_normal((nodes.size, sq.M, sq.M, sq.M))
+    hv = sq.HsubTimesVec(veff, nodes, v)
+    for b, nd in enumerate(nodes):
+        ref = o.hsub(veff, int(nd), v[b].reshape(-1))
+        assert H.rel(hv[b].reshape(-1), ref) < tol
