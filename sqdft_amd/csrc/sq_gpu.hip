@@ -212,8 +212,6 @@ int ensure_batch(sqg_ctx *c, int B)
     HIPCHK(c->NLv.ensure((size_t)B * c->M3 * rs));
     HIPCHK(c->s.ensure((size_t)B * std::max(c->n_ip, 1) * sizeof(double)));
     HIPCHK(c->node_list.ensure((size_t)B * sizeof(int)));
-    HIPCHK(c->list.ensure((size_t)B * LCAP * sizeof(int)));
-    HIPCHK(c->list_cnt.ensure((size_t)B * sizeof(int)));
     HIPCHK(c->flags.ensure(16 * sizeof(int)));
     HIPCHK(c->lred.ensure((size_t)B * ZHALF * 4 * sizeof(double)));
     for (DBuf *d : {&c->aa, &c->bb, &c->dq, &c->eq}) HIPCHK(d->ensure((size_t)B * S * sizeof(double)));
@@ -284,8 +282,6 @@ PArgs<T> pargs(sqg_ctx *c, const int *dn, const int *dd, const T *V)
     A.V = V;
     A.s = c->s.as<double>();
     A.n_ip = std::max(c->n_ip, 1);
-    A.list = c->list.as<int>();
-    A.list_cnt = c->list_cnt.as<int>();
     A.gst = c->gst.as<int>();
     A.glist = c->glist.as<int>();
     A.glist_cnt = c->glist_cnt.as<int>();
@@ -387,9 +383,10 @@ std::vector<int> make_groups(const sqg_ctx *c, const int *nodes, int B)
     return gst;
 }
 
-// Image lists of the B nodes in node_list (per node and per group) on the
-// groups gst; sets ng, gl_max and projr_R.  Overflow goes to flags[0].
-int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst)
+// Image lists of the B nodes in node_list on the groups gst, and per node where
+// node_lists asks for them (the forces); sets ng, gl_max and projr_R.  Overflow
+// goes to flags[0].
+int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
 {
     const int ng = (int)gst.size() - 1;
     c->ng = ng;
@@ -405,7 +402,6 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst)
     L.list_cnt = c->list_cnt.as<int>();
     L.overflow = c->flags.as<int>();
     L.gst = c->gst.as<int>();
-    L.ng = ng;
     L.glist = c->glist.as<int>();
     L.glist_cnt = c->glist_cnt.as<int>();
     // the projection shapes of the phases that will run on these lists (both
@@ -413,20 +409,18 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst)
     const ProjrShape shapes[2] = {projr_shape(c, c->split() ? 4 : c->real_size()), projr_shape(c, 8)};
     const int nsh = c->split() ? 2 : 1;
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)1, 0);
-    hipLaunchKernelGGL(k_node_images, dim3((B + 127) / 128), dim3(128), 0, c->st, L, B);
     bool any_nm = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
         const ProjrShape &ps = shapes[i];
-        LArgs Li = L;
-        if (ps.nm) {
-            Li.pr_bad = c->flags.as<int>() + 4;
-            Li.pr_nw = PROJR_NT / 64; Li.pr_sz = ps.sz;
-            any_nm = true;
-            any_mfma |= ps.mfma != 0;
-        }
-        // a second launch rebuilds the same group lists and adds its slot plan
-        if (i == 0 || ps.nm) hipLaunchKernelGGL(k_group_images, dim3((ng + 63) / 64), dim3(64), 0, c->st, Li);
+        if (!ps.nm) continue;
+        L.pr_bad = c->flags.as<int>() + 4;
+        L.pr_nw = PROJR_NT / 64;
+        L.pr_sz[L.pr_n++] = ps.sz;
+        any_nm = true;
+        any_mfma |= ps.mfma != 0;
     }
+    hipLaunchKernelGGL(k_group_images, dim3(ng), dim3(64), 0, c->st, L);
+    if (node_lists) hipLaunchKernelGGL(k_node_images, dim3(B), dim3(64), 0, c->st, L);
     std::vector<int> gc(ng + 1);
     HIPCHK(hipMemcpyAsync(gc.data(), c->glist_cnt.p, (size_t)ng * sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipMemcpyAsync(gc.data() + ng, c->flags.as<int>() + 4, sizeof(int), hipMemcpyDeviceToHost, c->st));
@@ -446,13 +440,13 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst)
 }
 
 // Groups and image lists of the B nodes in node_list (nodes: their host copy).
-int node_images(sqg_ctx *c, const int *nodes, int B)
+int node_images(sqg_ctx *c, const int *nodes, int B, bool node_lists = false)
 {
     const std::vector<int> gst = make_groups(c, nodes, B);
     HIPCHK(c->gst.ensure(gst.size() * sizeof(int)));
     HIPCHK(c->glist.ensure((gst.size() - 1) * GLCAP * sizeof(int)));
     HIPCHK(c->glist_cnt.ensure((gst.size() - 1) * sizeof(int)));
-    return image_lists(c, B, gst);
+    return image_lists(c, B, gst, node_lists);
 }
 
 // LDS bytes of one k_nlapplyg workgroup (loc table, row offsets, NG values per row)
@@ -1003,8 +997,10 @@ int forces_batch(sqg_ctx *c, int B, const int *hnodes, std::vector<double> &rec)
     const int *dn = c->node_list.as<int>();
     int *flags = c->flags.as<int>();
     HIPCHK(hipMemsetAsync(flags, 0, 16 * sizeof(int), c->st));
+    HIPCHK(c->list.ensure((size_t)B * LCAP * sizeof(int)));
+    HIPCHK(c->list_cnt.ensure((size_t)B * sizeof(int)));
     {
-        const int st = node_images(c, hnodes, B);
+        const int st = node_images(c, hnodes, B, true);
         if (st) return st;
     }
     const size_t vlen = (size_t)B * c->M3;
@@ -1490,9 +1486,9 @@ int sqg_hsub_apply_batch(sqg_ctx *c, const double *veff, const int *nodes, int n
 // own allocations; nothing here allocates or frees).
 struct ScratchView {
     sqg_ctx *c;
-    DBuf *bufs[12];
-    void *saved_p[12];
-    size_t saved_b[12];
+    DBuf *bufs[10];
+    void *saved_p[10];
+    size_t saved_b[10];
     int n = 0;
     size_t off = 0;
     explicit ScratchView(sqg_ctx *c_) : c(c_) {}
@@ -1510,7 +1506,8 @@ struct ScratchView {
 };
 
 // Scratch bytes the allocation-free H v of nb nodes in ng groups needs
-// (per-call buffers rounded to 256 bytes each, without the group table).
+// (per-call buffers rounded to 256 bytes each, without the group table; the
+// LCAP ints a node are part of the limit callers see and are left unused).
 size_t noalloc_bytes(const sqg_ctx *c, int nb, size_t ng)
 {
     auto r = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -1537,8 +1534,6 @@ static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int
     }
     ScratchView V(c);
     V.put(c->node_list, nb * sizeof(int));
-    V.put(c->list, (size_t)nb * LCAP * sizeof(int));
-    V.put(c->list_cnt, nb * sizeof(int));
     V.put(c->gst, gst.size() * sizeof(int));
     V.put(c->glist, ng * GLCAP * sizeof(int));
     V.put(c->glist_cnt, ng * sizeof(int));
@@ -1554,7 +1549,7 @@ static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int
     // flags start at zero (a fill kernel, not a memset node)
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>(), (size_t)16, 0);
     HIPCHK(hipMemcpyAsync(c->node_list.p, nodes, nb * sizeof(int), hipMemcpyHostToDevice, c->st));
-    int st = image_lists(c, nb, gst);
+    int st = image_lists(c, nb, gst, false);
     if (st) return st;
     const int *dn = c->node_list.as<int>();
     auto run = [&](auto tag) {
