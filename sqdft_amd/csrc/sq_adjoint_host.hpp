@@ -78,8 +78,12 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     const int cidx = (c->p.nloc * c->M + c->p.nloc) * c->M + c->p.nloc;
     int st = ensure_batch(c, B);
     if (st) return st;
-    std::vector<int> nodes(B);
+    std::vector<int> nodes(B), slot_of(B);
     for (int i = 0; i < B; ++i) nodes[i] = z0 * n * n + i;
+    NodeOrder(n).sort(nodes);   // brick order: full projection groups
+    for (int i = 0; i < B; ++i) slot_of[nodes[i] - z0 * n * n] = i;
+    HIPCHK(c->adj_slot.ensure((size_t)B * sizeof(int)));
+    HIPCHK(hipMemcpyAsync(c->adj_slot.p, slot_of.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->node_list.p, nodes.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));
     st = batch_images(c, nodes);
     if (st) return st;
@@ -148,8 +152,9 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     }
     hipLaunchKernelGGL((k_adj_center<T>), dim3((B + 127) / 128), dim3(128), 0, c->st, B, (int)M3, cidx,
                        (const T *)tb(1), G);
-    hipLaunchKernelGGL((k_adj_gather<T>), dim3(grid1(c->nn, 256)), dim3(256), 0, c->st, n, c->p.nloc, z0, nz,
-                       (const T *)G, c->zee_all.as<double>(), c->adj_out.as<double>());
+    const int X = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128;   // threads along x
+    hipLaunchKernelGGL((k_adj_gather<T>), dim3(n * n), dim3(AGT), 0, c->st, n, c->p.nloc, z0, nz, X,
+                       c->adj_slot.as<int>(), (const T *)G, c->zee_all.as<double>(), c->adj_out.as<double>());
     int ovf4[4] = {0, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(ovf4, c->flags.p, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     const int ovf = ovf4[0] | ovf4[2] | ovf4[3];

@@ -95,36 +95,58 @@ __global__ void k_adj_center(int B, int M3, int c, const T *tb1, T *G)
 }
 
 // dL/dVeff(g) += sum over the batch's nodes i whose cube holds g of G_i(p)/zee_i.
-// The batch is the nodes of z-planes [z0, z0 + nz) in natural order, so node
-// (x, y, z) sits in slot ((z - z0) n + y) n + x.  Every grid point is owned by
-// one thread, which visits the cube offsets in a fixed order: the sum is
-// deterministic and needs no atomics.
+// The batch is the nodes of z-planes [z0, z0 + nz); slot_of gives the slot of
+// the node at ((z - z0) n + y) n + x.  One workgroup per grid row (gy, gz):
+// thread (x, sub) owns gx = x, x + X, ... and the cube offsets dz = sub mod S,
+// and walks the nodes of each row of nodes, so that neighbouring lanes read
+// neighbouring values of one node's vector (each value is read once: HBM
+// bound).  Every sum runs in a fixed order over its nodes and then over the
+// subs: deterministic, no atomics.  A thread per grid point walked all its
+// (2 nloc + 1)^3 offsets alone, with loads a cube apart between lanes: 24.5 ms
+// for 4,096 nodes with 35^3 cubes (16 workgroups); an adjoint product on the
+// 16^3 Al grid 266 -> 242 ms with this kernel.
+constexpr int AGT = 256;
 template <typename T>
-__global__ void k_adj_gather(int n, int nloc, int z0, int nz, const T *G, const double *zee, double *out)
+__global__ void __launch_bounds__(AGT) k_adj_gather(int n, int nloc, int z0, int nz, int X, const int *slot_of,
+                                                    const T *G, const double *zee, double *out)
 {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nn = n * n * n;
-    if (g >= nn) return;
-    const int M = 2 * nloc + 1, M2 = M * M, M3 = M2 * M;
-    const int gx = g % n, gy = (g / n) % n, gz = g / (n * n);
-    double acc = 0.0;
-    for (int dz = -nloc; dz <= nloc; ++dz) {
-        const int bz = wrapn(gz - dz, n);
-        const int zs = wrapn(bz - z0, n);
-        if (zs >= nz) continue;
-        for (int dy = -nloc; dy <= nloc; ++dy) {
-            const int by = wrapn(gy - dy, n);
-            const size_t rowslot = ((size_t)zs * n + by) * n;
-            const int prow = ((dz + nloc) * M + (dy + nloc)) * M + nloc;
-            for (int dx = -nloc; dx <= nloc; ++dx) {
-                const int bx = wrapn(gx - dx, n);
-                const size_t slot = rowslot + bx;
-                const int node = (bz * n + by) * n + bx;
-                acc += (double)G[slot * M3 + prow + dx] / zee[node];
+    __shared__ double part[AGT];
+    const int gy = blockIdx.x % n, gz = blockIdx.x / n;
+    const int M = 2 * nloc + 1, M2 = M * M;
+    const size_t M3 = (size_t)M2 * M;
+    const int S = AGT / X, sub = threadIdx.x / X, tx = threadIdx.x - sub * X;
+    for (int x0 = 0; x0 < n; x0 += X) {
+        const int gx = x0 + tx;
+        double acc = 0.0;
+        if (sub < S && gx < n) {
+            for (int dz = -nloc + sub; dz <= nloc; dz += S) {
+                const int bz = wrapn(gz - dz, n), zs = bz - z0;
+                if (zs < 0 || zs >= nz) continue;
+                for (int dy = -nloc; dy <= nloc; ++dy) {
+                    const int by = wrapn(gy - dy, n);
+                    const int row = (zs * n + by) * n, zrow = (bz * n + by) * n;
+                    const T *g0 = G + ((dz + nloc) * M + (dy + nloc)) * M + nloc;
+                    for (int bx = 0; bx < n; ++bx) {
+                        const T *g = g0 + slot_of[row + bx] * M3;
+                        const double iz = 1.0 / zee[zrow + bx];
+                        // offsets dx = gx - bx modulo n inside the cube
+                        int dx = gx - bx;
+                        dx -= (dx + nloc) / n * n;
+                        if (dx < -nloc) dx += n;
+                        for (; dx <= nloc; dx += n) acc += (double)g[dx] * iz;
+                    }
+                }
             }
         }
+        part[threadIdx.x] = acc;
+        __syncthreads();
+        if (sub == 0 && gx < n) {
+            double t = acc;
+            for (int k = 1; k < S; ++k) t += part[k * X + tx];
+            out[((size_t)gz * n + gy) * n + gx] += t;
+        }
+        __syncthreads();
     }
-    out[g] += acc;
 }
 
 // ---------------------------------------------------------------- tangent

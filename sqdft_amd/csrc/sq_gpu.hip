@@ -89,7 +89,7 @@ struct sqg_ctx {
     DBuf costab, ynode, scal;
     // Veff derivatives: vectors, per-node sign / d rho/d lambda / weight,
     // n^3 input and output, per-step tangent records
-    DBuf adj, adj_sgn, adj_dl, adj_wt, adj_in, adj_out, adj_rec;
+    DBuf adj, adj_sgn, adj_dl, adj_wt, adj_in, adj_out, adj_rec, adj_slot;
     // AAJ Poisson: iterates, residual, history, rhs, result, block partials
     DBuf pz_phi, pz_new, pz_res, pz_X, pz_F, pz_rhs, pz_out, pz_DX, pz_DF, pz_part;
     // local forces: replica boxes, radial tables, block partials, error flag
