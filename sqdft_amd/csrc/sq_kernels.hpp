@@ -254,6 +254,16 @@ __global__ void __launch_bounds__(512) k_nlapply(NArgs<T> A)
 // cube centre writes the centre value.
 constexpr int ZHALF = 2;
 __host__ __device__ inline int zhalf_rows(int M, int h) { return h == 0 ? (M + 1) / 2 : M / 2; }
+// Workgroup -> (node, half): the halves of a node are eight workgroups apart,
+// so the round-robin over the eight XCDs puts them on the same one at about
+// the same time and the halo rows of one half are L2 hits of the other's.
+__device__ __forceinline__ void zhalf_of(int i, int total, int &b, int &h)
+{
+    const int set = i / (8 * ZHALF), r = i - set * 8 * ZHALF;
+    const int w = min(8, total / ZHALF - 8 * set);   // nodes of this set
+    h = r / w;
+    b = 8 * set + r - h * w;
+}
 
 template <typename T, int MODE>
 __device__ __forceinline__ void zmarch_body(const ZArgs<T> &A)
@@ -264,7 +274,8 @@ __device__ __forceinline__ void zmarch_body(const ZArgs<T> &A)
     constexpr bool YQ = MODE == MODE_LANCZOS && sizeof(T) == 8;
     constexpr unsigned TS = sizeof(T);
     const Geo &G = A.g;
-    const int b = blockIdx.x / ZHALF, h = blockIdx.x % ZHALF;
+    int b, h;
+    zhalf_of((int)blockIdx.x, (int)gridDim.x, b, h);
     if (G.done && G.done[b]) return;
     const int node = G.node_list[b];
     const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, PP = G.pitch;
