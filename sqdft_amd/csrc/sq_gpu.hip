@@ -81,7 +81,7 @@ struct sqg_ctx {
     DBuf gst, glist, glist_cnt;    // first slot of each group, group image lists
     int ng = 0;                    // groups of the current batch
     int gl_max = 0;                // longest group list of the current batch
-    int projr_R = 0;               // k_projr register slots for the batch (0: k_projs instead)
+    int proj_shape = -1;           // compiled shape of k_projr / k_projm for the batch (-1: k_projs instead)
     DBuf lred, aa, bb, dq, eq, lmin, lmax, lmin_prev, lmax_prev, lchg, cnt, done, ca, ib, bprev;
     DBuf chiB, zeeB, center, dots, htemp;
     // all-node state of the last density step
@@ -300,9 +300,18 @@ PArgs<T> pargs(sqg_ctx *c, const int *dn, const int *dd, const T *V)
 
 // Shape of k_projr (s-channel tables only): members per workgroup, register
 // slots per wave and planes per slab; nm = 0 when it does not apply.
-constexpr int PROJR_NT = 512, PROJR_RPI = 3;
-constexpr int PROJR_SLOTS[3] = {5, 10, 16};   // compiled slot counts (five keep FP64 out of scratch)
-constexpr int PROJM_SLOTS = 16;               // k_projm: one double per slot and lane
+constexpr int PROJR_RPI = 3;
+// Compiled shapes, the first that holds every group of the batch is taken:
+// waves per workgroup and register slots per wave.  One workgroup fills a
+// CU's LDS, so its waves are all that hides the loads: twelve, if the four
+// slots that their 168 VGPRs hold are enough (the Al and LiH cells), else eight
+// with more slots.  Twelve against eight, us a pass: 8,192 nodes with FP64
+// 35^3 cubes 1265 against 1549 (Lanczos) and 895 against 1175 (Chebyshev),
+// 4,096 with FP32 ones 468 and 402 against 542 and 488; k_projm, 4,096 nodes
+// with 31^3 cubes, 875 and 862 against 1142 and 1166.
+struct ProjShape { int nw, R; };
+constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
+constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // k_projm: two doubles per slot and lane
 struct ProjrShape { int nm, R, sz, mfma; };
 // ts: bytes per stored value of the phase (4 or 8).
 ProjrShape projr_shape(const sqg_ctx *c, size_t ts)
@@ -384,7 +393,7 @@ std::vector<int> make_groups(const sqg_ctx *c, const int *nodes, int B)
 }
 
 // Image lists of the B nodes in node_list on the groups gst, and per node where
-// node_lists asks for them (the forces); sets ng, gl_max and projr_R.  Overflow
+// node_lists asks for them (the forces); sets ng, gl_max and proj_shape.  Overflow
 // goes to flags[0].
 int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
 {
@@ -408,34 +417,29 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     // stored types in SQG_MIXED_LANCZOS): each plans its register slots
     const ProjrShape shapes[2] = {projr_shape(c, c->split() ? 4 : c->real_size()), projr_shape(c, 8)};
     const int nsh = c->split() ? 2 : 1;
-    hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)1, 0);
+    hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)2, 0);
     bool any_nm = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
         const ProjrShape &ps = shapes[i];
         if (!ps.nm) continue;
-        L.pr_bad = c->flags.as<int>() + 4;
-        L.pr_nw = PROJR_NT / 64;
+        L.pr_need = c->flags.as<int>() + 4;
         L.pr_sz[L.pr_n++] = ps.sz;
         any_nm = true;
         any_mfma |= ps.mfma != 0;
     }
     hipLaunchKernelGGL(k_group_images, dim3(ng), dim3(64), 0, c->st, L);
     if (node_lists) hipLaunchKernelGGL(k_node_images, dim3(B), dim3(64), 0, c->st, L);
-    std::vector<int> gc(ng + 1);
+    std::vector<int> gc(ng + 2);
     HIPCHK(hipMemcpyAsync(gc.data(), c->glist_cnt.p, (size_t)ng * sizeof(int), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(gc.data() + ng, c->flags.as<int>() + 4, sizeof(int), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipMemcpyAsync(gc.data() + ng, c->flags.as<int>() + 4, 2 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->gl_max = 0;
     for (int i = 0; i < ng; ++i) c->gl_max = std::max(c->gl_max, gc[i]);
-    // the smallest slot count that holds every group of the batch: k_projr
-    // gives the same sums with any slot count, so batches stay bitwise alike
-    c->projr_R = 0;
-    if (any_mfma) {
-        if (gc[ng] <= PROJM_SLOTS) c->projr_R = PROJM_SLOTS;
-    } else if (any_nm) {
-        for (int r : PROJR_SLOTS)
-            if (gc[ng] <= r) { c->projr_R = r; break; }
-    }
+    // the sums are the same in every shape, so batches stay bitwise alike
+    c->proj_shape = -1;
+    const ProjShape *sh = any_mfma ? PROJM_SHAPES : PROJR_SHAPES;
+    for (int i = 0; any_nm && i < (any_mfma ? 2 : 4); ++i)
+        if (gc[ng + (sh[i].nw == PROJ_NW[1])] <= sh[i].R) { c->proj_shape = i; break; }
     return SQG_OK;
 }
 
@@ -515,12 +519,15 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
     return false;
 }
 
-template <typename T, int FORMED, int SZ, int R>
+template <typename T, int FORMED, int SZ, bool MFMA, int I>
 void projr_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 {
-    auto fn = k_projr<T, FORMED, SZ, PROJR_NT, R, PROJR_RPI>;
+    constexpr ProjShape S = MFMA ? PROJM_SHAPES[MFMA ? I : 0] : PROJR_SHAPES[I];
+    void (*fn)(PArgs<T>);
+    if constexpr (MFMA) fn = k_projm<T, FORMED, SZ, S.nw * 64, S.R>;
+    else fn = k_projr<T, FORMED, SZ, S.nw * 64, S.R, PROJR_RPI>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(PROJR_NT), shm, c->st, P);
+    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(S.nw * 64), shm, c->st, P);
 }
 
 template <typename T, int FORMED>
@@ -536,16 +543,16 @@ bool launch_projr(sqg_ctx *c, PArgs<T> &P)
     if (ps.sz != SZ) return false;
     if constexpr (sizeof(T) == 8) {
         if (ps.mfma) {
-            auto fn = k_projm<T, FORMED, SZ, PROJR_NT, PROJM_SLOTS>;
-            if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-            hipLaunchKernelGGL(fn, dim3(c->ng), dim3(PROJR_NT), shm, c->st, P);
+            if (c->proj_shape == 0) projr_go<T, FORMED, SZ, true, 0>(c, shm, P);
+            else projr_go<T, FORMED, SZ, true, 1>(c, shm, P);
             return true;
         }
     }
     if (ps.mfma) return false;
-    if (c->projr_R == 5) projr_go<T, FORMED, SZ, 5>(c, shm, P);
-    else if (c->projr_R == 10) projr_go<T, FORMED, SZ, 10>(c, shm, P);
-    else projr_go<T, FORMED, SZ, 16>(c, shm, P);
+    if (c->proj_shape == 0) projr_go<T, FORMED, SZ, false, 0>(c, shm, P);
+    else if (c->proj_shape == 1) projr_go<T, FORMED, SZ, false, 1>(c, shm, P);
+    else if (c->proj_shape == 2) projr_go<T, FORMED, SZ, false, 2>(c, shm, P);
+    else projr_go<T, FORMED, SZ, false, 3>(c, shm, P);
     return true;
 }
 
@@ -563,7 +570,7 @@ void launch_proj(sqg_ctx *c, int B, const PArgs<T> &A, int which = -1, double al
     if (c->n_ip > 0) {
         PArgs<T> P = A;
         const dim3 grid(c->ng);
-        if (c->projr_R && launch_projr<T, FORMED>(c, P)) goto apply;
+        if (c->proj_shape >= 0 && launch_projr<T, FORMED>(c, P)) goto apply;
         const int mp = c->max_nproj <= 1 ? 1 : c->max_nproj <= 4 ? 4 : 0;
         if (mp && launch_projs<T, FORMED>(c, P, mp)) goto apply;
         if (c->max_nproj <= 1)

@@ -1036,7 +1036,9 @@ __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
     constexpr int LV = 3;
     static_assert(NV == 1 << LV, "k_projr: NG is 8");
     constexpr unsigned TS = sizeof(T);
-    constexpr int PPT = 2;                    // staged points per thread per load batch
+    // staged points per thread per load batch (two FP64 vectors of two points
+    // would not fit twelve waves' registers)
+    constexpr int PPT = NT > 512 && FORMED && sizeof(T) == 8 ? 1 : 2;
     const Geo &G = A.g;
     const int q = blockIdx.x;
     const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
@@ -1263,7 +1265,7 @@ __global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
 {
     constexpr int NM = NG;
     constexpr unsigned TS = sizeof(T);
-    constexpr int PPT = 2;
+    constexpr int PPT = NT > 512 && FORMED ? 1 : 2;   // as in k_projr
     const Geo &G = A.g;
     const int q = blockIdx.x;
     const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
@@ -1718,11 +1720,13 @@ struct LArgs {
     const int *gst;               // [groups + 1] first slot of each group
     int *glist, *glist_cnt;       // [groups][GLCAP], [groups]
     // register slots k_projr and k_projm need for any group of the batch (a
-    // maximum; 99 when the list mixes box sizes) with pr_nw waves walking
-    // slabs of pr_sz planes, for each of the pr_n slab depths in use
-    int *pr_bad;
-    int pr_nw, pr_n, pr_sz[2];
+    // maximum; 99 when the list mixes box sizes) with PROJ_NW[0] and
+    // PROJ_NW[1] waves walking slabs of pr_sz planes, for each of the pr_n
+    // slab depths in use
+    int *pr_need;
+    int pr_n, pr_sz[2];
 };
+constexpr int PROJ_NW[2] = {12, 8};
 
 // Images that meet the cube of a node of the block (one wave: gn nodes at
 // most NG), in list order: ids to id, centre z to cz, their number returned
@@ -1822,22 +1826,23 @@ __global__ void __launch_bounds__(64) k_group_images(LArgs A)
         if (bad) atomicOr(A.overflow, 1);
         A.glist_cnt[q] = cnt;
     }
-    if (!A.pr_bad || cnt == 0) return;
+    if (!A.pr_need || cnt == 0) return;
     __syncthreads();   // the sorted list is read back below
     const int nc0 = A.nlocc[A.img_type[id[0]]];
-    int need = 1;
+    int need[2] = {1, 1};
     for (int i = lane; i < cnt; i += 64)
-        if (A.nlocc[A.img_type[id[i]]] != nc0) need = 99;
+        if (A.nlocc[A.img_type[id[i]]] != nc0) need[0] = need[1] = 99;
     // the k-th image of a wave that meets the walk's union takes slot k mod R,
     // so R must exceed k - j for every earlier one j still alive in the slab
     // where k enters (a walk with fewer members clamps to a smaller z-range
-    // and only shortens lives).  Lane l plans wave l.
-    const int w = 2 * nc0 + 1;
-    for (int v = 0; v < A.pr_n && lane < A.pr_nw && need < 99; ++v) {
+    // and only shortens lives).  Lane l plans wave l mod 16 for the wave count
+    // and the slab depth that its quarter stands for.
+    const int w = 2 * nc0 + 1, wv = lane & 15, nv = (lane >> 4) & 1, v = lane >> 5;
+    if (v < A.pr_n && wv < PROJ_NW[nv]) {
         const int SZ = A.pr_sz[v], zs0 = (uz0 + 4096) / SZ * SZ - 4096;
         constexpr int WN = 32;   // live images looked back on
-        int kk[WN], ee[WN], nl = 0, k = -1;
-        for (int li = lane; li < cnt; li += A.pr_nw) {
+        int kk[WN], ee[WN], nl = 0, k = -1, nd = 1;
+        for (int li = wv; li < cnt; li += PROJ_NW[nv]) {
             const int J = L[li];
             const int oz = A.img_nn[3 * J + 2] - nc0, bx0 = A.img_nn[3 * J] - nc0, by0 = A.img_nn[3 * J + 1] - nc0;
             if (oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 || by0 + w - 1 < uy0 || by0 > uy1)
@@ -1849,14 +1854,18 @@ __global__ void __launch_bounds__(64) k_group_images(LArgs A)
             for (int i = 0; i < nl; ++i)
                 if (ee[i] >= S) { kk[j] = kk[i]; ee[j] = ee[i]; ++j; }
             nl = j;
-            if (nl > 0) need = max(need, k - kk[0] + 1);
-            if (nl == WN) { need = 99; break; }
+            if (nl > 0) nd = max(nd, k - kk[0] + 1);
+            if (nl == WN) { nd = 99; break; }
             kk[nl] = k; ee[nl] = E; ++nl;
         }
+        need[nv] = max(need[nv], nd);
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) need = max(need, __shfl_xor(need, o, 64));
-    if (lane == 0) atomicMax(A.pr_bad, need);
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) need[i] = max(need[i], __shfl_xor(need[i], o, 64));
+        if (lane == 0) atomicMax(A.pr_need + i, need[i]);
+    }
 }
 
 // ---------------------------------------------------------------- fills
