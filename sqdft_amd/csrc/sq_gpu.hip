@@ -713,7 +713,7 @@ int lanczos_batch(sqg_ctx *c, int B, long *passes_out)
         launch_zmarch<T, MODE_LANCZOS>(c, B, Z, 1, 4.0 * active * c->M3 * rs);
         passes += active;
         Q.pass = pass;
-        hipLaunchKernelGGL(k_lanczos_scalars, dim3((B + 63) / 64), dim3(64), 0, c->st, Q);
+        hipLaunchKernelGGL(k_lanczos_scalars, dim3((B + LQN - 1) / LQN), dim3(2 * LQN), 0, c->st, Q);
         if (pass >= 1) {
             HIPCHK(hipMemcpyAsync(hdone.data(), ddone, (size_t)B * sizeof(int), hipMemcpyDeviceToHost, c->st));
             HIPCHK(hipStreamSynchronize(c->st));

@@ -1953,158 +1953,139 @@ __device__ int ql_extremes(double *d, double *e, int n, double *lmin, double *lm
     return 0;
 }
 
-// Largest and smallest eigenvalue of the symmetric tridiagonal (d[0..n-1],
-// e[0..n-2], strided by st elements) by Newton's method on det(xI - T).
-// With q_i = p_i/p_{i-1} (Sturm ratios) and r_i = q_i'/q_i, p'/p = sum_i
-// q_i'/q_i; past an extreme root the characteristic polynomial is monotone
-// and convex (concave on the left), so iterates started outside the spectrum
-// move monotonically onto the root, and each stops at the first step that no
-// longer moves inward.  A start xh is outside (above) the spectrum iff every
-// q_i(xh) > 0 (xh I - T positive definite), xl below iff every q_i(xl) < 0.
-// Each side first tries the near start given (just past the previous pass's
-// extreme, which the new one can only exceed), widening the gap 16-fold per
-// failed sweep, and falls back to the far start (a Weyl bound, always
-// outside).  Both sides share every sweep over the rows, which are read in
-// chunks of CH with the next chunk's loads in flight.  Returns false when
-// either needs more than 200 sweeps.
-__device__ bool tridiag_extremes(const double *d, const double *e, size_t st, int n, double fh, double fl,
-                                 double bh, double bl, double gh, double gl, double *hi, double *lo)
+// 1/q to within an ulp or so: the hardware estimate and two Newton steps (a
+// correctly rounded division is a chain three times as long, and the Sturm
+// recurrences below are nothing but such chains).
+__device__ __forceinline__ double recip(double q)
 {
-#pragma clang fp contract(off)
-    constexpr int CH = 8;
-    enum { PROBE = 0, NEWTON = 1, DONE = 2 };
-    // each side starts just past the previous extreme (bh + gh, bl - gl) when
-    // that lies inside the far start, else at the far start
-    int mh = bh + gh < fh ? PROBE : NEWTON, ml = bl - gl > fl ? PROBE : NEWTON;
-    double xh = mh == PROBE ? bh + gh : fh, xl = ml == PROBE ? bl - gl : fl;
+    double r = __builtin_amdgcn_rcp(q);
+    r = fma(fma(-q, r, 1.0), r, r);
+    return fma(fma(-q, r, 1.0), r, r);
+}
+
+// Largest eigenvalue of the symmetric tridiagonal sg T (T: diagonal d(0..n-1),
+// off-diagonal e(0..n-2) through the accessors) by Newton's method on
+// det(xI - sg T).  With q_i = p_i/p_{i-1} (Sturm ratios) and r_i = q_i'/q_i,
+// p'/p = sum_i q_i'/q_i; past the largest root the characteristic polynomial
+// is monotone and convex, so iterates started outside the spectrum move
+// monotonically onto the root; the iteration stops at the first step that is
+// no longer inward by more than rounding.  A start x is outside iff every
+// q_i(x) > 0.  It first tries the near start b + g (just past the previous
+// pass's extreme, which the new one can only exceed), widening the gap 16-fold
+// per failed sweep, and falls back to the far start f (a Weyl bound, always
+// outside).  Returns false after 200 sweeps.
+template <typename D, typename E>
+__device__ bool tridiag_largest(D d, E e, int n, double sg, double f, double b, double g, double *out)
+{
+    bool probe = b + g < f;
+    double x = probe ? b + g : f;
     for (int it = 0; it < 200; ++it) {
-        double qh = xh - d[0], ql = xl - d[0], dqh = 1.0, dql = 1.0;
-        bool ph = qh > 0.0, pl = ql < 0.0;
-        double iqh = 1.0 / qh, iql = 1.0 / ql;
-        double sh = dqh * iqh, sl = dql * iql;
-        double dn[CH], en[CH];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const int i = 1 + j;
-            dn[j] = i < n ? d[(size_t)i * st] : 0.0;
-            en[j] = i < n ? e[(size_t)(i - 1) * st] : 0.0;
+        double q = x - sg * d(0), dq = 1.0, iq = recip(q), s = iq;
+        bool outside = q > 0.0;
+#pragma unroll 4
+        for (int i = 1; i < n; ++i) {
+            const double ei = e(i - 1), r = ei * ei * iq;
+            dq = 1.0 + r * dq * iq;
+            q = (x - sg * d(i)) - r;
+            outside = outside && q > 0.0;
+            iq = recip(q);
+            s += dq * iq;
         }
-        for (int i0 = 1; i0 < n; i0 += CH) {
-            double dc[CH], ec[CH];
-#pragma unroll
-            for (int j = 0; j < CH; ++j) { dc[j] = dn[j]; ec[j] = en[j]; }
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const int i = i0 + CH + j;
-                dn[j] = i < n ? d[(size_t)i * st] : 0.0;
-                en[j] = i < n ? e[(size_t)(i - 1) * st] : 0.0;
-            }
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                if (i0 + j < n) {
-                    const double em2 = ec[j] * ec[j];
-                    const double rh = em2 * iqh, rl = em2 * iql;
-                    dqh = 1.0 + rh * dqh * iqh;
-                    dql = 1.0 + rl * dql * iql;
-                    qh = (xh - dc[j]) - rh;
-                    ql = (xl - dc[j]) - rl;
-                    ph = ph && qh > 0.0;
-                    pl = pl && ql < 0.0;
-                    iqh = 1.0 / qh;
-                    iql = 1.0 / ql;
-                    sh += dqh * iqh;
-                    sl += dql * iql;
-                }
-            }
+        if (probe && !outside) {
+            g *= 16.0;           // inside: widen, or take the far start
+            x = b + g;
+            if (!(x < f)) { x = f; probe = false; }
+            continue;
         }
-        // upper side
-        bool step_h = mh == NEWTON;
-        if (mh == PROBE) {
-            if (ph) {
-                mh = NEWTON;          // outside: Newton from this sweep on
-                step_h = true;
-            } else {
-                gh *= 16.0;           // inside: widen, or take the far start
-                xh = bh + gh;
-                if (!(xh < fh)) { xh = fh; mh = NEWTON; }
-            }
-        }
-        if (step_h) {
-            const double xn = xh - 1.0 / sh;
-            if (!(xn < xh)) { *hi = xh; mh = DONE; }
-            else xh = xn;
-        }
-        // lower side
-        bool step_l = ml == NEWTON;
-        if (ml == PROBE) {
-            if (pl) {
-                ml = NEWTON;
-                step_l = true;
-            } else {
-                gl *= 16.0;
-                xl = bl - gl;
-                if (!(xl > fl)) { xl = fl; ml = NEWTON; }
-            }
-        }
-        if (step_l) {
-            const double xn = xl - 1.0 / sl;
-            if (!(xn > xl)) { *lo = xl; ml = DONE; }
-            else xl = xn;
-        }
-        if (mh == DONE && ml == DONE) return true;
+        probe = false;
+        const double xn = x - recip(s);
+        if (!(xn < x - 2.0e-16 * fabs(x))) { *out = x; return true; }
+        x = xn;
     }
     return false;
 }
 
-__global__ void k_lanczos_scalars(QArgs A)
+// Alpha and beta of a Lanczos pass and the extremes of the grown tridiagonal.
+// Two lanes per node, one per extreme, 32 nodes per wave; the tridiagonals'
+// first LQR rows are copied to LDS at once, so that the sweeps (about six of
+// p + 1 dependent rows, each a reciprocal) wait for no memory.  A pass of 4,096
+// nodes takes 37 us and one of 1,000 nodes 14 us; 245 and 51 us with the rows
+// read from memory sweep by sweep, one lane for both extremes and IEEE
+// divisions.
+constexpr int LQN = 32, LQR = 120;
+__global__ void __launch_bounds__(2 * LQN) k_lanczos_scalars(QArgs A)
 {
-#pragma clang fp contract(off)
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= A.B || A.done[b]) return;
-    const int S = MAXIT + 2;
-    // the two row halves of the z-march, added in half order
-    const double *r0 = A.lred + 8 * (size_t)b, *r1 = r0 + 4;
-    const double r[4] = {r0[0] + r1[0], r0[1] + r1[1], r0[2] + r1[2], r0[3] + r1[3]};
-    const int p = A.pass;
-    const double al = r[0];
-    double b2 = r[1] - 2.0 * al * r[2] + al * al * r[3];
-    if (b2 < 0.0) b2 = 0.0;
-    const double be = sqrt(b2);
+    __shared__ double sd[LQR][LQN], se[LQR][LQN];
+    const int nb = threadIdx.x >> 1, b = blockIdx.x * LQN + nb;
+    const bool act = b < A.B && !A.done[b];
+    if (__ballot(act) == 0) return;
+    const int S = MAXIT + 2, p = A.pass, nq = p + 1;
     const size_t st = (size_t)A.B;
-    A.aa[(size_t)p * st + b] = al;
-    A.bb[(size_t)p * st + b] = be;
-    A.ca[b] = al;
-    A.ib[b] = 1.0 / be;
-    A.bprev[b] = be;
+    {   // rows 0 .. p - 1 of this block's nodes (row p is made below)
+        const int l = threadIdx.x & (LQN - 1), bl = min(blockIdx.x * LQN + l, A.B - 1);
+        const int rows = min(p, LQR);
+        for (int i = threadIdx.x / LQN; i < rows; i += 2) {
+            sd[i][l] = A.aa[(size_t)i * st + bl];
+            se[i][l] = A.bb[(size_t)i * st + bl];
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    const bool low = threadIdx.x & 1;   // this lane's extreme: the smallest
+    // the two row halves of the z-march, added in half order
+    double al, be;
+    {
+#pragma clang fp contract(off)
+        const double *r0 = A.lred + 8 * (size_t)b, *r1 = r0 + 4;
+        const double r[4] = {r0[0] + r1[0], r0[1] + r1[1], r0[2] + r1[2], r0[3] + r1[3]};
+        al = r[0];
+        double b2 = r[1] - 2.0 * al * r[2] + al * al * r[3];
+        if (b2 < 0.0) b2 = 0.0;
+        be = sqrt(b2);
+    }
+    if (!low) {
+        A.aa[(size_t)p * st + b] = al;
+        A.bb[(size_t)p * st + b] = be;
+        A.ca[b] = al;
+        A.ib[b] = 1.0 / be;
+        A.bprev[b] = be;
+    }
     if (p == 0) return;
-    const int nq = p + 1;
     // Extreme eigenvalues of the (p+1)-sized tridiagonal.  The reference runs
     // the full QL (TridiagEigenSolve, sq.cpp:1094-1180) every pass; only the
     // extremes are used, and adding row p moves them by at most |beta_{p-1}|
     // beyond max(lambda_max(T_p), alpha_p) (min for lambda_min), which gives
     // Newton a start outside the spectrum.  QL stays as the fallback.
     const double *ad = A.aa + b, *be2 = A.bb + b;   // row i at [i * st]
-    double lo, hi, up, dn;
-    if (p == 1) {   // Gershgorin
-        const double r = fabs(be2[0]);
-        up = fmax(ad[0], ad[st]) + r;
-        dn = fmin(ad[0], ad[st]) - r;
+    auto d = [&](int i) { return i == p ? al : i < LQR ? sd[i][nb] : ad[(size_t)i * st]; };
+    auto e = [&](int i) { return i < LQR ? se[i][nb] : be2[(size_t)i * st]; };
+    const double sg = low ? -1.0 : 1.0;   // the smallest of T is the largest of -T
+    const double rad = fabs(e(p - 1));
+    const double last = p == 1 ? sg * d(0) : sg * (low ? A.lmin_prev[b] : A.lmax_prev[b]);
+    double far = fmax(last, sg * al) + rad;   // pass 1: Gershgorin
+    far += 8.0 * 2.2e-16 * fabs(far) + 1e-300;
+    // near start: past the previous extreme by twice its last change (pass 1
+    // has none: the Gershgorin bound)
+    const double bx = p == 1 ? far : last;
+    const double gap = 2.0 * A.lchg[2 * (size_t)b + low] + 1e-13 * (fabs(bx) + 1.0);
+    double x = 0.0;
+    bool ok;
+    if (p < LQR) {
+        sd[p][nb] = al;
+        ok = tridiag_largest([&](int i) { return sd[i][nb]; }, [&](int i) { return se[i][nb]; }, nq, sg, far, bx,
+                             gap, &x);
     } else {
-        const double r = fabs(be2[(size_t)(p - 1) * st]);
-        up = fmax(A.lmax_prev[b], ad[(size_t)p * st]) + r;
-        dn = fmin(A.lmin_prev[b], ad[(size_t)p * st]) - r;
+        ok = tridiag_largest(d, e, nq, sg, far, bx, gap, &x);
     }
-    up += 8.0 * 2.2e-16 * fabs(up) + 1e-300;
-    dn -= 8.0 * 2.2e-16 * fabs(dn) + 1e-300;
-    // near starts: past the previous extremes by twice their last change
-    // (pass 1 has no previous extremes: the Gershgorin bounds)
-    const double bh = p == 1 ? up : A.lmax_prev[b], bl = p == 1 ? dn : A.lmin_prev[b];
-    const double gh = 2.0 * A.lchg[2 * (size_t)b] + 1e-13 * (fabs(bh) + 1.0);
-    const double gl = 2.0 * A.lchg[2 * (size_t)b + 1] + 1e-13 * (fabs(bl) + 1.0);
-    if (!tridiag_extremes(ad, be2, st, nq, up, dn, bh, bl, gh, gl, &hi, &lo)) {
-        double *d = A.d + (size_t)b * S, *e = A.e + (size_t)b * S;
-        for (int i = 0; i < nq; ++i) { d[i] = ad[(size_t)i * st]; e[i] = be2[(size_t)i * st]; }
-        if (ql_extremes(d, e, nq, &lo, &hi)) { atomicOr(A.err, 1); A.done[b] = 1; return; }
+    // lane pairs: (largest, smallest) to both
+    const double mine = sg * x, other = __shfl_xor(mine, 1, 64);
+    const bool okb = __shfl_xor((int)ok, 1, 64) && ok;
+    if (low) return;
+    double hi = mine, lo = other;
+    if (!okb) {
+        double *dd = A.d + (size_t)b * S, *ee = A.e + (size_t)b * S;
+        for (int i = 0; i < nq; ++i) { dd[i] = ad[(size_t)i * st]; ee[i] = be2[(size_t)i * st]; }
+        if (ql_extremes(dd, ee, nq, &lo, &hi)) { atomicOr(A.err, 1); A.done[b] = 1; return; }
     }
     const double dl = fabs(lo - A.lmin_prev[b]), dm = fabs(hi - A.lmax_prev[b]);
     A.lmin_prev[b] = lo;
