@@ -81,7 +81,7 @@ struct sqg_ctx {
     DBuf gst, glist, glist_cnt;    // first slot of each group, group image lists
     int ng = 0;                    // groups of the current batch
     int gl_max = 0;                // longest group list of the current batch
-    int proj_shape = -1;           // compiled shape of k_projr / k_projm for the batch (-1: k_projs instead)
+    int proj_shape = -1;           // compiled shape of k_projw for the batch (-1: k_projs instead)
     DBuf lred, aa, bb, dq, eq, lmin, lmax, lmin_prev, lmax_prev, lchg, cnt, done, ca, ib, bprev;
     DBuf chiB, zeeB, center, dots, htemp;
     // all-node state of the last density step
@@ -298,55 +298,74 @@ PArgs<T> pargs(sqg_ctx *c, const int *dn, const int *dd, const T *V)
     return A;
 }
 
-// Shape of k_projr (s-channel tables only): members per workgroup, register
-// slots per wave and planes per slab; nm = 0 when it does not apply.
-constexpr int PROJR_RPI = 3;
-// Compiled shapes, the first that holds every group of the batch is taken:
-// waves per workgroup and register slots per wave.  One workgroup fills a
-// CU's LDS, so its waves are all that hides the loads: twelve, if the four
-// slots that their 168 VGPRs hold are enough (the Al and LiH cells), else eight
-// with more slots.  Twelve against eight, us a pass: 8,192 nodes with FP64
-// 35^3 cubes 1265 against 1549 (Lanczos) and 895 against 1175 (Chebyshev),
-// 4,096 with FP32 ones 468 and 402 against 542 and 488; k_projm, 4,096 nodes
-// with 31^3 cubes, 875 and 862 against 1142 and 1166.
+// Compiled shapes of k_projw, the first that holds every group of the batch is
+// taken: waves per workgroup and register slots per wave.  One workgroup fills
+// a CU's LDS, so its waves are all that hides the loads: twelve, if the slots
+// that their 168 VGPRs hold are enough (the Al and LiH cells), else eight with
+// more slots.  Twelve against eight, us a pass: 8,192 nodes with FP64 35^3
+// cubes 1265 against 1549 (Lanczos) and 895 against 1175 (Chebyshev), 4,096
+// with FP32 ones 468 and 402 against 542 and 488; MFMA, 4,096 nodes with 31^3
+// cubes, 875 and 862 against 1142 and 1166.  With the union columns worked out
+// once per walk the twelve-wave ones take 1192, 863, 459, 358, 838 and 760.
+constexpr int PROJW_RPI = 3;
 struct ProjShape { int nw, R; };
 constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
-constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // k_projm: two doubles per slot and lane
-struct ProjrShape { int nm, R, sz, mfma; };
-// ts: bytes per stored value of the phase (4 or 8).
-ProjrShape projr_shape(const sqg_ctx *c, size_t ts)
+constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // MFMA: two doubles per slot and lane
+
+// How k_projw runs on vectors of ts bytes per value: on = 0 when it does not
+// apply; the matrix cores for FP64 tables of several projectors.
+struct ProjwUse { int on, mfma, w; };
+ProjwUse projw_use(const sqg_ctx *c, size_t ts)
 {
-    if (c->max_nproj < 1 || c->max_nproj > 4 || c->n_ip == 0) return {0, 0, 0, 0};
-    // p channels in FP64: k_projm on the matrix cores.  FP32 tables (mixed
-    // precision) stay with k_projs: its VALU sums of FP32 operands ran at
-    // 1.18 ms a pass on the 216-atom LiH batches against k_projm's 1.67 ms
-    // (FP64 MFMAs fed by conversions), while in FP64 the two tie (2.3 ms).
-    if (c->max_nproj > 1 && ts == 4) return {0, 0, 0, 0};
+    if (c->max_nproj < 1 || c->max_nproj > 4 || c->n_ip == 0) return {0, 0, 0};
+    // p channels in FP64: the matrix cores.  FP32 tables (mixed precision)
+    // stay with k_projs: its VALU sums of FP32 operands ran at 1.18 ms a pass
+    // on the 216-atom LiH batches against 1.67 ms (FP64 MFMAs fed by
+    // conversions), while in FP64 the two tied (2.3 ms).
+    if (c->max_nproj > 1 && ts == 4) return {0, 0, 0};
     const int mfma = c->max_nproj > 1;
     int w = 0;
     for (int t = 0; t < c->n_typ; ++t)
         if (c->h_nproj[t] > 0) w = std::max(w, 2 * c->h_nlocc[t] + 1);
-    if (mfma ? w > 16 : w * w > 64 * PROJR_RPI) return {0, 0, 0, 0};
-    // eight members per workgroup; FP32 slabs of two planes fit the LDS
-    return {8, 0, ts == 4 ? 2 : 1, mfma};
+    if (mfma ? w > 16 : w * w > 64 * PROJW_RPI) return {0, 0, 0};
+    return {1, mfma, w};
 }
 
-// LDS values per plane and member of a staged block of ux x uy points: rows
-// padded to a pitch congruent to the box side modulo 32 (as k_projr and
-// k_projm pad them), k_projm's member stride congruent to 8.
-int projr_slab(const sqg_ctx *c, const ProjrShape &ps, int ux, int uy)
+// LDS values per plane and member of a staged block of ux x uy columns: rows
+// padded to a pitch congruent to the box side modulo 32, the MFMA member
+// stride to 8 (as k_projw pads them).
+int projw_slab(const ProjwUse &pw, int ux, int uy)
 {
-    int wbox = 0;
-    for (int t = 0; t < c->n_typ; ++t)
-        if (c->h_nproj[t] > 0) wbox = 2 * c->h_nlocc[t] + 1;
-    const int u = (ux + (((wbox - ux) % 32) + 32) % 32) * uy;
-    return ps.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
+    const int u = (ux + (((pw.w - ux) % 32) + 32) % 32) * uy;
+    return pw.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
 }
 
-// k_projr's slab capacity: the union plane of a 4x2 block of cubes or one cube.
-int projr_pu(const sqg_ctx *c, const ProjrShape &ps)
+// Slab capacity per plane and member: the union plane of a 4x2 block of cubes
+// or one cube.
+int projw_pu(const sqg_ctx *c, const ProjwUse &pw)
 {
-    return std::max(projr_slab(c, ps, c->M + 3, c->M + 1), projr_slab(c, ps, c->M, c->M));
+    return std::max(projw_slab(pw, c->M + 3, c->M + 1), projw_slab(pw, c->M, c->M));
+}
+
+// LDS bytes of k_projw beside the slab: image data and union columns.
+size_t projw_head(const sqg_ctx *c, int gl_max)
+{
+    return ((size_t)std::max(gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16 +
+           (std::max((size_t)(c->M + 3) * (c->M + 3), (size_t)(c->M + 7) * c->M) * 4 + 15) / 16 * 16;
+}
+
+// Planes per slab.  VALU: one FP64 or two FP32 planes (a deeper slab keeps more
+// images alive than the slots of twelve waves: 17^3 cubes with three planes
+// took 269 us a pass with ten slots in eight waves against 81).  MFMA, whose
+// slots are small: about four load rounds of a workgroup between two barriers,
+// at most eight planes, as far as the LDS holds them beside a list of 256
+// images (25^3 cubes, two planes: 373 against 496 us a pass).
+int projw_sz(const sqg_ctx *c, const ProjwUse &pw, size_t ts)
+{
+    const size_t plane = (size_t)projw_pu(c, pw) * NG * ts, head = projw_head(c, 256);
+    const int lds = plane + head <= 160 * 1024 ? (int)((160 * 1024 - head) / plane) : 1;
+    if (!pw.mfma) return ts == 4 ? 2 : 1;
+    return std::max(1, std::min({8, lds, 3072 / ((c->M + 3) * (c->M + 1))}));
 }
 
 // k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
@@ -364,12 +383,12 @@ int projs_pu(const sqg_ctx *c) { return (c->M + 3) * (c->M + 3); }
 std::vector<int> make_groups(const sqg_ctx *c, const int *nodes, int B)
 {
     const int n = c->p.n, M = c->M;
-    const ProjrShape shapes[2] = {projr_shape(c, c->split() ? 4 : c->real_size()), projr_shape(c, 8)};
+    const ProjwUse use[2] = {projw_use(c, c->split() ? 4 : c->real_size()), projw_use(c, 8)};
     const int nsh = c->split() ? 2 : 1;
     auto fits = [&](int dx, int dy, int dz) {
         if (dz > 1 || (M + dx) * (M + dy) > projs_pu(c)) return false;
         for (int i = 0; i < nsh; ++i)
-            if (shapes[i].nm && projr_slab(c, shapes[i], M + dx, M + dy) > projr_pu(c, shapes[i])) return false;
+            if (use[i].on && projw_slab(use[i], M + dx, M + dy) > projw_pu(c, use[i])) return false;
         return true;
     };
     std::vector<int> gst{0};
@@ -415,17 +434,17 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     L.glist_cnt = c->glist_cnt.as<int>();
     // the projection shapes of the phases that will run on these lists (both
     // stored types in SQG_MIXED_LANCZOS): each plans its register slots
-    const ProjrShape shapes[2] = {projr_shape(c, c->split() ? 4 : c->real_size()), projr_shape(c, 8)};
+    const size_t ts[2] = {c->split() ? 4 : c->real_size(), 8};
     const int nsh = c->split() ? 2 : 1;
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)2, 0);
-    bool any_nm = false, any_mfma = false;
+    bool any_on = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
-        const ProjrShape &ps = shapes[i];
-        if (!ps.nm) continue;
+        const ProjwUse pw = projw_use(c, ts[i]);
+        if (!pw.on) continue;
         L.pr_need = c->flags.as<int>() + 4;
-        L.pr_sz[L.pr_n++] = ps.sz;
-        any_nm = true;
-        any_mfma |= ps.mfma != 0;
+        L.pr_sz[L.pr_n++] = projw_sz(c, pw, ts[i]);
+        any_on = true;
+        any_mfma |= pw.mfma != 0;
     }
     hipLaunchKernelGGL(k_group_images, dim3(ng), dim3(64), 0, c->st, L);
     if (node_lists) hipLaunchKernelGGL(k_node_images, dim3(B), dim3(64), 0, c->st, L);
@@ -438,7 +457,7 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     // the sums are the same in every shape, so batches stay bitwise alike
     c->proj_shape = -1;
     const ProjShape *sh = any_mfma ? PROJM_SHAPES : PROJR_SHAPES;
-    for (int i = 0; any_nm && i < (any_mfma ? 2 : 4); ++i)
+    for (int i = 0; any_on && i < (any_mfma ? 2 : 4); ++i)
         if (gc[ng + (sh[i].nw == PROJ_NW[1])] <= sh[i].R) { c->proj_shape = i; break; }
     return SQG_OK;
 }
@@ -519,40 +538,35 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
     return false;
 }
 
-template <typename T, int FORMED, int SZ, bool MFMA, int I>
-void projr_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
+template <typename T, int FORMED, bool MFMA, int I>
+void projw_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 {
     constexpr ProjShape S = MFMA ? PROJM_SHAPES[MFMA ? I : 0] : PROJR_SHAPES[I];
-    void (*fn)(PArgs<T>);
-    if constexpr (MFMA) fn = k_projm<T, FORMED, SZ, S.nw * 64, S.R>;
-    else fn = k_projr<T, FORMED, SZ, S.nw * 64, S.R, PROJR_RPI>;
+    auto fn = k_projw<T, FORMED, S.nw * 64, S.R, PROJW_RPI, MFMA, MFMA ? 0 : sizeof(T) == 4 ? 2 : 1>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     hipLaunchKernelGGL(fn, dim3(c->ng), dim3(S.nw * 64), shm, c->st, P);
 }
 
 template <typename T, int FORMED>
-bool launch_projr(sqg_ctx *c, PArgs<T> &P)
+bool launch_projw(sqg_ctx *c, PArgs<T> &P)
 {
-    const ProjrShape ps = projr_shape(c, sizeof(T));
-    const size_t sa = ((size_t)std::max(c->gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16;
-    const int pu = projr_pu(c, ps);
-    const size_t shm = sa + (size_t)pu * ps.nm * sizeof(T) * ps.sz;
+    const ProjwUse pw = projw_use(c, sizeof(T));
+    if (!pw.on) return false;
+    P.sz = projw_sz(c, pw, sizeof(T));
+    const size_t shm = projw_head(c, c->gl_max) + (size_t)projw_pu(c, pw) * NG * sizeof(T) * P.sz;
     if (shm > 160 * 1024) return false;
-    P.pu = pu;
-    constexpr int SZ = sizeof(T) == 8 ? 1 : 2;
-    if (ps.sz != SZ) return false;
     if constexpr (sizeof(T) == 8) {
-        if (ps.mfma) {
-            if (c->proj_shape == 0) projr_go<T, FORMED, SZ, true, 0>(c, shm, P);
-            else projr_go<T, FORMED, SZ, true, 1>(c, shm, P);
+        if (pw.mfma) {
+            if (c->proj_shape == 0) projw_go<T, FORMED, true, 0>(c, shm, P);
+            else projw_go<T, FORMED, true, 1>(c, shm, P);
             return true;
         }
     }
-    if (ps.mfma) return false;
-    if (c->proj_shape == 0) projr_go<T, FORMED, SZ, false, 0>(c, shm, P);
-    else if (c->proj_shape == 1) projr_go<T, FORMED, SZ, false, 1>(c, shm, P);
-    else if (c->proj_shape == 2) projr_go<T, FORMED, SZ, false, 2>(c, shm, P);
-    else projr_go<T, FORMED, SZ, false, 3>(c, shm, P);
+    if (pw.mfma) return false;
+    if (c->proj_shape == 0) projw_go<T, FORMED, false, 0>(c, shm, P);
+    else if (c->proj_shape == 1) projw_go<T, FORMED, false, 1>(c, shm, P);
+    else if (c->proj_shape == 2) projw_go<T, FORMED, false, 2>(c, shm, P);
+    else projw_go<T, FORMED, false, 3>(c, shm, P);
     return true;
 }
 
@@ -570,7 +584,7 @@ void launch_proj(sqg_ctx *c, int B, const PArgs<T> &A, int which = -1, double al
     if (c->n_ip > 0) {
         PArgs<T> P = A;
         const dim3 grid(c->ng);
-        if (c->proj_shape >= 0 && launch_projr<T, FORMED>(c, P)) goto apply;
+        if (c->proj_shape >= 0 && launch_projw<T, FORMED>(c, P)) goto apply;
         const int mp = c->max_nproj <= 1 ? 1 : c->max_nproj <= 4 ? 4 : 0;
         if (mp && launch_projs<T, FORMED>(c, P, mp)) goto apply;
         if (c->max_nproj <= 1)

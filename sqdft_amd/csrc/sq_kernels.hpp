@@ -156,14 +156,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t brsrc(const void *p, size_t by
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
 }
-template <typename T> __device__ __forceinline__ T bload(__amdgpu_buffer_rsrc_t r, unsigned off);
-template <> __device__ __forceinline__ float bload<float>(__amdgpu_buffer_rsrc_t r, unsigned off)
+template <typename T> __device__ __forceinline__ T bload(__amdgpu_buffer_rsrc_t r, unsigned off, int soff = 0);
+template <> __device__ __forceinline__ float bload<float>(__amdgpu_buffer_rsrc_t r, unsigned off, int soff)
 {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
 }
-template <> __device__ __forceinline__ double bload<double>(__amdgpu_buffer_rsrc_t r, unsigned off)
+template <> __device__ __forceinline__ double bload<double>(__amdgpu_buffer_rsrc_t r, unsigned off, int soff)
 {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
 }
 __device__ __forceinline__ int bload_i32(__amdgpu_buffer_rsrc_t r, unsigned off)
 {
@@ -592,7 +592,8 @@ struct PArgs {
     const double *ca, *ib;        // LANCZOS: projects v = (V - ca V2) * ib
     const int *gst;               // [groups + 1] first slot of each group
     const int *glist, *glist_cnt; // group image lists
-    int pu;                       // staged kernels: LDS values per plane and member
+    int pu;                       // k_projs: LDS values per plane and member
+    int sz;                       // k_projw: planes per slab
 };
 
 // Projections s[b][ip] = <U_ip, v_b>/Denom over the intersection of the
@@ -1015,61 +1016,86 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 
 // The projections of k_projs with every image owned by one wave for its
 // whole z-extent.  The workgroup walks the union of its members' cubes in
-// slabs of SZ planes staged in LDS as in k_projs; image li of the z-sorted
-// group list belongs to wave li mod nwave, and the k-th of a wave's images
-// that meets the walk's union holds that wave's register slot k mod R from
-// the slab where its box enters the union to the slab where it leaves.  Lane l keeps, for each slot, the partial sums of the
-// box points whose xy index is l mod 64 over every plane, so the wave reduces
-// (wave_sums) and stores each projection once, when its image leaves: no
-// per-slab reduction, no atomics, no zeroing pass.  Per lane and member the
-// products are added plane by plane, z ascending, in the same round order
-// for every grouping of the nodes, so each member's totals depend only on its
-// own cube.  An image whose box misses the union in z contributes zero.
-// Requires one box size for every image of the list and R larger than the
-// slot distance of any two images of a wave alive at once (k_group_images
-// computes the R a batch needs; the host picks a compiled R at least that).
-template <typename T, int FORMED, int SZ, int NT, int R, int RPI>
-__global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
+// slabs of A.sz planes (global z multiples of A.sz) staged in LDS member-major
+// with zeros outside a member's cube; image li of the z-sorted group list
+// belongs to wave li mod nwave, and the k-th of a wave's images that meets the
+// union holds that wave's register slot k mod R from the slab where its box
+// enters the union to the slab where it leaves, so each projection is reduced
+// and stored once: no per-slab reduction, no atomics, no zeroing pass.  Sums
+// run plane by plane, z ascending, whatever the slab depth, in an order that
+// depends on the image's box alone, so each member's totals depend only on its
+// own cube.  An image whose box misses the union contributes zero.  Requires
+// one box size for every image of the list and R larger than the slot distance
+// of any two images of a wave alive at once (k_group_images computes the R a
+// batch needs; the host picks a compiled R at least that).
+//
+// MFMA = 0, tables of one projector (the s channel): lane l keeps, for each
+// slot and member, the partial sums of the box points whose xy index is l mod
+// 64 (RPI rounds of 64 cover the box plane); wave_sums adds the lanes when the
+// image leaves.
+// MFMA = 1, FP64 tables of up to four projectors (the p channel): every slot
+// owns two FP64 4x4x4 MFMA accumulators (four 4x4 blocks, one double per
+// lane).  Block b = q + 2 ph multiplies members 4q..4q+3 (rows) by the image's
+// projectors (columns) over four box points (K) of phase ph: a box row of side
+// w <= 16 is covered by two MFMAs, point x = 8 hh + 4 ph + k, each into its own
+// accumulator (two independent chains).  The accumulators and the two phases
+// are added when the image leaves the union (lane l + lane l ^ 8).  Operands: A
+// = the member's staged value at the point, B = the projector value (zero past
+// the box or the union).  Lane layout of v_mfma_f64_4x4x4f64 on gfx950:
+// A[b][i][k] at lane 16k + 4b + i, B[b][k][j] at 16k + 4b + j, D[b][i][j] at
+// 16i + 4b + j.
+//
+// LDS rows are padded to a pitch congruent to the box side modulo 32 values, so
+// that the box rows one wave reads fall on disjoint banks; with MFMA the member
+// stride is congruent to 8, so that the 8 members of a point do.  Bound by the
+// vectors' HBM reads and, since one workgroup fills a CU's LDS, by what its
+// waves overlap; which members hold a union column and where it sits is worked
+// out once per walk (xyt), not per plane and member.
+// SZC: planes per slab, 0: A.sz (a loop of unknown length over a slot's planes
+// costs the VALU shapes the registers of their slots).
+template <typename T, int FORMED, int NT, int R, int RPI, bool MFMA, int SZC>
+__global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
 {
     constexpr int NM = NG;
-    constexpr int NV = NM;                    // one projector per image (s channel)
     constexpr int LV = 3;
-    static_assert(NV == 1 << LV, "k_projr: NG is 8");
+    static_assert(NM == 1 << LV, "k_projw: NG is 8");
     constexpr unsigned TS = sizeof(T);
-    // staged points per thread per load batch (two FP64 vectors of two points
-    // would not fit twelve waves' registers)
-    constexpr int PPT = NT > 512 && FORMED && sizeof(T) == 8 ? 1 : 2;
+    // staged points per thread per load batch (two would not fit the registers
+    // of twelve waves beside the VALU slots)
+    constexpr int PPT = NT > 512 && (!MFMA || FORMED) ? 1 : 2;
+    constexpr int NW = NT / 64;
     const Geo &G = A.g;
     const int q = blockIdx.x;
     const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
-    const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
+    const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3, SZ = SZC ? SZC : A.sz;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int NW = NT / 64;
     int ni[NM], nj[NM], nk[NM];
-    bool on[NM];
     T cab[NM], ibb[NM];
-    int nact = 0;
     unsigned onmask = 0;
+    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        on[m] = m < gn && !(G.done && G.done[b0 + m]);
         const int node = G.node_list[b0 + min(m, gn - 1)];
         ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
         cab[m] = 0; ibb[m] = 1;
-        if (on[m]) {
-            ++nact;
+        if (m < gn && !(G.done && G.done[b0 + m])) {
             onmask |= 1u << m;
             if (FORMED) { cab[m] = (T)A.ca[b0 + m]; ibb[m] = (T)A.ib[b0 + m]; }
+            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
+            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
+            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
         }
     }
     const int cnt = A.glist_cnt[q];
-    if (nact == 0 || cnt == 0) return;
-    // LDS: image data [cnt] | staged slab [SZ][NM][padded plane]
+    if (onmask == 0 || cnt == 0) return;
+    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, np_ = ux * uy;
+    // LDS: image data [cnt] | union columns [np_] | staged slab [SZ][NM][ms]
     extern __shared__ unsigned char smem_raw[];
     ImgMeta *im = reinterpret_cast<ImgMeta *>(smem_raw);
-    T *pl = reinterpret_cast<T *>(smem_raw + ((size_t)cnt * sizeof(ImgMeta) + 15) / 16 * 16);
-    for (int li = tid; li < cnt; li += blockDim.x) {
+    unsigned *xyt = reinterpret_cast<unsigned *>(smem_raw + ((size_t)cnt * sizeof(ImgMeta) + 15) / 16 * 16);
+    T *pl = reinterpret_cast<T *>(reinterpret_cast<unsigned char *>(xyt) + ((size_t)np_ * 4 + 15) / 16 * 16);
+    for (int li = tid; li < cnt; li += NT) {
         const int J = A.glist[(size_t)q * GLCAP + li];
         const int t = A.img_type[J], nc = A.nlocc[t];
         ImgMeta e;
@@ -1078,83 +1104,98 @@ __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
         e.uoff = A.udv_off[J];
         im[li] = e;
     }
-    __syncthreads();
-    const size_t gb = (size_t)gn * M3 * TS;
-    const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3, gb);
-    const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3, gb);
-    // LDS rows of the slab are padded to a pitch congruent to the box side
-    // modulo 32 values, so that the box rows one wave reads fall on disjoint
-    // banks
-    const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
-    auto upitch_of = [&](int u) { return u + (((wbox - u) % 32) + 32) % 32; };
-    // the value this lane stores for a leaving image: member kw
-    const int kw = lane >> (6 - LV);
-    const bool wlane = (lane & ((64 >> LV) - 1)) == 0;
-    double *sw = A.s + (size_t)(b0 + kw) * A.n_ip;
-    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
+    // union column -> x, y (12 bits each) and the members whose cube holds it
+    for (int p = tid; p < np_; p += NT) {
+        const int yy = p / ux, xx = p - yy * ux;
+        unsigned v = (unsigned)xx | (unsigned)yy << 12;
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        if (on[m]) {
-            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
-        }
+        for (int m = 0; m < NM; ++m)
+            if (((onmask >> m) & 1u) && (unsigned)(ux0 + xx - ni[m] + nloc) < (unsigned)M &&
+                (unsigned)(uy0 + yy - nj[m] + nloc) < (unsigned)M)
+                v |= 1u << (24 + m);
+        xyt[p] = v;
     }
-    const bool writer = wlane && ((onmask >> kw) & 1u);
-    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), up = upx * uy;
-    const int np_ = ux * uy, sp = SZ * np_;   // staged points of a slab (unpadded)
+    __syncthreads();
+    // A column's offset in a member's vector is its offset in the union plus a
+    // constant of the member, the scalar offset of the loads; the resources
+    // start pad values early so that none is negative (the masks keep every
+    // address inside the member's cube)
+    const int pad = M2 + M + 8;
+    const size_t gb = ((size_t)gn * M3 + pad) * TS;
+    const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3 - pad, gb);
+    const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3 - pad, gb);
+    int kof[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+        kof[m] = (pad + m * M3 + (uz0 - nk[m] + nloc) * M2 + (uy0 - nj[m] + nloc) * M + ux0 - ni[m] + nloc) * (int)TS;
+    const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
+    const int upx = ux + (((wbox - ux) % 32) + 32) % 32, up = upx * uy;
+    const int ms = MFMA ? up + (((8 - up) % 32) + 32) % 32 : up;
+    // MFMA lane roles: K index, block (member quad, point phase), row/column
+    const int kk = lane >> 4, bb = (lane >> 2) & 3, ii = lane & 3;
+    const int mA = 4 * (bb & 1) + ii;          // member of the lane's A value
+    const int bxl0 = 4 * (bb >> 1) + kk;       // box x of the lane's point, first MFMA of a row
+    // member (and projector jw) whose total this lane stores for a leaving image
+    const int mw = MFMA ? 4 * ((lane >> 2) & 1) + (lane >> 4) : lane >> (6 - LV), jw = lane & 3;
+    const bool writer = (MFMA ? (lane & 8) == 0 : (lane & ((64 >> LV) - 1)) == 0) && ((onmask >> mw) & 1u);
+    double *sw = A.s + (size_t)(b0 + mw) * A.n_ip;
     const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
-    // per-wave slot state: images started (slotted or not), slotted
-    // images, live-slot mask, per-slot image data
+    // per-wave slot state: images started (slotted or not), slotted images,
+    // live-slot mask, per-slot image data
     int nstart = 0, nslot = 0;
     unsigned live = 0;
-    int s_oz[R], s_ze[R], s_w[R], s_ipb[R], s_t[R];
+    int s_oz[R], s_ze[R], s_ipb[R], s_t[R], s_np[R], s_ox[R], s_oy[R];
     long s_uoff[R];
-    int s_pp[R][RPI];                     // LDS point of the lane's box point, or -1
-    double acc[R][NM];
+    int s_pp[MFMA ? 1 : R][RPI];               // LDS point of the lane's box point, or -1
+    double acc[R][MFMA ? 2 : NM];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        s_oz[r] = s_ze[r] = s_w[r] = s_ipb[r] = s_t[r] = 0;
+        s_oz[r] = s_ze[r] = s_ipb[r] = s_t[r] = s_np[r] = s_ox[r] = s_oy[r] = 0;
         s_uoff[r] = 0;
+        if constexpr (!MFMA) {
 #pragma unroll
-        for (int k = 0; k < RPI; ++k) s_pp[r][k] = -1;
+            for (int k = 0; k < RPI; ++k) s_pp[r][k] = -1;
+        }
 #pragma unroll
-        for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
+        for (int m = 0; m < (MFMA ? 2 : NM); ++m) acc[r][m] = 0.0;
     }
 #pragma unroll 1
     for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
         // the previous slab is consumed before it is overwritten
         __syncthreads();
 #pragma unroll 1
-        for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
-            T xv[PPT][NM], yv[PPT][NM];
+        for (int sl = 0; sl < SZ; ++sl) {
+            const int gz = gzs + sl;
+            unsigned zm = 0;                   // members that hold the plane
 #pragma unroll
-            for (int r = 0; r < PPT; ++r) {
-                const int p = p0 + r * (int)blockDim.x + tid;
-                const int sl = p / np_, pq = p - sl * np_;
-                const int yy = pq / ux, xx = pq - yy * ux;
-                const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
+            for (int m = 0; m < NM; ++m)
+                if ((unsigned)(gz - nk[m] + nloc) < (unsigned)M) zm |= 1u << (24 + m);
+            T *dpl = pl + (size_t)sl * NM * ms;
+#pragma unroll 1
+            for (int p0 = 0; p0 < np_; p0 += PPT * NT) {
+                T xv[PPT][NM], yv[PPT][NM];
+                unsigned cv[PPT];
 #pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
-                    const bool ok = p < sp && on[m] && (unsigned)lx < (unsigned)M &&
-                                    (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
-                    const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
-                    xv[r][m] = bload<T>(rX, o);
-                    yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                for (int r = 0; r < PPT; ++r) {
+                    const int p = p0 + r * NT + tid;
+                    cv[r] = p < np_ ? xyt[p] : 0;
+                    const unsigned co = (unsigned)((gz - uz0) * M2 + (int)((cv[r] >> 12) & 4095) * M + (int)(cv[r] & 4095)) * TS;
+                    const unsigned mk = cv[r] & zm;
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) {
+                        const unsigned o = (mk & (1u << (24 + m))) ? co : OOB;
+                        xv[r][m] = bload<T>(rX, o, kof[m]);
+                        yv[r][m] = FORMED ? bload<T>(rY, o, kof[m]) : (T)0;
+                    }
                 }
-            }
 #pragma unroll
-            for (int r = 0; r < PPT; ++r) {
-                const int p = p0 + r * (int)blockDim.x + tid;
-                if (p < sp) {
-                    // member-major: [plane][member][row][padded column]
-                    const int sl = p / np_, pq = p - sl * np_;
-                    const int yy = pq / ux, xx = pq - yy * ux;
-                    T *dst = pl + (size_t)sl * NM * up + yy * upx + xx;
+                for (int r = 0; r < PPT; ++r) {
+                    if (p0 + r * NT + tid < np_) {
+                        T *dst = dpl + (int)((cv[r] >> 12) & 4095) * upx + (int)(cv[r] & 4095);
 #pragma unroll
-                    for (int m = 0; m < NM; ++m)
-                        dst[(size_t)m * up] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
+                        for (int m = 0; m < NM; ++m)
+                            dst[(size_t)m * ms] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
+                    }
                 }
             }
         }
@@ -1165,45 +1206,48 @@ __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
         for (;;) {
             const int li = wave + NW * nstart;
             if (li >= cnt) break;
+            const int w = wbox;
             const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
-            const int w = __builtin_amdgcn_readfirstlane(im[li].w);
-            const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
-            const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
-                              by0 + w - 1 < uy0 || by0 > uy1;
-            const int zs = max(oz, uz0);
-            if (!miss && zs > zl) break;
-            if (miss) {   // the box misses the union: the projection is zero
-                const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
-                if (writer) sw[ipb] = 0.0;
+            const int ox = __builtin_amdgcn_readfirstlane(im[li].ox), oy = __builtin_amdgcn_readfirstlane(im[li].oy);
+            const bool miss = oz + w - 1 < uz0 || oz > uz1 || ox + w - 1 < ux0 || ox > ux1 ||
+                              oy + w - 1 < uy0 || oy > uy1;
+            if (!miss && max(oz, uz0) > zl) break;
+            const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
+            const int np = MFMA ? __builtin_amdgcn_readfirstlane(im[li].np) : 1;
+            if (miss) {   // the box misses the union: the projections are zero
+                if (writer && (!MFMA || jw < np)) sw[ipb + (MFMA ? jw : 0)] = 0.0;
                 ++nstart;
                 continue;
             }
             const int slot = nslot % R;
             ++nslot;
-            const int ox = __builtin_amdgcn_readfirstlane(im[li].ox), oy = __builtin_amdgcn_readfirstlane(im[li].oy);
-            const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
-            const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
-            const float rw = 1.0f / (float)w;
             int pp[RPI];
+            if constexpr (!MFMA) {
+                const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
+                const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
+                const float rw = 1.0f / (float)w;
 #pragma unroll
-            for (int k = 0; k < RPI; ++k) {
-                const int a = 64 * k + lane;
-                const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
-                const bool in = a < w * w && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
-                pp[k] = in ? (oy + by - uy0) * upx + (ox + bx - ux0) : -1;
+                for (int k = 0; k < RPI; ++k) {
+                    const int a = 64 * k + lane;
+                    const int by = (int)(((float)a + 0.5f) * rw), bx = a - by * w;
+                    const bool in = a < w * w && by >= rlo && by <= rhi && bx >= clo && bx <= chi;
+                    pp[k] = in ? (oy + by - uy0) * upx + (ox + bx - ux0) : -1;
+                }
             }
-            const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb), t = __builtin_amdgcn_readfirstlane(im[li].t);
+            const int t = __builtin_amdgcn_readfirstlane(im[li].t);
             const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
                                      (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 if (r == slot) {
-                    s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_w[r] = w; s_ipb[r] = ipb; s_t[r] = t;
-                    s_uoff[r] = uoff;
+                    s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_ipb[r] = ipb; s_t[r] = t; s_np[r] = np;
+                    s_ox[r] = ox; s_oy[r] = oy; s_uoff[r] = uoff;
+                    if constexpr (!MFMA) {
 #pragma unroll
-                    for (int k = 0; k < RPI; ++k) s_pp[r][k] = pp[k];
+                        for (int k = 0; k < RPI; ++k) s_pp[r][k] = pp[k];
+                    }
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) acc[r][m] = 0.0;
+                    for (int m = 0; m < (MFMA ? 2 : NM); ++m) acc[r][m] = 0.0;
                 }
             }
             live |= 1u << slot;
@@ -1213,267 +1257,88 @@ __global__ void __launch_bounds__(NT) k_projr(PArgs<T> A)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (!((live >> r) & 1u)) continue;
-            const int w = s_w[r], w2 = w * w;
+            const int w = wbox, w2 = w * w, w3 = w2 * w;
             const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
-            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)w2 * w * TS);
-            for (int z = za; z <= zb; ++z) {
-                const int bz = z - s_oz[r];
-                T u[RPI];
+            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)s_np[r] * w3 * TS);
+            if constexpr (MFMA) {
+                const int ox = s_ox[r], oy = s_oy[r];
+                const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
+                const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
+                const bool colj = ii < s_np[r];
+                bool okx[2];
 #pragma unroll
-                for (int k = 0; k < RPI; ++k)
-                    u[k] = bload<T>(rU, s_pp[r][k] >= 0 ? (unsigned)(bz * w2 + 64 * k + lane) * TS : OOB);
+                for (int hh = 0; hh < 2; ++hh) okx[hh] = bxl0 + 8 * hh >= clo && bxl0 + 8 * hh <= chi;
+                for (int z = za; z <= zb; ++z) {
+                    const int bz = z - s_oz[r];
+                    const T *pz = pl + (size_t)(z - gzs) * NM * ms + (size_t)mA * ms;
+                    // rows in chunks of RC, the next chunk's operands loaded
+                    // while the current chunk's MFMAs run
+                    constexpr int RC = 4;
+                    T an[RC][2], bn[RC][2];
+                    auto load_rows = [&](int by0) {
 #pragma unroll
-                for (int k = 0; k < RPI; ++k) {
-                    const T *pv = pl + (size_t)(z - gzs) * NM * up + max(s_pp[r][k], 0);
-                    T v[NM];
+                        for (int j = 0; j < RC; ++j) {
+                            const int by = by0 + j;
+                            const bool rowok = by <= rhi;
+                            const int lrow = (oy + by - uy0) * upx + (ox - ux0);
+                            const int urow = ii * w3 + bz * w2 + by * w;
 #pragma unroll
-                    for (int m = 0; m < NM; ++m) v[m] = pv[(size_t)m * up];
-                    if (s_pp[r][k] >= 0) {
+                            for (int hh = 0; hh < 2; ++hh) {
+                                const int bx = bxl0 + 8 * hh;
+                                const bool ok = rowok && okx[hh];
+                                an[j][hh] = ok ? pz[lrow + bx] : (T)0;
+                                bn[j][hh] = bload<T>(rU, (ok && colj) ? (unsigned)(urow + bx) * TS : OOB);
+                            }
+                        }
+                    };
+                    load_rows(rlo);
+                    for (int by0 = rlo; by0 <= rhi; by0 += RC) {
+                        T ac[RC][2], bc[RC][2];
 #pragma unroll
-                        for (int m = 0; m < NM; ++m) acc[r][m] += (double)v[m] * (double)u[k];
+                        for (int j = 0; j < RC; ++j)
+#pragma unroll
+                            for (int hh = 0; hh < 2; ++hh) { ac[j][hh] = an[j][hh]; bc[j][hh] = bn[j][hh]; }
+                        if (by0 + RC <= rhi) load_rows(by0 + RC);
+#pragma unroll
+                        for (int j = 0; j < RC; ++j) {
+                            if (by0 + j <= rhi) {
+#pragma unroll
+                                for (int hh = 0; hh < 2; ++hh)
+                                    acc[r][hh] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)ac[j][hh], (double)bc[j][hh],
+                                                                                    acc[r][hh], 0, 0, 0);
+                            }
+                        }
+                    }
+                }
+            } else {
+                for (int z = za; z <= zb; ++z) {
+                    const int bz = z - s_oz[r];
+                    T u[RPI];
+#pragma unroll
+                    for (int k = 0; k < RPI; ++k)
+                        u[k] = bload<T>(rU, s_pp[r][k] >= 0 ? (unsigned)(bz * w2 + 64 * k + lane) * TS : OOB);
+#pragma unroll
+                    for (int k = 0; k < RPI; ++k) {
+                        const T *pv = pl + (size_t)(z - gzs) * NM * ms + max(s_pp[r][k], 0);
+                        T v[NM];
+#pragma unroll
+                        for (int m = 0; m < NM; ++m) v[m] = pv[(size_t)m * ms];
+                        if (s_pp[r][k] >= 0) {
+#pragma unroll
+                            for (int m = 0; m < NM; ++m) acc[r][m] += (double)v[m] * (double)u[k];
+                        }
                     }
                 }
             }
             if (s_ze[r] <= zl) {   // the image leaves the union in this slab
-                const double tot = wave_sums<NV>(acc[r], lane);
-                if (writer) sw[s_ipb[r]] = tot * A.inv_denom[16 * s_t[r]];
-                live &= ~(1u << r);
-            }
-        }
-    }
-}
-
-// The projections of k_projr for tables of up to four projectors (the p
-// channel), accumulated on the matrix cores: every live image of a wave owns
-// one FP64 4x4x4 MFMA accumulator (four 4x4 blocks, one double per lane).
-// Block b = q + 2 ph multiplies members 4q..4q+3 (rows) by the image's
-// projectors (columns) over four box points (K) of phase ph: a box row of
-// side w <= 16 is covered by two MFMAs, point x = 8 hh + 4 ph + k, each into
-// its own accumulator (two independent chains).  The accumulators and the
-// two phases are added when the image leaves the union (lane l + lane l ^ 8),
-// so each total is one fixed sum of MFMA partial sums.  Operands: A = the
-// member's staged value at the point (LDS, member-major, member stride
-// congruent to 8 modulo 32 values so that the 8 members of one point fall on
-// distinct banks), B = the projector value (zero past the box or the
-// union).  A member's row of the product depends only on its own values, so
-// each member's totals are independent of the grouping.  Slot plan, walks and
-// staging as in k_projr.  Lane layout of v_mfma_f64_4x4x4f64 on gfx950:
-// A[b][i][k] at lane 16k + 4b + i, B[b][k][j] at 16k + 4b + j, D[b][i][j] at
-// 16i + 4b + j.
-template <typename T, int FORMED, int SZ, int NT, int R>
-__global__ void __launch_bounds__(NT) k_projm(PArgs<T> A)
-{
-    constexpr int NM = NG;
-    constexpr unsigned TS = sizeof(T);
-    constexpr int PPT = NT > 512 && FORMED ? 1 : 2;   // as in k_projr
-    const Geo &G = A.g;
-    const int q = blockIdx.x;
-    const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
-    const int n = G.n, nloc = G.nloc, M = G.M, M2 = G.M2, M3 = G.M3;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    constexpr int NW = NT / 64;
-    int ni[NM], nj[NM], nk[NM];
-    bool on[NM];
-    T cab[NM], ibb[NM];
-    int nact = 0;
-    unsigned onmask = 0;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        on[m] = m < gn && !(G.done && G.done[b0 + m]);
-        const int node = G.node_list[b0 + min(m, gn - 1)];
-        ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
-        cab[m] = 0; ibb[m] = 1;
-        if (on[m]) {
-            ++nact;
-            onmask |= 1u << m;
-            if (FORMED) { cab[m] = (T)A.ca[b0 + m]; ibb[m] = (T)A.ib[b0 + m]; }
-        }
-    }
-    const int cnt = A.glist_cnt[q];
-    if (nact == 0 || cnt == 0) return;
-    // LDS: image data [cnt] | staged slab [SZ][NM][member stride]
-    extern __shared__ unsigned char smem_raw[];
-    ImgMeta *im = reinterpret_cast<ImgMeta *>(smem_raw);
-    T *pl = reinterpret_cast<T *>(smem_raw + ((size_t)cnt * sizeof(ImgMeta) + 15) / 16 * 16);
-    for (int li = tid; li < cnt; li += blockDim.x) {
-        const int J = A.glist[(size_t)q * GLCAP + li];
-        const int t = A.img_type[J], nc = A.nlocc[t];
-        ImgMeta e;
-        e.ox = A.img_nn[3 * J] - nc; e.oy = A.img_nn[3 * J + 1] - nc; e.oz = A.img_nn[3 * J + 2] - nc;
-        e.w = 2 * nc + 1; e.np = A.nproj[t]; e.t = t; e.ipb = A.ip_base[J];
-        e.uoff = A.udv_off[J];
-        im[li] = e;
-    }
-    __syncthreads();
-    const size_t gb = (size_t)gn * M3 * TS;
-    const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3, gb);
-    const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3, gb);
-    const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
-    auto upitch_of = [&](int u) { return u + (((wbox - u) % 32) + 32) % 32; };
-    auto mstride_of = [&](int u) { return u + (((8 - u) % 32) + 32) % 32; };
-    // lane roles in the MFMA: K index, block (member quad, point phase), row/column
-    const int kk = lane >> 4, bb = (lane >> 2) & 3, ii = lane & 3;
-    const int mA = 4 * (bb & 1) + ii;          // member of the lane's A value
-    const int bxl0 = 4 * (bb >> 1) + kk;       // box x of the lane's point, first MFMA of a row
-    // writers of the totals: lanes of phase 0; member 4q + i, projector j
-    const int mw = 4 * ((lane >> 2) & 1) + (lane >> 4), jw = lane & 3;
-    const bool wl = (lane & 8) == 0;
-    double *sw = A.s + (size_t)(b0 + mw) * A.n_ip;
-    int ux0 = 1 << 30, ux1 = -(1 << 30), uy0 = 1 << 30, uy1 = -(1 << 30), uz0 = 1 << 30, uz1 = -(1 << 30);
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-        if (on[m]) {
-            ux0 = min(ux0, ni[m] - nloc); ux1 = max(ux1, ni[m] + nloc);
-            uy0 = min(uy0, nj[m] - nloc); uy1 = max(uy1, nj[m] + nloc);
-            uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
-        }
-    }
-    const bool writer = wl && ((onmask >> mw) & 1u);
-    const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, upx = upitch_of(ux), ms = mstride_of(upx * uy);
-    const int np_ = ux * uy, sp = SZ * np_;
-    const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
-    int nstart = 0, nslot = 0;
-    unsigned live = 0;
-    int s_oz[R], s_ze[R], s_ipb[R], s_t[R], s_np[R], s_ox[R], s_oy[R];
-    long s_uoff[R];
-    double cacc[R][2];   // per slot: the first and second MFMA of each box row
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        s_oz[r] = s_ze[r] = s_ipb[r] = s_t[r] = s_np[r] = s_ox[r] = s_oy[r] = 0;
-        s_uoff[r] = 0;
-        cacc[r][0] = cacc[r][1] = 0.0;
-    }
-#pragma unroll 1
-    for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
-        __syncthreads();
-#pragma unroll 1
-        for (int p0 = 0; p0 < sp; p0 += PPT * (int)blockDim.x) {
-            T xv[PPT][NM], yv[PPT][NM];
-#pragma unroll
-            for (int r = 0; r < PPT; ++r) {
-                const int p = p0 + r * (int)blockDim.x + tid;
-                const int sl = p / np_, pq = p - sl * np_;
-                const int yy = pq / ux, xx = pq - yy * ux;
-                const int gx = ux0 + xx, gy = uy0 + yy, gz = gzs + sl;
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    const int lx = gx - ni[m] + nloc, ly = gy - nj[m] + nloc, lz = gz - nk[m] + nloc;
-                    const bool ok = p < sp && on[m] && (unsigned)lx < (unsigned)M &&
-                                    (unsigned)ly < (unsigned)M && (unsigned)lz < (unsigned)M;
-                    const unsigned o = ok ? (unsigned)(m * M3 + lz * M2 + ly * M + lx) * TS : OOB;
-                    xv[r][m] = bload<T>(rX, o);
-                    yv[r][m] = FORMED ? bload<T>(rY, o) : (T)0;
+                if constexpr (MFMA) {   // add the partial sums and store
+                    const double c = acc[r][0] + acc[r][1];
+                    const double tot = c + __shfl_xor(c, 8, 64);
+                    if (writer && jw < s_np[r]) sw[s_ipb[r] + jw] = tot * A.inv_denom[16 * s_t[r] + jw];
+                } else {
+                    const double tot = wave_sums<NM>(acc[r], lane);
+                    if (writer) sw[s_ipb[r]] = tot * A.inv_denom[16 * s_t[r]];
                 }
-            }
-#pragma unroll
-            for (int r = 0; r < PPT; ++r) {
-                const int p = p0 + r * (int)blockDim.x + tid;
-                if (p < sp) {
-                    const int sl = p / np_, pq = p - sl * np_;
-                    const int yy = pq / ux, xx = pq - yy * ux;
-                    T *dst = pl + (size_t)sl * NM * ms + yy * upx + xx;
-#pragma unroll
-                    for (int m = 0; m < NM; ++m)
-                        dst[(size_t)m * ms] = FORMED ? (xv[r][m] - cab[m] * yv[r][m]) * ibb[m] : xv[r][m];
-                }
-            }
-        }
-        __syncthreads();
-        const int zl = gzs + SZ - 1;
-#pragma unroll 1
-        for (;;) {
-            const int li = wave + NW * nstart;
-            if (li >= cnt) break;
-            const int oz = __builtin_amdgcn_readfirstlane(im[li].oz);
-            const int w = wbox;
-            const int bx0 = __builtin_amdgcn_readfirstlane(im[li].ox), by0 = __builtin_amdgcn_readfirstlane(im[li].oy);
-            const bool miss = oz + w - 1 < uz0 || oz > uz1 || bx0 + w - 1 < ux0 || bx0 > ux1 ||
-                              by0 + w - 1 < uy0 || by0 > uy1;
-            const int zs = max(oz, uz0);
-            if (!miss && zs > zl) break;
-            const int ipb = __builtin_amdgcn_readfirstlane(im[li].ipb);
-            const int np = __builtin_amdgcn_readfirstlane(im[li].np);
-            if (miss) {   // the box misses the union: the projections are zero
-                if (writer && jw < np) sw[ipb + jw] = 0.0;
-                ++nstart;
-                continue;
-            }
-            const int slot = nslot % R;
-            ++nslot;
-            const int t = __builtin_amdgcn_readfirstlane(im[li].t);
-            const long uoff = (long)(((unsigned long)(unsigned)__builtin_amdgcn_readfirstlane((int)(im[li].uoff >> 32)) << 32) |
-                                     (unsigned)__builtin_amdgcn_readfirstlane((int)im[li].uoff));
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                if (r == slot) {
-                    s_oz[r] = oz; s_ze[r] = min(oz + w - 1, uz1); s_ipb[r] = ipb; s_t[r] = t; s_np[r] = np;
-                    s_ox[r] = bx0; s_oy[r] = by0; s_uoff[r] = uoff;
-                    cacc[r][0] = cacc[r][1] = 0.0;
-                }
-            }
-            live |= 1u << slot;
-            ++nstart;
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (!((live >> r) & 1u)) continue;
-            const int w = wbox, w2 = w * w, w3 = w2 * w;
-            const int ox = s_ox[r], oy = s_oy[r];
-            const int za = max(gzs, max(s_oz[r], uz0)), zb = min(zl, s_ze[r]);
-            const int rlo = max(0, uy0 - oy), rhi = min(w - 1, uy1 - oy);
-            const int clo = max(0, ux0 - ox), chi = min(w - 1, ux1 - ox);
-            const __amdgpu_buffer_rsrc_t rU = brsrc(A.udv + s_uoff[r], (size_t)s_np[r] * w3 * TS);
-            const bool colj = ii < s_np[r];
-            bool okx[2];
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh) okx[hh] = bxl0 + 8 * hh >= clo && bxl0 + 8 * hh <= chi;
-            for (int z = za; z <= zb; ++z) {
-                const int bz = z - s_oz[r];
-                const T *pz = pl + (size_t)(z - gzs) * NM * ms + (size_t)mA * ms;
-                // rows in chunks of RC, the next chunk's operands loaded
-                // while the current chunk's MFMAs run
-                constexpr int RC = 4;
-                T an[RC][2], bn[RC][2];
-                auto load_rows = [&](int by0) {
-#pragma unroll
-                    for (int j = 0; j < RC; ++j) {
-                        const int by = by0 + j;
-                        const bool rowok = by <= rhi;
-                        const int lrow = (oy + by - uy0) * upx + (ox - ux0);
-                        const int urow = ii * w3 + bz * w2 + by * w;
-#pragma unroll
-                        for (int hh = 0; hh < 2; ++hh) {
-                            const int bx = bxl0 + 8 * hh;
-                            const bool ok = rowok && okx[hh];
-                            an[j][hh] = ok ? pz[lrow + bx] : (T)0;
-                            bn[j][hh] = bload<T>(rU, (ok && colj) ? (unsigned)(urow + bx) * TS : OOB);
-                        }
-                    }
-                };
-                load_rows(rlo);
-                for (int by0 = rlo; by0 <= rhi; by0 += RC) {
-                    T ac[RC][2], bc[RC][2];
-#pragma unroll
-                    for (int j = 0; j < RC; ++j)
-#pragma unroll
-                        for (int hh = 0; hh < 2; ++hh) { ac[j][hh] = an[j][hh]; bc[j][hh] = bn[j][hh]; }
-                    if (by0 + RC <= rhi) load_rows(by0 + RC);
-#pragma unroll
-                    for (int j = 0; j < RC; ++j) {
-                        if (by0 + j <= rhi) {
-#pragma unroll
-                            for (int hh = 0; hh < 2; ++hh)
-                                cacc[r][hh] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)ac[j][hh], (double)bc[j][hh],
-                                                                                 cacc[r][hh], 0, 0, 0);
-                        }
-                    }
-                }
-            }
-            if (s_ze[r] <= zl) {   // the image leaves the union: add the partial sums and store
-                const double c = cacc[r][0] + cacc[r][1];
-                const double tot = c + __shfl_xor(c, 8, 64);
-                if (writer && jw < s_np[r]) sw[s_ipb[r] + jw] = tot * A.inv_denom[16 * s_t[r] + jw];
                 live &= ~(1u << r);
             }
         }
@@ -1719,7 +1584,7 @@ struct LArgs {
     int *list, *list_cnt, *overflow;   // [B][LCAP], [B] (k_node_images)
     const int *gst;               // [groups + 1] first slot of each group
     int *glist, *glist_cnt;       // [groups][GLCAP], [groups]
-    // register slots k_projr and k_projm need for any group of the batch (a
+    // register slots k_projw needs for any group of the batch (a
     // maximum; 99 when the list mixes box sizes) with PROJ_NW[0] and
     // PROJ_NW[1] waves walking slabs of pr_sz planes, for each of the pr_n
     // slab depths in use
