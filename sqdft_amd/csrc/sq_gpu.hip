@@ -91,7 +91,7 @@ struct sqg_ctx {
     // n^3 input and output, per-step tangent records
     DBuf adj, adj_sgn, adj_dl, adj_wt, adj_in, adj_out, adj_rec, adj_slot;
     // AAJ Poisson: iterates, residual, history, rhs, result, block partials
-    DBuf pz_phi, pz_new, pz_res, pz_X, pz_F, pz_rhs, pz_out, pz_DX, pz_DF, pz_part;
+    DBuf pz_phi, pz_new, pz_res, pz_X, pz_F, pz_rhs, pz_out, pz_DX, pz_DF, pz_part, pz_ctl;
     // local forces: replica boxes, radial tables, block partials, error flag
     DBuf lf_V, lf_Vt, lf_bJ, lf_bJt, lf_img, lf_R, lf_RV, lf_DV, lf_RU, lf_DU, lf_toff, lf_tsize, lf_Z, lf_part, lf_err;
     bool have_state = false;

@@ -35,8 +35,17 @@ __device__ __forceinline__ void grid_block_sum(double (&v)[NV], double *red /* [
         }
 }
 
+// Where the iteration stands: set by k_aaj_check, read by every later kernel
+// of the solve, so that the host enqueues the iterations up to the next
+// Anderson step at once and waits once for all of them.
+struct AajCtl {
+    int done, iter;               // the iteration whose residual met tol, or the last one
+    double r;                     // its relative residual
+};
+
 struct AajArgs {
     int n;
+    const AajCtl *ctl;
     double lap[FDN + 1];
     const double *phi, *rhs;
     double *phinew, *res;
@@ -52,11 +61,14 @@ struct AajArgs {
 __global__ void __launch_bounds__(PB) k_aaj_step(AajArgs A)
 {
     __shared__ double red[PB / 64];
+    if (A.ctl->done) return;
     const int n = A.n;
     const size_t N = (size_t)n * n * n;
     double acc[1] = {0.0};
     for (size_t c = blockIdx.x * (size_t)PB + threadIdx.x; c < N; c += (size_t)gridDim.x * PB) {
-        const int i = (int)(c % n), j = (int)((c / n) % n), k = (int)(c / ((size_t)n * n));
+        // 32-bit indices (n^3 < 2^28): 64-bit divisions are long instruction chains
+        const unsigned row = (unsigned)c / n;
+        const int i = (int)((unsigned)c - row * n), k = (int)(row / n), j = (int)(row - (unsigned)k * n);
         const double *P = A.phi;
         double L = P[c] * 3 * A.lap[0];
 #pragma unroll
@@ -64,9 +76,9 @@ __global__ void __launch_bounds__(PB) k_aaj_step(AajArgs A)
             const int im = i - a < 0 ? i - a + n : i - a, ip = i + a >= n ? i + a - n : i + a;
             const int jm = j - a < 0 ? j - a + n : j - a, jp = j + a >= n ? j + a - n : j + a;
             const int km = k - a < 0 ? k - a + n : k - a, kp = k + a >= n ? k + a - n : k + a;
-            const size_t rowk = (size_t)k * n;
+            const int rowk = k * n;
             L += (P[(rowk + j) * n + im] + P[(rowk + j) * n + ip] + P[(rowk + jm) * n + i] + P[(rowk + jp) * n + i] +
-                  P[((size_t)km * n + j) * n + i] + P[((size_t)kp * n + j) * n + i]) *
+                  P[(km * n + j) * n + i] + P[(kp * n + j) * n + i]) *
                  A.lap[a];
         }
         const double r = -(((4 * M_PI) * (A.rhs[c]) + L) / (3 * A.lap[0]));
@@ -84,13 +96,33 @@ __global__ void __launch_bounds__(PB) k_aaj_step(AajArgs A)
     if (threadIdx.x == 0) A.part[blockIdx.x] = acc[0];
 }
 
+// Relative residual of iteration `iter` from its block partials; stops the
+// solve where it meets tol or iter is the last.
+__global__ void __launch_bounds__(PB) k_aaj_check(const double *part, int nb, double rn, double tol, int iter,
+                                                  int last, AajCtl *ctl)
+{
+    __shared__ double red[PB / 64];
+    if (ctl->done) return;
+    double v[1] = {0.0};
+    for (int i = threadIdx.x; i < nb; i += PB) v[0] += part[i];
+    grid_block_sum<1>(v, red);
+    if (threadIdx.x == 0) {
+        const double r = sqrt(v[0]) / rn;
+        ctl->r = r;
+        ctl->iter = iter;
+        ctl->done = !(r > tol) || last;
+    }
+}
+
 // Partial sums of DF_i . DF_j (i <= j < m) and DF_j . r for the Anderson step
 // (AndersonExtrapolation, src/anderson.cpp:20-100).
 template <int M>
-__global__ void __launch_bounds__(PB) k_aaj_gram(const double *DF, const double *res, size_t N, double *part)
+__global__ void __launch_bounds__(PB) k_aaj_gram(const AajCtl *ctl, const double *DF, const double *res, size_t N,
+                                                 double *part)
 {
     constexpr int NV = M * (M + 1) / 2 + M;
     __shared__ double red[(PB / 64) * NV];
+    if (ctl->done) return;
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
