@@ -86,7 +86,7 @@ struct sqg_ctx {
     DBuf chiB, zeeB, center, dots, htemp;
     // all-node state of the last density step
     DBuf veff, chi_all, zee_all, lmin_all, lmax_all, iters_all, mu_all, W, Ci_all, rho_d, part;
-    DBuf costab, ynode, scal;
+    DBuf costab, ynode;
     // Veff derivatives: vectors, per-node sign / d rho/d lambda / weight,
     // n^3 input and output, per-step tangent records
     DBuf adj, adj_sgn, adj_dl, adj_wt, adj_in, adj_out, adj_rec, adj_slot;
@@ -96,6 +96,11 @@ struct sqg_ctx {
     DBuf lf_V, lf_Vt, lf_bJ, lf_bJt, lf_img, lf_R, lf_RV, lf_DV, lf_RU, lf_DU, lf_toff, lf_tsize, lf_Z, lf_part, lf_err;
     bool have_state = false;
     double lambda_f = 0.0;
+    // pinned host words: active nodes per Lanczos pass, the Fermi sum
+    int *h_act = nullptr;
+    double *h_sum = nullptr;
+    DBuf act;
+    hipEvent_t pass_ev[2] = {nullptr, nullptr};
     unsigned char *scratch_ptr = nullptr;   // this device's copy of `scratch` (sqg_hsub_apply_batch_noalloc)
     // device timing of the hot kernels over the last density call (which:
     // 0 Chebyshev z-march, 1 Lanczos z-march, 2 projections of the Lanczos
@@ -115,6 +120,10 @@ struct sqg_ctx {
     ~sqg_ctx()
     {
         for (auto e : pool) (void)hipEventDestroy(e);
+        for (auto e : pass_ev)
+            if (e) (void)hipEventDestroy(e);
+        if (h_act) (void)hipHostFree(h_act);
+        if (h_sum) (void)hipHostFree(h_sum);
         if (st) (void)hipStreamDestroy(st);
     }
     hipEvent_t ev_get()
@@ -708,33 +717,53 @@ int lanczos_batch(sqg_ctx *c, int B, long *passes_out)
     Q.ca = c->ca.as<double>(); Q.ib = c->ib.as<double>(); Q.bprev = c->bprev.as<double>();
     Q.chi = c->chiB.as<double>(); Q.zee = c->zeeB.as<double>();
     Q.err = flags + 1;
-    std::vector<int> hdone(B);
-    int active = B;
-    long passes = 0;
+    Q.act = c->act.as<int>();
+    hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(512), 0, c->st, c->act.as<int>(), (size_t)MAXIT + 2, 0);
+    // The host reads the count of active nodes one pass behind the launches, so
+    // that the GPU never waits for it (a wait per pass cost about 20 us, most
+    // of a small batch's pass); the pass launched beyond the last returns at
+    // once, every node being frozen.
+    std::vector<int> active{B};              // nodes active at the start of each pass
+    const size_t ev_p = c->ev[2].size(), ev_z = c->ev[1].size();
+    const bool timed_p = c->n_ip > 0;
+    auto settle = [&](int p) -> hipError_t {   // active nodes after pass p
+        if (p == 0) { active.push_back(B); return hipSuccess; }
+        const hipError_t e = hipEventSynchronize(c->pass_ev[p & 1]);
+        active.push_back(c->h_act[p]);
+        return e;
+    };
     T *X2 = c->X2.as<T>(), *Y2 = c->Y2.as<T>();
-    for (int pass = 0; pass <= MAXIT && active > 0; ++pass) {
+    for (int pass = 0; pass <= MAXIT && active.back() > 0; ++pass) {
         // (r', v_{k-1}) in one pair of buffers, (r'_{k+1}, v_k) out into the other
         T *Xi = (pass & 1) ? X2 : X, *Yi = (pass & 1) ? Y2 : Y;
         T *Xo = (pass & 1) ? X : X2, *Yo = (pass & 1) ? Y : Y2;
         PArgs<T> P = pargs<T>(c, dn, ddone, Xi);
         P.V2 = Yi;
-        launch_proj<T, 1>(c, B, P, 2, 2.0 * active * c->M3 * rs);   // reads r' and v_{k-1}
+        launch_proj<T, 1>(c, B, P, 2, 2.0 * c->M3 * rs);   // reads r' and v_{k-1}
         ZArgs<T> Z = zargs<T>(c, dn, ddone);
         Z.X = Xi; Z.Y = Yi; Z.XO = Xo; Z.YO = Yo;
         Z.ca = c->ca.as<double>(); Z.ib = c->ib.as<double>(); Z.bprev = c->bprev.as<double>();
         Z.lred = c->lred.as<double>();
         // reads r' and v_{k-1}, writes v_k and r'_{k+1}
-        launch_zmarch<T, MODE_LANCZOS>(c, B, Z, 1, 4.0 * active * c->M3 * rs);
-        passes += active;
+        launch_zmarch<T, MODE_LANCZOS>(c, B, Z, 1, 4.0 * c->M3 * rs);
         Q.pass = pass;
         hipLaunchKernelGGL(k_lanczos_scalars, dim3((B + LQN - 1) / LQN), dim3(2 * LQN), 0, c->st, Q);
         if (pass >= 1) {
-            HIPCHK(hipMemcpyAsync(hdone.data(), ddone, (size_t)B * sizeof(int), hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
-            active = 0;
-            for (int i = 0; i < B; ++i) active += hdone[i] == 0;
+            HIPCHK(hipMemcpyAsync(c->h_act + pass, c->act.as<int>() + pass, sizeof(int), hipMemcpyDeviceToHost, c->st));
+            HIPCHK(hipEventRecord(c->pass_ev[pass & 1], c->st));
         }
+        if (pass >= 1) HIPCHK(settle(pass - 1));
     }
+    // the algorithmic bytes of each pass count its active nodes; the launches of
+    // the pass beyond the last are not passes
+    long passes = 0;
+    auto settle_bytes = [&](std::vector<EventPair> &ev, size_t e0) {
+        while (ev.size() > e0 && active.size() > 1 && ev.size() - e0 >= active.size() && active.back() == 0) ev.pop_back();
+        for (size_t i = e0; i < ev.size(); ++i) ev[i].bytes *= active[std::min(i - e0, active.size() - 1)];
+    };
+    if (timed_p) settle_bytes(c->ev[2], ev_p);
+    settle_bytes(c->ev[1], ev_z);
+    for (int a : active) passes += a;
     if (passes_out) *passes_out += passes;
     if (ph0 && ph1) {
         (void)hipEventRecord(ph1, c->st);
@@ -920,9 +949,9 @@ int fermi_eval(sqg_ctx *c, double lf, int mode, double *out)
     hipLaunchKernelGGL(k_fermi_sum, dim3(nb), dim3(bs), 0, c->st, c->W.as<double>(), c->chi_all.as<double>(),
                        c->zee_all.as<double>(), c->ynode.as<double>(), nn, c->p.npl, lf, c->p.bet, mode,
                        c->part.as<double>());
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->st, c->part.as<double>(), nb, c->scal.as<double>());
-    HIPCHK(hipMemcpyAsync(out, c->scal.p, sizeof(double), hipMemcpyDeviceToHost, c->st));
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, c->st, c->part.as<double>(), nb, c->h_sum);
     HIPCHK(hipStreamSynchronize(c->st));
+    *out = *c->h_sum;
     return SQG_OK;
 }
 
@@ -1152,6 +1181,10 @@ int sqg_create(const sqg_params *p, sqg_ctx **out)
     c->p = *p;
     HIPCHK(hipSetDevice(p->device));
     HIPCHK(hipStreamCreate(&c->st));
+    for (auto &e : c->pass_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    HIPCHK(hipHostMalloc((void **)&c->h_act, (MAXIT + 2) * sizeof(int), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&c->h_sum, sizeof(double), hipHostMallocDefault));
+    HIPCHK(c->act.ensure((MAXIT + 2) * sizeof(int)));
     // this device's address of the allocation-free entry point's scratch array
     {
         void *sp = nullptr;
@@ -1180,7 +1213,6 @@ int sqg_create(const sqg_params *p, sqg_ctx **out)
         HIPCHK(c->costab.ensure((size_t)K * K * sizeof(double)));
         HIPCHK(hipMemcpy(c->ynode.p, y.data(), K * sizeof(double), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(c->costab.p, ct.data(), (size_t)K * K * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(c->scal.ensure(16 * sizeof(double)));
     }
     *out = c.release();
     return SQG_OK;

@@ -1765,6 +1765,7 @@ struct QArgs {
     double *ca, *ib, *bprev;  // next pass scalars
     double *chi, *zee;        // outputs at convergence
     int *err;
+    int *act;                 // [MAXIT + 2] nodes still active after each pass
 };
 
 __device__ int ql_extremes(double *d, double *e, int n, double *lmin, double *lmax)
@@ -1967,6 +1968,9 @@ __global__ void __launch_bounds__(2 * LQN) k_lanczos_scalars(QArgs A)
         A.chi[b] = (hi + lo) / 2;
         A.zee[b] = (hi - lo) / 2;
         A.done[b] = 1;
+    } else {
+        const unsigned long long on = __ballot(1);
+        if ((threadIdx.x & 63) == __ffsll((long long)on) - 1) atomicAdd(A.act + p, __popcll(on));
     }
 }
 
