@@ -165,6 +165,10 @@ template <> __device__ __forceinline__ double bload<double>(__amdgpu_buffer_rsrc
 {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
 }
+// The most values by which a member's cube may start after the corner of its
+// group's union: one plane, and rows and columns within (M + 3)^2 (the host's
+// rule for groups, whatever order their nodes come in).
+__device__ __forceinline__ int group_pad(int M) { return M * M + 6 * M + 24; }
 __device__ __forceinline__ int bload_i32(__amdgpu_buffer_rsrc_t r, unsigned off)
 {
     return (int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
@@ -1120,7 +1124,7 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
     // constant of the member, the scalar offset of the loads; the resources
     // start pad values early so that none is negative (the masks keep every
     // address inside the member's cube)
-    const int pad = M2 + M + 8;
+    const int pad = group_pad(M);
     const size_t gb = ((size_t)gn * M3 + pad) * TS;
     const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3 - pad, gb);
     const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3 - pad, gb);

@@ -42,3 +42,28 @@ def test_hsub_of_scattered_nodes(elem, prec, tol):
     for b, nd in enumerate(nodes):
         ref = o.hsub(veff, int(nd), v[b].reshape(-1))
         assert H.rel(hv[b].reshape(-1), ref) < tol
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("elem", ["al", "lih"])
+def test_hsub_of_pairs_in_any_order(elem, prec):
+    """Two nodes share a group up to one plane and several rows or columns
+    apart, and either may come first; next to them, pairs too far away to join.
+    Every product is the one that the node gives alone."""
+    print(elem, prec, flush=True)
+    S = (H.small_al if elem == "al" else H.small_lih)(n_cell=13)[0]
+    n, veff, nodes, at = 13, smooth_veff(S), [], 0
+    for dx, dy in [(0, 1), (0, 2), (1, 2), (0, 3), (0, 5), (0, 6), (3, 3), (6, 0), (-2, 2), (-3, 1)]:
+        for dz in (0, 1):
+            a = [3, 1, 5 * (at % 3)]
+            b = [3 + dx, 1 + dy, a[2] + dz]
+            at += 1
+            nodes += [(p[2] * n + p[1]) * n + p[0] for p in ([b, a] if at % 4 < 3 else [a, b])]
+    nodes = np.array(nodes)
+    sq = SpectralQuadrature(S, precision=prec)
+    rng = np.random.Generator(np.random.PCG64(8))
+    v = rng.standard_normal((nodes.size, sq.M, sq.M, sq.M))
+    hv = sq.HsubTimesVec(veff, nodes, v)
+    for b, nd in enumerate(nodes):
+        one = sq.HsubTimesVec(veff, nodes[b:b + 1], v[b:b + 1])
+        assert np.array_equal(hv[b].reshape(-1), one.reshape(-1)), (b, nd)
