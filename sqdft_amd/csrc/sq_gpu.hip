@@ -481,11 +481,13 @@ int node_images(sqg_ctx *c, const int *nodes, int B, bool node_lists = false)
     return image_lists(c, B, gst, node_lists);
 }
 
-// LDS bytes of one k_nlapplyg workgroup (loc table, row offsets, NG values per row)
+// LDS bytes of one k_nlapplyg workgroup (loc table, NG values per row, union
+// columns)
 size_t nlapplyg_lds(const sqg_ctx *c)
 {
-    const size_t head = ((size_t)(std::max(c->n_ip, 1) + c->gl_max + 1) * 4 + 15) / 16 * 16;
-    return head + (size_t)std::max(c->gl_max * c->max_nproj, 1) * SLW * sizeof(double);
+    const size_t head = ((size_t)std::max(c->n_ip, 1) * 4 + 15) / 16 * 16;
+    return head + (size_t)std::max(c->gl_max * c->max_nproj, 1) * SLW * sizeof(double) +
+           std::max((size_t)(c->M + 3) * (c->M + 3), (size_t)(c->M + 7) * c->M) * 4;
 }
 
 template <typename T, int K>
@@ -497,9 +499,14 @@ void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
         N.g = A.g; N.nl = A.nl; N.nlv = A.nlv;
         N.gst = c->gst.as<int>(); N.glist = c->glist.as<int>(); N.glist_cnt = c->glist_cnt.as<int>();
         N.img_type = c->img_type.as<int>(); N.nproj = c->nproj.as<int>(); N.ip_base = c->ip_base.as<int>();
+        N.mp = std::max(c->max_nproj, 1);
         auto fn = N.nl.ip16 ? k_nlapplyg<T, true> : k_nlapplyg<T, false>;
         if (shg > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shg);
-        hipLaunchKernelGGL(fn, dim3(c->ng), dim3(512), shg, c->st, N);
+        // three workgroups share a CU: about eight rounds of them, so that the
+        // last one costs little, with at least four points a thread each
+        const int pts = (c->M + 3) * (c->M + 1) * c->M;
+        const int split = std::max(1, std::min(6144 / std::max(c->ng, 1), pts / (4 * 512)));
+        hipLaunchKernelGGL(fn, dim3(c->ng, split), dim3(512), shg, c->st, N);
         return;
     }
     const size_t shm = (size_t)std::max(c->n_ip, 1) * sizeof(double);

@@ -165,6 +165,16 @@ template <> __device__ __forceinline__ double bload<double>(__amdgpu_buffer_rsrc
 {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
 }
+// Stores past the range are dropped.
+template <typename T> __device__ __forceinline__ void bstore(T v, __amdgpu_buffer_rsrc_t r, unsigned off, int soff)
+{
+    if constexpr (sizeof(T) == 8) {
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, soff, 0);
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, soff, 0);
+    }
+}
 // The most values by which a member's cube may start after the corner of its
 // group's union: one plane, and rows and columns within (M + 3)^2 (the host's
 // rule for groups, whatever order their nodes come in).
@@ -1353,8 +1363,21 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
 // each point of the union of the members' cubes reads its ELL entries once
 // and applies them to every member's projections, which sit in LDS
 // compacted to the images of the group list (loc maps an image-projector id
-// to its row, sl holds NG values per row).  Each member's sum runs over the
-// point's entries in slot order, as in k_nlapply.
+// to its row, sl holds NG values per row, mp rows an image).  Each member's sum
+// runs over the point's entries in slot order, as in k_nlapply.
+//
+// Bound by its stores (8 M^3 values a group; the tables stay in the caches) and
+// by the chain count -> entries -> loc -> row -> store of a point, hidden by
+// waves alone: two entries at a time keep it at 69 VGPRs and three workgroups
+// a CU (four at a time: 892 against 867 us; the next point's entries fetched
+// early as well: 128 VGPRs, spills, 1147 us).  Where a point sits and which
+// members hold it comes from a table of the union's columns, its place in a
+// member's cube is a scalar offset.  Several workgroups share a group, each with
+// a run of planes (shares that alternate point by point split cache lines:
+// 879 us).  Before these changes against now, us a pass: 8,192 nodes with FP64
+// 35^3 cubes 888 and 732 (2.8 GB: 3.8 TB/s), 4,096 with FP32 ones 285 and 213,
+// 1,000 with FP64 17^3 cubes 34 and 24; 4,096 with 31^3 LiH ones (eight entries
+// a point: LDS rows) 386 and 387.
 template <typename T>
 struct NGArgs {
     Geo g;
@@ -1363,6 +1386,7 @@ struct NGArgs {
     const int *gst;               // [groups + 1] first slot of each group
     const int *glist, *glist_cnt;
     const int *img_type, *nproj, *ip_base;
+    int mp;                       // projectors of an image at most: rows per image
 };
 
 template <typename T, bool IP16>
@@ -1374,46 +1398,52 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     const int b0 = A.gst[q], gn = A.gst[q + 1] - b0;
     const int n = G.n, M = G.M, M2 = G.M2, M3 = G.M3, E = G.E;
     int ni[NG], nj[NG], nk[NG];
-    bool on[NG];
-    int nact = 0;
+    unsigned onmask = 0;
     int ex0 = 1 << 30, ex1 = -1, ey0 = 1 << 30, ey1 = -1, ez0 = 1 << 30, ez1 = -1;
 #pragma unroll
     for (int m = 0; m < NG; ++m) {
-        on[m] = m < gn && !(G.done && G.done[b0 + m]);
         const int node = G.node_list[b0 + min(m, gn - 1)];
         ni[m] = node % n; nj[m] = (node / n) % n; nk[m] = node / (n * n);
-        if (on[m]) {
-            ++nact;
+        if (m < gn && !(G.done && G.done[b0 + m])) {
+            onmask |= 1u << m;
             ex0 = min(ex0, ni[m]); ex1 = max(ex1, ni[m] + M - 1);
             ey0 = min(ey0, nj[m]); ey1 = max(ey1, nj[m] + M - 1);
             ez0 = min(ez0, nk[m]); ez1 = max(ez1, nk[m] + M - 1);
         }
     }
-    if (nact == 0) return;
-    // LDS: loc [n_ip] | row offsets [cnt + 1] | sl [rows][SLW]
+    if (onmask == 0) return;
+    // LDS: loc [n_ip] | sl [cnt mp][SLW] | union columns
     extern __shared__ unsigned char smem_raw[];
     int *loc = reinterpret_cast<int *>(smem_raw);
     const int cnt = A.glist_cnt[q];
-    int *roff = loc + A.nl.n_ip;
-    double *sl = reinterpret_cast<double *>(smem_raw + (((size_t)A.nl.n_ip + cnt + 1) * 4 + 15) / 16 * 16);
+    double *sl = reinterpret_cast<double *>(smem_raw + ((size_t)A.nl.n_ip * 4 + 15) / 16 * 16);
+    unsigned *xyt = reinterpret_cast<unsigned *>(sl + (size_t)max(cnt * A.mp, 1) * SLW);
     const int *gl = A.glist + (size_t)q * GLCAP;
     for (int i = threadIdx.x; i < A.nl.n_ip; i += blockDim.x) loc[i] = 0;
-    if (threadIdx.x == 0) {
-        int r = 0;
-        for (int l = 0; l < cnt; ++l) { roff[l] = r; r += A.nproj[A.img_type[gl[l]]]; }
-        roff[cnt] = r;
-    }
     __syncthreads();
     for (int l = threadIdx.x; l < cnt; l += blockDim.x) {
-        const int J = gl[l], r0 = roff[l], np = roff[l + 1] - r0, ipb = A.ip_base[J];
+        const int J = gl[l], r0 = l * A.mp, np = A.nproj[A.img_type[J]], ipb = A.ip_base[J];
         for (int i = 0; i < np; ++i) {
             loc[ipb + i] = r0 + i;
 #pragma unroll
             for (int m = 0; m < NG; ++m)
-                sl[(size_t)(r0 + i) * SLW + m] = on[m] ? A.nl.s[(size_t)(b0 + m) * A.nl.n_ip + ipb + i] : 0.0;
+                sl[(size_t)(r0 + i) * SLW + m] =
+                    ((onmask >> m) & 1u) ? A.nl.s[(size_t)(b0 + m) * A.nl.n_ip + ipb + i] : 0.0;
         }
     }
     if (cnt == 0 && threadIdx.x < SLW) sl[threadIdx.x] = 0.0;
+    // union column -> x, y (12 bits each) and the members whose cube holds it
+    const int ux = ex1 - ex0 + 1, uy = ey1 - ey0 + 1, uz = ez1 - ez0 + 1, np_ = ux * uy;
+    for (int p = threadIdx.x; p < np_; p += blockDim.x) {
+        const int yy = p / ux, xx = p - yy * ux;
+        unsigned v = (unsigned)xx | (unsigned)yy << 12;
+#pragma unroll
+        for (int m = 0; m < NG; ++m)
+            if (((onmask >> m) & 1u) && (unsigned)(ex0 + xx - ni[m]) < (unsigned)M &&
+                (unsigned)(ey0 + yy - nj[m]) < (unsigned)M)
+                v |= 1u << (24 + m);
+        xyt[p] = v;
+    }
     __syncthreads();
     const int E3 = (int)A.nl.E3;
     const int KA = A.nl.k_alloc;
@@ -1422,50 +1452,72 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     const __amdgpu_buffer_rsrc_t rEI =
         brsrc(IP16 ? (const void *)A.nl.ip16 : (const void *)A.nl.ip, (size_t)KA * E3 * IS);
     const __amdgpu_buffer_rsrc_t rEC = brsrc(A.nl.cnt, (size_t)E3);
-    T *out = A.nlv + (size_t)b0 * M3;
-    // one extended-grid point: sum its entries against every member's
-    // projections, four slots at a time up to the wave's largest count (a
-    // slot past the point's count loads u = 0 and adds exact zeros)
-    constexpr int CH = 4;
-    auto point = [&](int gx, int gy, int gz, double a[NG]) {
-        const int g = (gz * E + gy) * E + gx;
-        const int cn = bload_u8(rEC, (unsigned)g);
+    // a member's offset of a union point is the union's plus a constant, the
+    // scalar offset of the stores (pad keeps it from being negative)
+    const int pad = group_pad(M);
+    const __amdgpu_buffer_rsrc_t rO = brsrc(A.nlv + (size_t)b0 * M3 - pad, ((size_t)gn * M3 + pad) * TS);
+    // One union point at a time: its entries against every member's
+    // projections, CH slots at a time up to the wave's largest count (a slot
+    // past the point's count holds u = 0 and adds exact zeros), the first ones
+    // loaded together with the count.  This workgroup's share of the points: a
+    // run of planes of the union.
+    constexpr int CH = 2;
+    const int za = (int)((long)uz * blockIdx.y / gridDim.y), zb = (int)((long)uz * (blockIdx.y + 1) / gridDim.y);
+    const int sz = (int)blockDim.x / np_, sp = (int)blockDim.x - sz * np_;
+    struct Pt { int z, p; unsigned cv; int g, cn; T u[CH]; int ip[CH]; };
+    auto entries = [&](int g, int j0, bool on, T (&u)[CH], int (&ip)[CH]) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const bool ok = on && j0 + c < KA;
+            const unsigned e = (unsigned)((j0 + c) * E3 + g);
+            u[c] = bload<T>(rEU, ok ? e * TS : OOB);
+            ip[c] = IP16 ? bload_u16(rEI, ok ? e * IS : OOB) : bload_i32(rEI, ok ? e * IS : OOB);
+        }
+    };
+    auto load = [&](Pt &P) {
+        const bool on = P.z < zb;
+        P.cv = on ? xyt[P.p] : 0u;
+        P.g = ((ez0 + P.z) * E + ey0 + (int)((P.cv >> 12) & 4095)) * E + ex0 + (int)(P.cv & 4095);
+        P.cn = bload_u8(rEC, on ? (unsigned)P.g : OOB);
+        entries(P.g, 0, on, P.u, P.ip);
+    };
+    auto sum = [&](Pt &P) {
+        double a[NG];
 #pragma unroll
         for (int m = 0; m < NG; ++m) a[m] = 0.0;
 #pragma unroll 1
-        for (int j0 = 0; j0 < KA && __ballot(cn > j0) != 0; j0 += CH) {
-            T u[CH];
-            int ip[CH];
+        for (int j0 = 0;;) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
-                const int j = j0 + c;
-                const bool ok = j < cn;
-                u[c] = bload<T>(rEU, ok ? (unsigned)(j * E3 + g) * TS : OOB);
-                ip[c] = IP16 ? bload_u16(rEI, ok ? (unsigned)(j * E3 + g) * IS : OOB)
-                             : bload_i32(rEI, ok ? (unsigned)(j * E3 + g) * IS : OOB);
-            }
+                const double *row = sl + (size_t)loc[P.ip[c]] * SLW;
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const double *row = sl + (size_t)loc[ip[c]] * SLW;
-#pragma unroll
-                for (int m = 0; m < NG; ++m) a[m] += row[m] * (double)u[c];
+                for (int m = 0; m < NG; ++m) a[m] += row[m] * (double)P.u[c];
+                if (c & 1) __builtin_amdgcn_sched_barrier(0);   // two rows in flight (registers)
             }
+            j0 += CH;
+            if (j0 >= KA || __ballot(P.cn > j0) == 0) break;
+            entries(P.g, j0, P.cn > j0, P.u, P.ip);
         }
-    };
-    const int ux = ex1 - ex0 + 1, uy = ey1 - ey0 + 1, uz = ez1 - ez0 + 1;
-    const int uxy = ux * uy, tot = uxy * uz;
-#pragma unroll 1
-    for (int p = threadIdx.x; p < tot; p += blockDim.x) {
-        const int z = p / uxy, r = p - z * uxy, y = r / ux, x = r - y * ux;
-        const int gx = ex0 + x, gy = ey0 + y, gz = ez0 + z;
-        double a[NG];
-        point(gx, gy, gz, a);
+        const int gz = ez0 + P.z;
+        const unsigned co = (unsigned)((P.z * M2 + (int)((P.cv >> 12) & 4095) * M + (int)(P.cv & 4095)) * (int)TS);
 #pragma unroll
         for (int m = 0; m < NG; ++m) {
-            const unsigned lx = gx - ni[m], ly = gy - nj[m], lz = gz - nk[m];
-            if (on[m] && lx < (unsigned)M && ly < (unsigned)M && lz < (unsigned)M)
-                out[(size_t)m * M3 + (lz * M2 + ly * M + lx)] = (T)a[m];
+            const int kof = (pad + m * M3 + (ez0 - nk[m]) * M2 + (ey0 - nj[m]) * M + ex0 - ni[m]) * (int)TS;
+            const bool ok = (P.cv & (1u << (24 + m))) && (unsigned)(gz - nk[m]) < (unsigned)M;
+            bstore<T>((T)a[m], rO, ok ? co : OOB, kof);
         }
+    };
+    Pt P;
+    P.z = (int)threadIdx.x / np_;
+    P.p = (int)threadIdx.x - P.z * np_;
+    P.z += za;
+#pragma unroll 1
+    while (P.z < zb) {
+        load(P);
+        sum(P);
+        P.z += sz;
+        P.p += sp;
+        if (P.p >= np_) { P.p -= np_; ++P.z; }
     }
 }
 
