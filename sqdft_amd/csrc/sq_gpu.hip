@@ -554,13 +554,32 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
     return false;
 }
 
+// Workgroups that share the images of a group in k_projw.  A workgroup fills a
+// CU, so ng groups take ceil(ng / 256) rounds.  Half of a group's images,
+// consecutive in z, take 0.6 of a whole walk (they reach about three quarters of
+// its planes), a quarter 0.52: shares pay where they fill CUs that would idle.
+// us a pass with 1, 2 and 4 workgroups: a few nodes 63, 45, 36; 64 groups of
+// 17^3 cubes 25, 21, 19; about 150 of them 74, 88, 96; 364 of 25^3 LiH cubes 418,
+// 384, 466; 480 of them 385, 453, 565.
+int projw_split(int ng)
+{
+    int best = 1;
+    double t = 1e30;
+    const double cost[3] = {1.0, 0.6, 0.52};
+    for (int i = 0; i < 3; ++i) {
+        const double ti = (((long)ng << i) + 255) / 256 * cost[i];
+        if (ti < t) { t = ti; best = 1 << i; }
+    }
+    return best;
+}
+
 template <typename T, int FORMED, bool MFMA, int I>
 void projw_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 {
     constexpr ProjShape S = MFMA ? PROJM_SHAPES[MFMA ? I : 0] : PROJR_SHAPES[I];
     auto fn = k_projw<T, FORMED, S.nw * 64, S.R, PROJW_RPI, MFMA, MFMA ? 0 : sizeof(T) == 4 ? 2 : 1>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(S.nw * 64), shm, c->st, P);
+    hipLaunchKernelGGL(fn, dim3(c->ng, projw_split(c->ng)), dim3(S.nw * 64), shm, c->st, P);
 }
 
 template <typename T, int FORMED>

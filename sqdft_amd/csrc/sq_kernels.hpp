@@ -1065,6 +1065,8 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 // vectors' HBM reads and, since one workgroup fills a CU's LDS, by what its
 // waves overlap; which members hold a union column and where it sits is worked
 // out once per walk (xyt), not per plane and member.
+// gridDim.y workgroups share a group's images (each image is one workgroup's, so
+// the sums are the same): the slots a share needs are those of the whole list.
 // SZC: planes per slab, 0: A.sz (a loop of unknown length over a slot's planes
 // costs the VALU shapes the registers of their slots).
 template <typename T, int FORMED, int NT, int R, int RPI, bool MFMA, int SZC>
@@ -1101,7 +1103,9 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
             uz0 = min(uz0, nk[m] - nloc); uz1 = max(uz1, nk[m] + nloc);
         }
     }
-    const int cnt = A.glist_cnt[q];
+    // this workgroup's share of the group's images, consecutive in z
+    const int gcnt = A.glist_cnt[q];
+    const int l0 = (int)(gcnt * blockIdx.y / gridDim.y), cnt = (int)(gcnt * (blockIdx.y + 1) / gridDim.y) - l0;
     if (onmask == 0 || cnt == 0) return;
     const int ux = ux1 - ux0 + 1, uy = uy1 - uy0 + 1, np_ = ux * uy;
     // LDS: image data [cnt] | union columns [np_] | staged slab [SZ][NM][ms]
@@ -1110,7 +1114,7 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
     unsigned *xyt = reinterpret_cast<unsigned *>(smem_raw + ((size_t)cnt * sizeof(ImgMeta) + 15) / 16 * 16);
     T *pl = reinterpret_cast<T *>(reinterpret_cast<unsigned char *>(xyt) + ((size_t)np_ * 4 + 15) / 16 * 16);
     for (int li = tid; li < cnt; li += NT) {
-        const int J = A.glist[(size_t)q * GLCAP + li];
+        const int J = A.glist[(size_t)q * GLCAP + l0 + li];
         const int t = A.img_type[J], nc = A.nlocc[t];
         ImgMeta e;
         e.ox = A.img_nn[3 * J] - nc; e.oy = A.img_nn[3 * J + 1] - nc; e.oz = A.img_nn[3 * J + 2] - nc;
@@ -1153,7 +1157,11 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
     const int mw = MFMA ? 4 * ((lane >> 2) & 1) + (lane >> 4) : lane >> (6 - LV), jw = lane & 3;
     const bool writer = (MFMA ? (lane & 8) == 0 : (lane & ((64 >> LV) - 1)) == 0) && ((onmask >> mw) & 1u);
     double *sw = A.s + (size_t)(b0 + mw) * A.n_ip;
-    const int zs0 = (uz0 + 4096) / SZ * SZ - 4096;
+    // planes of the union that these images reach (at least one: images that
+    // miss the union are zeroed on the way)
+    const int za0 = min(max(uz0, __builtin_amdgcn_readfirstlane(im[0].oz)), uz1);
+    const int ze0 = max(za0, min(uz1, __builtin_amdgcn_readfirstlane(im[cnt - 1].oz) + wbox - 1));
+    const int zs0 = (za0 + 4096) / SZ * SZ - 4096;
     // per-wave slot state: images started (slotted or not), slotted images,
     // live-slot mask, per-slot image data
     int nstart = 0, nslot = 0;
@@ -1174,7 +1182,7 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
         for (int m = 0; m < (MFMA ? 2 : NM); ++m) acc[r][m] = 0.0;
     }
 #pragma unroll 1
-    for (int gzs = zs0; gzs <= uz1; gzs += SZ) {
+    for (int gzs = zs0; gzs <= ze0; gzs += SZ) {
         // the previous slab is consumed before it is overwritten
         __syncthreads();
 #pragma unroll 1

@@ -67,3 +67,24 @@ def test_hsub_of_pairs_in_any_order(elem, prec):
     for b, nd in enumerate(nodes):
         one = sq.HsubTimesVec(veff, nodes[b:b + 1], v[b:b + 1])
         assert np.array_equal(hv[b].reshape(-1), one.reshape(-1)), (b, nd)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("elem,n", [("al", 9), ("lih", 9)])
+def test_shares_of_a_group_sum_alike(elem, n, prec):
+    """The images of a group go to one, two or four workgroups by the number of
+    groups in the call: the same nodes give the same bits in calls of 9 (four
+    shares), 100 (two), 150 and 300 isolated nodes (one, two) and repeated."""
+    print(elem, n, prec, flush=True)
+    S = (H.small_al if elem == "al" else H.small_lih)(n_cell=n)[0]
+    veff = smooth_veff(S)
+    sq = SpectralQuadrature(S, precision=prec)
+    rng = np.random.Generator(np.random.PCG64(21))
+    # alternately from the lowest and the highest planes: groups of one node each
+    lo, hi = rng.integers(0, n * n, 150), S.nn - 1 - rng.integers(0, n * n, 150)
+    nodes = np.stack([lo, hi], axis=1).reshape(-1)
+    v = rng.standard_normal((nodes.size, sq.M, sq.M, sq.M))
+    whole = sq.HsubTimesVec(veff, nodes, v).reshape(nodes.size, -1)
+    for cnt in (9, 100, 150):
+        part = sq.HsubTimesVec(veff, nodes[:cnt], v[:cnt]).reshape(cnt, -1)
+        assert np.array_equal(part, whole[:cnt]), cnt
