@@ -12,8 +12,8 @@
 // through the cube along z, keeping a 13-plane register window per column
 // (z-neighbours), staging the current plane in LDS (x/y-neighbours, with six
 // halo rows beyond its half) and streaming each output plane to HBM as soon
-// as it is complete.  The projections of 8 consecutive cubes (a 4x2 half
-// brick) are formed by one workgroup from their union, slab by slab.
+// as it is complete.  The projections of up to 8 neighbouring cubes (a 4x2 half
+// brick where the grid allows) are formed from their union, slab by slab.
 #pragma once
 
 #include <hip/hip_runtime.h>
