@@ -117,6 +117,13 @@ struct sqg_ctx {
     // SQG_MIXED_LANCZOS: FP32 Lanczos passes, everything else in FP64 (the
     // operator data are kept in both types)
     bool split() const { return p.precision == SQG_MIXED_LANCZOS; }
+    ProjDims dims() const
+    {
+        int w = 0;
+        for (int t = 0; t < n_typ; ++t)
+            if (h_nproj[t] > 0) w = std::max(w, 2 * h_nlocc[t] + 1);
+        return {M, max_nproj, n_ip, w};
+    }
     ~sqg_ctx()
     {
         for (auto e : pool) (void)hipEventDestroy(e);
@@ -307,117 +314,20 @@ PArgs<T> pargs(sqg_ctx *c, const int *dn, const int *dd, const T *V)
     return A;
 }
 
-// Compiled shapes of k_projw, the first that holds every group of the batch is
-// taken: waves per workgroup and register slots per wave.  One workgroup fills
-// a CU's LDS, so its waves are all that hides the loads: twelve, if the slots
-// that their 168 VGPRs hold are enough (the Al and LiH cells), else eight with
-// more slots.  Twelve against eight, us a pass: 8,192 nodes with FP64 35^3
-// cubes 1265 against 1549 (Lanczos) and 895 against 1175 (Chebyshev), 4,096
-// with FP32 ones 468 and 402 against 542 and 488; MFMA, 4,096 nodes with 31^3
-// cubes, 875 and 862 against 1142 and 1166.  With the union columns worked out
-// once per walk the twelve-wave ones take 1192, 863, 459, 358, 838 and 760.
-constexpr int PROJW_RPI = 3;
-struct ProjShape { int nw, R; };
-constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
-constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // MFMA: two doubles per slot and lane
-
-// How k_projw runs on vectors of ts bytes per value: on = 0 when it does not
-// apply; the matrix cores for FP64 tables of several projectors.
-struct ProjwUse { int on, mfma, w; };
-ProjwUse projw_use(const sqg_ctx *c, size_t ts)
+// Bytes per value of the vectors of the phases that run on one batch: both
+// types in SQG_MIXED_LANCZOS.
+int stored_types(const sqg_ctx *c, size_t (&ts)[2])
 {
-    if (c->max_nproj < 1 || c->max_nproj > 4 || c->n_ip == 0) return {0, 0, 0};
-    // p channels in FP64: the matrix cores.  FP32 tables (mixed precision)
-    // stay with k_projs: its VALU sums of FP32 operands ran at 1.18 ms a pass
-    // on the 216-atom LiH batches against 1.67 ms (FP64 MFMAs fed by
-    // conversions), while in FP64 the two tied (2.3 ms).
-    if (c->max_nproj > 1 && ts == 4) return {0, 0, 0};
-    const int mfma = c->max_nproj > 1;
-    int w = 0;
-    for (int t = 0; t < c->n_typ; ++t)
-        if (c->h_nproj[t] > 0) w = std::max(w, 2 * c->h_nlocc[t] + 1);
-    if (mfma ? w > 16 : w * w > 64 * PROJW_RPI) return {0, 0, 0};
-    return {1, mfma, w};
+    ts[0] = c->split() ? 4 : c->real_size();
+    ts[1] = 8;
+    return c->split() ? 2 : 1;
 }
 
-// LDS values per plane and member of a staged block of ux x uy columns: rows
-// padded to a pitch congruent to the box side modulo 32, the MFMA member
-// stride to 8 (as k_projw pads them).
-int projw_slab(const ProjwUse &pw, int ux, int uy)
+std::vector<int> groups_of(const sqg_ctx *c, const int *nodes, int B)
 {
-    const int u = (ux + (((pw.w - ux) % 32) + 32) % 32) * uy;
-    return pw.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
-}
-
-// Slab capacity per plane and member: the union plane of a 4x2 block of cubes
-// or one cube.
-int projw_pu(const sqg_ctx *c, const ProjwUse &pw)
-{
-    return std::max(projw_slab(pw, c->M + 3, c->M + 1), projw_slab(pw, c->M, c->M));
-}
-
-// LDS bytes of k_projw beside the slab: image data and union columns.
-size_t projw_head(const sqg_ctx *c, int gl_max)
-{
-    return ((size_t)std::max(gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16 +
-           (std::max((size_t)(c->M + 3) * (c->M + 3), (size_t)(c->M + 7) * c->M) * 4 + 15) / 16 * 16;
-}
-
-// Planes per slab.  VALU: one FP64 or two FP32 planes (a deeper slab keeps more
-// images alive than the slots of twelve waves: 17^3 cubes with three planes
-// took 269 us a pass with ten slots in eight waves against 81).  MFMA, whose
-// slots are small: about four load rounds of a workgroup between two barriers,
-// at most eight planes, as far as the LDS holds them beside a list of 256
-// images (25^3 cubes, two planes: 373 against 496 us a pass).
-int projw_sz(const sqg_ctx *c, const ProjwUse &pw, size_t ts)
-{
-    const size_t plane = (size_t)projw_pu(c, pw) * NG * ts, head = projw_head(c, 256);
-    const int lds = plane + head <= 160 * 1024 ? (int)((160 * 1024 - head) / plane) : 1;
-    if (!pw.mfma) return ts == 4 ? 2 : 1;
-    return std::max(1, std::min({8, lds, 3072 / ((c->M + 3) * (c->M + 1))}));
-}
-
-// k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
-int projs_pu(const sqg_ctx *c) { return (c->M + 3) * (c->M + 3); }
-
-// Cuts B slots into groups of up to NG consecutive ones whose cubes the
-// staged projection kernels can walk together: the union plane fits the slab
-// capacity of every kernel that may run on the batch, and the cubes are at
-// most one plane apart in z.  A run ends where the next node is too far away
-// (a brick's edge, a gap in the caller's list): walking such members one
-// after the other in one workgroup, as unions that do not fit would need, is
-// several times slower: with runs of 8 slots cut anywhere, a density step on a
-// 15^3 LiH grid (25^3 cubes) took 534 ms and on a 10^3 Al grid (17^3) 44.6 ms,
-// against 155 and 15.2 ms.
-std::vector<int> make_groups(const sqg_ctx *c, const int *nodes, int B)
-{
-    const int n = c->p.n, M = c->M;
-    const ProjwUse use[2] = {projw_use(c, c->split() ? 4 : c->real_size()), projw_use(c, 8)};
-    const int nsh = c->split() ? 2 : 1;
-    auto fits = [&](int dx, int dy, int dz) {
-        if (dz > 1 || (M + dx) * (M + dy) > projs_pu(c)) return false;
-        for (int i = 0; i < nsh; ++i)
-            if (use[i].on && projw_slab(use[i], M + dx, M + dy) > projw_pu(c, use[i])) return false;
-        return true;
-    };
-    std::vector<int> gst{0};
-    int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-    for (int b = 0; b < B; ++b) {
-        const int r[3] = {nodes[b] % n, (nodes[b] / n) % n, nodes[b] / (n * n)};
-        const int cnt = b - gst.back();
-        int l[3], h[3];
-        for (int d = 0; d < 3; ++d) {
-            l[d] = cnt ? std::min(lo[d], r[d]) : r[d];
-            h[d] = cnt ? std::max(hi[d], r[d]) : r[d];
-        }
-        if (cnt && (cnt == NG || !fits(h[0] - l[0], h[1] - l[1], h[2] - l[2]))) {
-            gst.push_back(b);
-            for (int d = 0; d < 3; ++d) l[d] = h[d] = r[d];
-        }
-        for (int d = 0; d < 3; ++d) { lo[d] = l[d]; hi[d] = h[d]; }
-    }
-    gst.push_back(B);
-    return gst;
+    size_t ts[2];
+    const int nts = stored_types(c, ts);
+    return make_groups(c->dims(), c->p.n, ts, nts, nodes, B);
 }
 
 // Image lists of the B nodes in node_list on the groups gst, and per node where
@@ -441,17 +351,18 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     L.gst = c->gst.as<int>();
     L.glist = c->glist.as<int>();
     L.glist_cnt = c->glist_cnt.as<int>();
-    // the projection shapes of the phases that will run on these lists (both
-    // stored types in SQG_MIXED_LANCZOS): each plans its register slots
-    const size_t ts[2] = {c->split() ? 4 : c->real_size(), 8};
-    const int nsh = c->split() ? 2 : 1;
+    // the projection shapes of the phases that will run on these lists: each
+    // plans its register slots
+    const ProjDims dm = c->dims();
+    size_t ts[2];
+    const int nsh = stored_types(c, ts);
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)2, 0);
     bool any_on = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
-        const ProjwUse pw = projw_use(c, ts[i]);
+        const ProjwUse pw = projw_use(dm, ts[i]);
         if (!pw.on) continue;
         L.pr_need = c->flags.as<int>() + 4;
-        L.pr_sz[L.pr_n++] = projw_sz(c, pw, ts[i]);
+        L.pr_sz[L.pr_n++] = projw_sz(c->M, pw, ts[i]);
         any_on = true;
         any_mfma |= pw.mfma != 0;
     }
@@ -474,26 +385,17 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
 // Groups and image lists of the B nodes in node_list (nodes: their host copy).
 int node_images(sqg_ctx *c, const int *nodes, int B, bool node_lists = false)
 {
-    const std::vector<int> gst = make_groups(c, nodes, B);
+    const std::vector<int> gst = groups_of(c, nodes, B);
     HIPCHK(c->gst.ensure(gst.size() * sizeof(int)));
     HIPCHK(c->glist.ensure((gst.size() - 1) * GLCAP * sizeof(int)));
     HIPCHK(c->glist_cnt.ensure((gst.size() - 1) * sizeof(int)));
     return image_lists(c, B, gst, node_lists);
 }
 
-// LDS bytes of one k_nlapplyg workgroup (loc table, NG values per row, union
-// columns)
-size_t nlapplyg_lds(const sqg_ctx *c)
-{
-    const size_t head = ((size_t)std::max(c->n_ip, 1) * 4 + 15) / 16 * 16;
-    return head + (size_t)std::max(c->gl_max * c->max_nproj, 1) * SLW * sizeof(double) +
-           std::max((size_t)(c->M + 3) * (c->M + 3), (size_t)(c->M + 7) * c->M) * 4;
-}
-
 template <typename T, int K>
 void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
 {
-    const size_t shg = nlapplyg_lds(c);
+    const size_t shg = nlapplyg_lds(c->dims(), c->gl_max);
     if (shg <= 160 * 1024) {
         NGArgs<T> N{};
         N.g = A.g; N.nl = A.nl; N.nlv = A.nlv;
@@ -539,10 +441,10 @@ template <typename T, int FORMED>
 bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
 {
     constexpr int D = sizeof(T) == 4 ? 4 : 2;   // deep slab (planes)
-    const size_t sa = ((size_t)std::max(c->gl_max, 1) * sizeof(ImgMeta) + 15) / 16 * 16;
+    const size_t sa = images_lds(c->gl_max);
     // projector values are loaded and summed for npu of the mp slots
     const int npu = mp == 1 ? 1 : c->max_nproj == 3 ? 3 : 4;
-    P.pu = projs_pu(c);
+    P.pu = projs_pu(c->M);
     for (int sz : {D, D / 2, 1}) {
         const size_t shs = sa + (size_t)P.pu * NG * sizeof(T) * sz;
         if (shs > 160 * 1024) continue;
@@ -552,25 +454,6 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
         return true;
     }
     return false;
-}
-
-// Workgroups that share the images of a group in k_projw.  A workgroup fills a
-// CU, so ng groups take ceil(ng / 256) rounds.  Half of a group's images,
-// consecutive in z, take 0.6 of a whole walk (they reach about three quarters of
-// its planes), a quarter 0.52: shares pay where they fill CUs that would idle.
-// us a pass with 1, 2 and 4 workgroups: a few nodes 63, 45, 36; 64 groups of
-// 17^3 cubes 25, 21, 19; about 150 of them 74, 88, 96; 364 of 25^3 LiH cubes 418,
-// 384, 466; 480 of them 385, 453, 565.
-int projw_split(int ng)
-{
-    int best = 1;
-    double t = 1e30;
-    const double cost[3] = {1.0, 0.6, 0.52};
-    for (int i = 0; i < 3; ++i) {
-        const double ti = (((long)ng << i) + 255) / 256 * cost[i];
-        if (ti < t) { t = ti; best = 1 << i; }
-    }
-    return best;
 }
 
 template <typename T, int FORMED, bool MFMA, int I>
@@ -585,10 +468,10 @@ void projw_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
 template <typename T, int FORMED>
 bool launch_projw(sqg_ctx *c, PArgs<T> &P)
 {
-    const ProjwUse pw = projw_use(c, sizeof(T));
+    const ProjwUse pw = projw_use(c->dims(), sizeof(T));
     if (!pw.on) return false;
-    P.sz = projw_sz(c, pw, sizeof(T));
-    const size_t shm = projw_head(c, c->gl_max) + (size_t)projw_pu(c, pw) * NG * sizeof(T) * P.sz;
+    P.sz = projw_sz(c->M, pw, sizeof(T));
+    const size_t shm = projw_head(c->M, c->gl_max) + (size_t)projw_pu(c->M, pw) * NG * sizeof(T) * P.sz;
     if (shm > 160 * 1024) return false;
     if constexpr (sizeof(T) == 8) {
         if (pw.mfma) {
@@ -1602,7 +1485,7 @@ size_t noalloc_bytes(const sqg_ctx *c, int nb, size_t ng)
 // need more list space than full groups do: such a batch runs as two halves.
 static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int nb, const double *d_v, double *d_hv)
 {
-    const std::vector<int> gst = make_groups(c, nodes, nb);
+    const std::vector<int> gst = groups_of(c, nodes, nb);
     const size_t len = (size_t)nb * c->M3, rs = c->real_size(), ng = gst.size() - 1;
     if (noalloc_bytes(c, nb, ng) + (gst.size() * sizeof(int) + 255) / 256 * 256 > (size_t)SQG_NOALLOC_SCRATCH_BYTES) {
         if (nb == 1) return SQG_E_OVERFLOW;

@@ -16,6 +16,8 @@
 // brick where the grid allows) are formed from their union, slab by slab.
 #pragma once
 
+#include "sq_plan.hpp"
+
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -23,11 +25,6 @@ namespace sqk {
 
 constexpr int FDN = 6;          // half FD order (12th-order stencil)
 constexpr int WIN = 2 * FDN + 1;
-constexpr int LCAP = 512;       // max images meeting one node cube
-constexpr int NG = 8;           // node cubes per workgroup of the grouped projector kernels
-constexpr int SLW = 10;         // LDS row of k_nlapplyg: NG projections padded to 80 B (rows
-                                // r and r + 4 would share banks at 64 B)
-constexpr int GLCAP = 1024;     // max images meeting the cubes of one group
 constexpr int MAXM = 43;        // largest cube side one workgroup marches ((M+1)/2*M <= 1024)
 constexpr int MAXIT = 500;      // Lanczos max_iter (sq.cpp:967)
 
@@ -175,10 +172,6 @@ template <typename T> __device__ __forceinline__ void bstore(T v, __amdgpu_buffe
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off, soff, 0);
     }
 }
-// The most values by which a member's cube may start after the corner of its
-// group's union: one plane, and rows and columns within (M + 3)^2 (the host's
-// rule for groups, whatever order their nodes come in).
-__device__ __forceinline__ int group_pad(int M) { return M * M + 6 * M + 24; }
 __device__ __forceinline__ int bload_i32(__amdgpu_buffer_rsrc_t r, unsigned off)
 {
     return (int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
@@ -812,13 +805,6 @@ __device__ __forceinline__ double wave_sums(double (&v)[NV], int lane)
 // whose xy index in the image box is l mod 64; the plane's partial sums are
 // combined by wave_sums and added plane after plane, so a member's totals
 // depend only on its own cube.
-
-// Image data that k_projs reads per image and plane, cached in LDS per group
-struct ImgMeta {
-    int ox, oy, oz;               // rc-box origin (unwrapped grid coordinates)
-    int w, np, t, ipb;            // box side, projectors, type, first image-projector id
-    long uoff;                    // offset of the image's U block in udv
-};
 
 // First index of the z-sorted group list whose image centre z exceeds zc - 1
 // (centre z = oz + (w - 1) / 2).
@@ -1655,7 +1641,6 @@ struct LArgs {
     int *pr_need;
     int pr_n, pr_sz[2];
 };
-constexpr int PROJ_NW[2] = {12, 8};
 
 // Images that meet the cube of a node of the block (one wave: gn nodes at
 // most NG), in list order: ids to id, centre z to cz, their number returned

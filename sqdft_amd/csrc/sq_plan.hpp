@@ -1,0 +1,180 @@
+// sq_plan.hpp -- sizes and rules behind the launches of the grouped projector
+// kernels: how a batch is cut into groups, which shape and how much LDS a walk
+// takes.  Plain C++ without HIP, so that the rules can be tested on the CPU.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <vector>
+
+namespace sqk {
+
+constexpr int LCAP = 512;       // max images meeting one node cube
+constexpr int NG = 8;           // node cubes per workgroup of the grouped projector kernels
+constexpr int SLW = 10;         // LDS row of k_nlapplyg: NG projections padded to 80 B (rows
+                                // r and r + 4 would share banks at 64 B)
+constexpr int GLCAP = 1024;     // max images meeting the cubes of one group
+constexpr size_t LDS_MAX = 160 * 1024;
+
+// Image data that k_projs and k_projw read per image and plane, cached in LDS per group
+struct ImgMeta {
+    int ox, oy, oz;               // rc-box origin (unwrapped grid coordinates)
+    int w, np, t, ipb;            // box side, projectors, type, first image-projector id
+    long uoff;                    // offset of the image's U block in udv
+};
+
+// What the rules depend on: cube side, most projectors of an image, number of
+// image-projectors, side of the widest rc-box.
+struct ProjDims { int M, max_nproj, n_ip, w; };
+
+// The most values by which a member's cube may start after the corner of its
+// group's union: one plane, and rows and columns within (M + 3)^2 (the rule of
+// make_groups, whatever order the nodes come in).
+constexpr int group_pad(int M) { return M * M + 6 * M + 24; }
+
+// Compiled shapes of k_projw, the first that holds every group of the batch is
+// taken: waves per workgroup and register slots per wave.  One workgroup fills
+// a CU's LDS, so its waves are all that hides the loads: twelve, if the slots
+// that their 168 VGPRs hold are enough (the Al and LiH cells), else eight with
+// more slots.  Twelve against eight, us a pass: 8,192 nodes with FP64 35^3
+// cubes 1265 against 1549 (Lanczos) and 895 against 1175 (Chebyshev), 4,096
+// with FP32 ones 468 and 402 against 542 and 488; MFMA, 4,096 nodes with 31^3
+// cubes, 875 and 862 against 1142 and 1166.  With the union columns worked out
+// once per walk the twelve-wave ones take 1192, 863, 459, 358, 838 and 760.
+constexpr int PROJW_RPI = 3;
+struct ProjShape { int nw, R; };
+constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
+constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // MFMA: two doubles per slot and lane
+constexpr int PROJ_NW[2] = {12, 8};
+
+// How k_projw runs on vectors of ts bytes per value: on = 0 when it does not
+// apply; the matrix cores for FP64 tables of several projectors.
+struct ProjwUse { int on, mfma, w; };
+inline ProjwUse projw_use(const ProjDims &d, size_t ts)
+{
+    if (d.max_nproj < 1 || d.max_nproj > 4 || d.n_ip == 0) return {0, 0, 0};
+    // p channels in FP64: the matrix cores.  FP32 tables (mixed precision)
+    // stay with k_projs: its VALU sums of FP32 operands ran at 1.18 ms a pass
+    // on the 216-atom LiH batches against 1.67 ms (FP64 MFMAs fed by
+    // conversions), while in FP64 the two tied (2.3 ms).
+    if (d.max_nproj > 1 && ts == 4) return {0, 0, 0};
+    const int mfma = d.max_nproj > 1;
+    if (mfma ? d.w > 16 : d.w * d.w > 64 * PROJW_RPI) return {0, 0, 0};
+    return {1, mfma, d.w};
+}
+
+// LDS values per plane and member of a staged block of ux x uy columns: rows
+// padded to a pitch congruent to the box side modulo 32, the MFMA member
+// stride to 8 (as k_projw pads them).
+inline int projw_slab(const ProjwUse &pw, int ux, int uy)
+{
+    const int u = (ux + (((pw.w - ux) % 32) + 32) % 32) * uy;
+    return pw.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
+}
+
+// Slab capacity per plane and member: the union plane of a 4x2 block of cubes
+// or one cube.
+inline int projw_pu(int M, const ProjwUse &pw)
+{
+    return std::max(projw_slab(pw, M + 3, M + 1), projw_slab(pw, M, M));
+}
+
+// LDS bytes of a list of image data
+inline size_t images_lds(int images) { return ((size_t)std::max(images, 1) * sizeof(ImgMeta) + 15) / 16 * 16; }
+
+// LDS bytes of a table of a union's columns
+inline size_t columns_lds(int M)
+{
+    return (std::max((size_t)(M + 3) * (M + 3), (size_t)(M + 7) * M) * 4 + 15) / 16 * 16;
+}
+
+// LDS bytes of k_projw beside the slab: image data and union columns.
+inline size_t projw_head(int M, int images) { return images_lds(images) + columns_lds(M); }
+
+// Planes per slab.  VALU: one FP64 or two FP32 planes (a deeper slab keeps more
+// images alive than the slots of twelve waves: 17^3 cubes with three planes
+// took 269 us a pass with ten slots in eight waves against 81).  MFMA, whose
+// slots are small: about four load rounds of a workgroup between two barriers,
+// at most eight planes, as far as the LDS holds them beside a list of 256
+// images (25^3 cubes, two planes: 373 against 496 us a pass).
+inline int projw_sz(int M, const ProjwUse &pw, size_t ts)
+{
+    const size_t plane = (size_t)projw_pu(M, pw) * NG * ts, head = projw_head(M, 256);
+    const int lds = plane + head <= LDS_MAX ? (int)((LDS_MAX - head) / plane) : 1;
+    if (!pw.mfma) return ts == 4 ? 2 : 1;
+    return std::max(1, std::min({8, lds, 3072 / ((M + 3) * (M + 1))}));
+}
+
+// k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
+inline int projs_pu(int M) { return (M + 3) * (M + 3); }
+
+// Cuts B slots into groups of up to NG consecutive ones whose cubes the
+// staged projection kernels can walk together: the union plane fits the slab
+// capacity of every kernel that may run on the batch (vectors of ts[0 .. nts)
+// bytes per value), and the cubes are at most one plane apart in z.  A run ends
+// where the next node is too far away (a brick's edge, a gap in the caller's
+// list): walking such members one after the other in one workgroup, as unions
+// that do not fit would need, is several times slower: with runs of 8 slots cut
+// anywhere, a density step on a 15^3 LiH grid (25^3 cubes) took 534 ms and on a
+// 10^3 Al grid (17^3) 44.6 ms, against 155 and 15.2 ms.
+inline std::vector<int> make_groups(const ProjDims &dm, int n, const size_t *ts, int nts, const int *nodes, int B)
+{
+    const int M = dm.M;
+    std::vector<ProjwUse> use;
+    for (int i = 0; i < nts; ++i)
+        if (projw_use(dm, ts[i]).on) use.push_back(projw_use(dm, ts[i]));
+    auto fits = [&](int dx, int dy, int dz) {
+        if (dz > 1 || (M + dx) * (M + dy) > projs_pu(M)) return false;
+        for (const ProjwUse &pw : use)
+            if (projw_slab(pw, M + dx, M + dy) > projw_pu(M, pw)) return false;
+        return true;
+    };
+    std::vector<int> gst{0};
+    int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+    for (int b = 0; b < B; ++b) {
+        const int r[3] = {nodes[b] % n, (nodes[b] / n) % n, nodes[b] / (n * n)};
+        const int cnt = b - gst.back();
+        int l[3], h[3];
+        for (int d = 0; d < 3; ++d) {
+            l[d] = cnt ? std::min(lo[d], r[d]) : r[d];
+            h[d] = cnt ? std::max(hi[d], r[d]) : r[d];
+        }
+        if (cnt && (cnt == NG || !fits(h[0] - l[0], h[1] - l[1], h[2] - l[2]))) {
+            gst.push_back(b);
+            for (int d = 0; d < 3; ++d) l[d] = h[d] = r[d];
+        }
+        for (int d = 0; d < 3; ++d) { lo[d] = l[d]; hi[d] = h[d]; }
+    }
+    gst.push_back(B);
+    return gst;
+}
+
+// Workgroups that share the images of a group in k_projw.  A workgroup fills a
+// CU, so ng groups take ceil(ng / 256) rounds.  Half of a group's images,
+// consecutive in z, take 0.6 of a whole walk (they reach about three quarters of
+// its planes), a quarter 0.52: shares pay where they fill CUs that would idle.
+// us a pass with 1, 2 and 4 workgroups: a few nodes 63, 45, 36; 64 groups of
+// 17^3 cubes 25, 21, 19; about 150 of them 74, 88, 96; 364 of 25^3 LiH cubes 418,
+// 384, 466; 480 of them 385, 453, 565.
+inline int projw_split(int ng)
+{
+    int best = 1;
+    double t = 1e30;
+    const double cost[3] = {1.0, 0.6, 0.52};
+    for (int i = 0; i < 3; ++i) {
+        const double ti = (((long)ng << i) + 255) / 256 * cost[i];
+        if (ti < t) { t = ti; best = 1 << i; }
+    }
+    return best;
+}
+
+// LDS bytes of one k_nlapplyg workgroup (loc table, NG values per row, union
+// columns)
+inline size_t nlapplyg_lds(const ProjDims &d, int gl_max)
+{
+    const size_t head = ((size_t)std::max(d.n_ip, 1) * 4 + 15) / 16 * 16;
+    return head + (size_t)std::max(gl_max * d.max_nproj, 1) * SLW * sizeof(double) +
+           std::max((size_t)(d.M + 3) * (d.M + 3), (size_t)(d.M + 7) * d.M) * 4;
+}
+
+}  // namespace sqk

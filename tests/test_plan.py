@@ -1,0 +1,81 @@
+"""The host rules behind the projector kernels' launches (csrc/sq_plan.hpp),
+compiled for the CPU: groups of nodes, offsets inside a group and LDS sizes, over
+the cube sides and node lists that the kernels accept."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "sqdft_amd", "csrc")
+MAXM = 43   # largest cube side the kernels take
+
+SRC = r"""
+#include "sq_plan.hpp"
+#include <cstring>
+using namespace sqk;
+extern "C" {
+int groups(int M, int max_nproj, int n_ip, int w, int n, const int *ts, int nts, const int *nodes, int B, int *out)
+{
+    size_t t[2] = {(size_t)ts[0], (size_t)ts[1]};
+    const std::vector<int> g = make_groups({M, max_nproj, n_ip, w}, n, t, nts, nodes, B);
+    std::memcpy(out, g.data(), g.size() * sizeof(int));
+    return (int)g.size() - 1;
+}
+int pad(int M) { return group_pad(M); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src, lib = d / "plan.cpp", d / "libplan.so"
+    src.write_text(SRC)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC, str(src), "-o",
+                    str(lib)], check=True)
+    return C.CDLL(str(lib))
+
+
+def iptr(a):
+    return a.ctypes.data_as(C.POINTER(C.c_int))
+
+
+def groups_of(plan, M, np_, w, n, types, nodes):
+    nodes = np.ascontiguousarray(nodes, dtype=np.int32)
+    ts = np.array(list(types) + [8], dtype=np.int32)
+    out = np.zeros(nodes.size + 2, dtype=np.int32)
+    ng = plan.groups(M, np_, 100, w, n, iptr(ts), len(types), iptr(nodes), nodes.size, iptr(out))
+    return [nodes[out[i]:out[i + 1]] for i in range(ng)]
+
+
+def node_lists(M):
+    """(grid side, nodes): pairs a few rows, columns and planes apart, either one
+    first, and a shuffled whole grid."""
+    n = 40
+    rng = np.random.Generator(np.random.PCG64(M))
+    for dx in range(-20, 21):
+        for dy in range(0, 21):
+            a, b = (20, 1, 7), (20 + dx, 1 + dy, 7 + int(rng.integers(0, 3)))
+            p = [(c[2] * n + c[1]) * n + c[0] for c in (a, b)]
+            yield n, p if rng.integers(0, 2) else p[::-1]
+    yield 9, rng.permutation(9 ** 3)
+    yield 9, np.arange(9 ** 3)
+
+
+@pytest.mark.parametrize("np_,w", [(1, 9), (1, 13), (3, 9), (3, 15)])
+@pytest.mark.parametrize("types", [(8,), (4,), (4, 8)])
+def test_groups_stay_within_what_the_kernels_walk(plan, np_, w, types):
+    for M in range(3, MAXM + 1, 2):
+        for n, nodes in node_lists(M):
+            gs = groups_of(plan, M, np_, w, n, types, nodes)
+            assert np.array_equal(np.concatenate(gs), nodes)
+            for g in gs:
+                assert 1 <= g.size <= 8
+                r = np.stack([g % n, (g // n) % n, g // (n * n)])
+                d = r.max(axis=1) - r.min(axis=1)
+                assert (M + d[0]) * (M + d[1]) <= (M + 3) ** 2 and d[2] <= 1
+                # a member's cube starts at most group_pad values after the corner
+                assert d[2] * M * M + d[1] * M + d[0] <= plan.pad(M)
