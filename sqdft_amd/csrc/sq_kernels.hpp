@@ -1125,13 +1125,13 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
     // start pad values early so that none is negative (the masks keep every
     // address inside the member's cube)
     const int pad = group_pad(M);
-    const size_t gb = ((size_t)gn * M3 + pad) * TS;
+    const size_t gb = (size_t)group_range(M) * TS;
     const __amdgpu_buffer_rsrc_t rX = brsrc(A.V + (size_t)b0 * M3 - pad, gb);
     const __amdgpu_buffer_rsrc_t rY = brsrc((FORMED ? A.V2 : A.V) + (size_t)b0 * M3 - pad, gb);
     int kof[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
-        kof[m] = (pad + m * M3 + (uz0 - nk[m] + nloc) * M2 + (uy0 - nj[m] + nloc) * M + ux0 - ni[m] + nloc) * (int)TS;
+        kof[m] = member_offset(m, pad, M, M2, M3, ux0 - ni[m] + nloc, uy0 - nj[m] + nloc, uz0 - nk[m] + nloc) * (int)TS;
     const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
     const int upx = ux + (((wbox - ux) % 32) + 32) % 32, up = upx * uy;
     const int ms = MFMA ? up + (((8 - up) % 32) + 32) % 32 : up;
@@ -1449,7 +1449,7 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     // a member's offset of a union point is the union's plus a constant, the
     // scalar offset of the stores (pad keeps it from being negative)
     const int pad = group_pad(M);
-    const __amdgpu_buffer_rsrc_t rO = brsrc(A.nlv + (size_t)b0 * M3 - pad, ((size_t)gn * M3 + pad) * TS);
+    const __amdgpu_buffer_rsrc_t rO = brsrc(A.nlv + (size_t)b0 * M3 - pad, (size_t)group_range(M) * TS);
     // One union point at a time: its entries against every member's
     // projections, CH slots at a time up to the wave's largest count (a slot
     // past the point's count holds u = 0 and adds exact zeros), the first ones
@@ -1496,7 +1496,7 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
         const unsigned co = (unsigned)((P.z * M2 + (int)((P.cv >> 12) & 4095) * M + (int)(P.cv & 4095)) * (int)TS);
 #pragma unroll
         for (int m = 0; m < NG; ++m) {
-            const int kof = (pad + m * M3 + (ez0 - nk[m]) * M2 + (ey0 - nj[m]) * M + ex0 - ni[m]) * (int)TS;
+            const int kof = member_offset(m, pad, M, M2, M3, ex0 - ni[m], ey0 - nj[m], ez0 - nk[m]) * (int)TS;
             const bool ok = (P.cv & (1u << (24 + m))) && (unsigned)(gz - nk[m]) < (unsigned)M;
             bstore<T>((T)a[m], rO, ok ? co : OOB, kof);
         }

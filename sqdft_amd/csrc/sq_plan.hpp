@@ -32,6 +32,23 @@ struct ProjDims { int M, max_nproj, n_ip, w; };
 // make_groups, whatever order the nodes come in).
 constexpr int group_pad(int M) { return M * M + 6 * M + 24; }
 
+// Values in the resources of k_projw and k_nlapplyg: from group_pad before the
+// group's first vector to past a full group's last one.  Every scalar offset below
+// lies inside, that of an idle member (past the group's end or frozen) too, so that
+// nothing rests on what the hardware's range check makes of one past the end.
+// Lanes stay within the members' vectors by their masks: a masked lane's own
+// offset lies past the range.
+constexpr int group_range(int M) { return NG * M * M * M + 2 * group_pad(M); }
+
+// Scalar offset, in values, that takes an offset inside the group's union
+// (z M^2 + y M + x from its corner) to member m's vector; dx, dy, dz: the corner
+// minus the start of the member's cube, pad: group_pad (M2 and M3 come from the
+// caller: formed again from M they cost the FP64 Lanczos walk 6 % of its time).
+constexpr int member_offset(int m, int pad, int M, int M2, int M3, int dx, int dy, int dz)
+{
+    return pad + m * M3 + dz * M2 + dy * M + dx;
+}
+
 // Compiled shapes of k_projw, the first that holds every group of the batch is
 // taken: waves per workgroup and register slots per wave.  One workgroup fills
 // a CU's LDS, so its waves are all that hides the loads: twelve, if the slots

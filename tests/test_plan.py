@@ -25,6 +25,8 @@ int groups(int M, int max_nproj, int n_ip, int w, int n, const int *ts, int nts,
     return (int)g.size() - 1;
 }
 int pad(int M) { return group_pad(M); }
+int range(int M) { return group_range(M); }
+int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
 }
 """
 
@@ -79,3 +81,24 @@ def test_groups_stay_within_what_the_kernels_walk(plan, np_, w, types):
                 assert (M + d[0]) * (M + d[1]) <= (M + 3) ** 2 and d[2] <= 1
                 # a member's cube starts at most group_pad values after the corner
                 assert d[2] * M * M + d[1] * M + d[0] <= plan.pad(M)
+
+
+@pytest.mark.parametrize("M", [3, 5, 7, 9, 13, 17, 25, 35, 43])
+def test_scalar_offsets_stay_inside_their_resource(plan, M):
+    """Whichever members of a group are active: the offset of an active member
+    takes its cube to its own vector, that of an idle one is inside the range."""
+    rng = np.random.Generator(np.random.PCG64(M))
+    pad = plan.pad(M)
+    for n, nodes in list(node_lists(M))[::7] + [(9, rng.permutation(9 ** 3)), (9, np.arange(9 ** 3))]:
+        for g in groups_of(plan, M, 1, 9, n, (8,), nodes):
+            on = rng.integers(0, 2, 8).astype(bool) & (np.arange(8) < g.size)
+            if not on.any():
+                continue
+            start = np.stack([g % n, (g // n) % n, g // (n * n)], axis=1)
+            corner = start[on[:g.size]].min(axis=0)
+            for m in range(8):
+                d = corner - start[min(m, g.size - 1)]
+                off = plan.offset(m, M, int(d[0]), int(d[1]), int(d[2]))
+                assert 0 <= off < plan.range(M) < 2 ** 28, (n, g, m)
+                if on[m]:   # the first point of its cube, seen from the union's corner
+                    assert off - (d[2] * M * M + d[1] * M + d[0]) == pad + m * M ** 3
