@@ -1459,7 +1459,7 @@ struct ScratchView {
         bufs[n] = &d; saved_p[n] = d.p; saved_b[n] = d.bytes; ++n;
         d.p = c->scratch_ptr + off;
         d.bytes = bytes;
-        off += (bytes + 255) / 256 * 256;
+        off += NoallocSizes::round(bytes);
     }
     ~ScratchView()
     {
@@ -1467,27 +1467,16 @@ struct ScratchView {
     }
 };
 
-// Scratch bytes the allocation-free H v of nb nodes in ng groups needs
-// (per-call buffers rounded to 256 bytes each, without the group table; the
-// LCAP ints a node are part of the limit callers see and are left unused).
-size_t noalloc_bytes(const sqg_ctx *c, int nb, size_t ng)
-{
-    auto r = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t rs = c->real_size(), len = (size_t)nb * c->M3;
-    size_t t = r(nb * sizeof(int)) + r((size_t)nb * LCAP * sizeof(int)) + r(nb * sizeof(int)) +
-               r(ng * GLCAP * sizeof(int)) + r(ng * sizeof(int)) + r(16 * sizeof(int)) +
-               r((size_t)nb * std::max(c->n_ip, 1) * sizeof(double)) + r(len * rs);
-    if (c->p.precision == SQG_MIXED) t += 2 * r(len * rs) + r((size_t)c->nn * rs);
-    return t;
-}
-
 // H v of nb nodes in the scratch array.  Nodes too far apart to share groups
-// need more list space than full groups do: such a batch runs as two halves.
+// need more list space than full groups do: a batch that does not fit so runs as
+// two halves.
 static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int nb, const double *d_v, double *d_hv)
 {
     const std::vector<int> gst = groups_of(c, nodes, nb);
-    const size_t len = (size_t)nb * c->M3, rs = c->real_size(), ng = gst.size() - 1;
-    if (noalloc_bytes(c, nb, ng) + (gst.size() * sizeof(int) + 255) / 256 * 256 > (size_t)SQG_NOALLOC_SCRATCH_BYTES) {
+    const size_t len = (size_t)nb * c->M3;
+    const bool mixed = c->p.precision == SQG_MIXED;
+    const NoallocSizes z(c->dims(), nb, gst.size() - 1, c->real_size(), mixed, c->nn);
+    if (z.total() > (size_t)SQG_NOALLOC_SCRATCH_BYTES) {
         if (nb == 1) return SQG_E_OVERFLOW;
         const int h = nb / 2;
         const int st = noalloc_piece(c, d_veff, nodes, h, d_v, d_hv);
@@ -1495,18 +1484,17 @@ static int noalloc_piece(sqg_ctx *c, const double *d_veff, const int *nodes, int
         return noalloc_piece(c, d_veff, nodes + h, nb - h, d_v + (size_t)h * c->M3, d_hv + (size_t)h * c->M3);
     }
     ScratchView V(c);
-    V.put(c->node_list, nb * sizeof(int));
-    V.put(c->gst, gst.size() * sizeof(int));
-    V.put(c->glist, ng * GLCAP * sizeof(int));
-    V.put(c->glist_cnt, ng * sizeof(int));
-    V.put(c->flags, 16 * sizeof(int));
-    V.put(c->s, (size_t)nb * std::max(c->n_ip, 1) * sizeof(double));
-    V.put(c->NLv, len * rs);
-    const bool mixed = c->p.precision == SQG_MIXED;
+    V.put(c->node_list, z.node_list);
+    V.put(c->gst, z.gst);
+    V.put(c->glist, z.glist);
+    V.put(c->glist_cnt, z.glist_cnt);
+    V.put(c->flags, z.flags);
+    V.put(c->s, z.s);
+    V.put(c->NLv, z.NLv);
     if (mixed) {   // FP32 copies of the input, the output and Veff
-        V.put(c->X, len * rs);
-        V.put(c->Y, len * rs);
-        V.put(c->veff, (size_t)c->nn * rs);
+        V.put(c->X, z.X);
+        V.put(c->Y, z.Y);
+        V.put(c->veff, z.veff);
     }
     // flags start at zero (a fill kernel, not a memset node)
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>(), (size_t)16, 0);
@@ -1552,8 +1540,9 @@ int sqg_hsub_apply_batch_noalloc(sqg_ctx *c, const double *d_veff, const int *no
     for (int i = 0; i < nb; ++i)
         if (nodes[i] < 0 || nodes[i] >= c->nn) return SQG_E_ARG;
     if (nb == 0) return SQG_OK;
-    // the limit callers see: nb nodes in full groups
-    if (noalloc_bytes(c, nb, (size_t)(nb + NG - 1) / NG) > (size_t)SQG_NOALLOC_SCRATCH_BYTES) return SQG_E_OVERFLOW;
+    if (noalloc_limit(c->dims(), nb, c->real_size(), c->p.precision == SQG_MIXED, c->nn) >
+        (size_t)SQG_NOALLOC_SCRATCH_BYTES)
+        return SQG_E_OVERFLOW;
     HIPCHK(hipSetDevice(c->p.device));
     return noalloc_piece(c, d_veff, nodes, nb, d_v, d_hv);
 }

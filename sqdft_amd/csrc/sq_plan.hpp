@@ -194,4 +194,41 @@ inline size_t nlapplyg_lds(const ProjDims &d, int gl_max)
            std::max((size_t)(d.M + 3) * (d.M + 3), (size_t)(d.M + 7) * d.M) * 4;
 }
 
+// Per-call buffers of the allocation-free H v of nb nodes in ng groups, in
+// bytes: vectors of rs bytes per value, FP32 copies of the input, the output and
+// Veff (nn values) where mixed.
+struct NoallocSizes {
+    size_t node_list, gst, glist, glist_cnt, flags, s, NLv, X, Y, veff;
+    static constexpr size_t round(size_t b) { return (b + 255) / 256 * 256; }
+    NoallocSizes(const ProjDims &d, int nb, size_t ng, size_t rs, bool mixed, size_t nn)
+    {
+        const size_t len = (size_t)nb * d.M * d.M * d.M;
+        node_list = nb * sizeof(int);
+        gst = (ng + 1) * sizeof(int);
+        glist = ng * GLCAP * sizeof(int);
+        glist_cnt = ng * sizeof(int);
+        flags = 16 * sizeof(int);
+        s = (size_t)nb * std::max(d.n_ip, 1) * sizeof(double);
+        NLv = len * rs;
+        X = Y = mixed ? len * rs : 0;
+        veff = mixed ? nn * rs : 0;
+    }
+    // what they take, each rounded to 256 bytes
+    size_t total() const
+    {
+        size_t t = 0;
+        for (size_t b : {node_list, gst, glist, glist_cnt, flags, s, NLv, X, Y, veff}) t += round(b);
+        return t;
+    }
+};
+
+// Scratch bytes by which nb nodes are taken or refused (the limit that callers
+// see): full groups, and LCAP + 1 ints a node, room for lists of its own that this
+// path does not build and that lists of groups with fewer nodes may take.
+inline size_t noalloc_limit(const ProjDims &d, int nb, size_t rs, bool mixed, size_t nn)
+{
+    const NoallocSizes z(d, nb, (size_t)(nb + NG - 1) / NG, rs, mixed, nn);
+    return z.total() - z.round(z.gst) + z.round((size_t)nb * LCAP * sizeof(int)) + z.round((size_t)nb * sizeof(int));
+}
+
 }  // namespace sqk

@@ -24,6 +24,14 @@ int groups(int M, int max_nproj, int n_ip, int w, int n, const int *ts, int nts,
     std::memcpy(out, g.data(), g.size() * sizeof(int));
     return (int)g.size() - 1;
 }
+long noalloc_need(int M, int n_ip, int nb, long ng, int rs, int nn)
+{
+    return (long)NoallocSizes({M, 1, n_ip, 9}, nb, ng, rs, rs == 4, nn).total();
+}
+long noalloc_cap(int M, int n_ip, int nb, int rs, int nn)
+{
+    return (long)noalloc_limit({M, 1, n_ip, 9}, nb, rs, rs == 4, nn);
+}
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -38,7 +46,10 @@ def plan(tmp_path_factory):
     src.write_text(SRC)
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC, str(src), "-o",
                     str(lib)], check=True)
-    return C.CDLL(str(lib))
+    d = C.CDLL(str(lib))
+    d.noalloc_need.restype = d.noalloc_cap.restype = C.c_long
+    d.noalloc_need.argtypes = [C.c_int, C.c_int, C.c_int, C.c_long, C.c_int, C.c_int]
+    return d
 
 
 def iptr(a):
@@ -102,3 +113,21 @@ def test_scalar_offsets_stay_inside_their_resource(plan, M):
                 assert 0 <= off < plan.range(M) < 2 ** 28, (n, g, m)
                 if on[m]:   # the first point of its cube, seen from the union's corner
                     assert off - (d[2] * M * M + d[1] * M + d[0]) == pad + m * M ** 3
+
+
+@pytest.mark.parametrize("rs", [8, 4])
+@pytest.mark.parametrize("M,n_ip", [(7, 62), (7, 186), (17, 900), (35, 3000), (43, 20000)])
+def test_allocation_free_calls_split_only_where_they_must(plan, M, n_ip, rs):
+    """A batch that the scratch limit accepts fits whole when its groups are full,
+    and up to a quarter of them may hold one node; the limit itself is the sum of
+    the buffers in full groups and LCAP + 1 ints a node."""
+    up = lambda b: -(-b // 256) * 256   # noqa: E731
+    for nb in (1, 2, 7, 8, 9, 64, 1000, 1001, 9133, 60000):
+        ng, nn = -(-nb // 8), 4096
+        ints = [nb, nb * 512, nb, ng * 1024, ng, 16]
+        cap = sum(up(4 * i) for i in ints) + up(8 * nb * n_ip) + up(nb * M ** 3 * rs)
+        if rs == 4:
+            cap += 2 * up(nb * M ** 3 * rs) + up(nn * rs)
+        assert plan.noalloc_cap(M, n_ip, nb, rs, nn) == cap
+        assert plan.noalloc_need(M, n_ip, nb, ng, rs, nn) <= cap
+        assert plan.noalloc_need(M, n_ip, nb, ng + nb // 4, rs, nn) <= cap
