@@ -60,6 +60,11 @@ void pinv_solve(const double *Ac, const double *b, double *x, int m)
     }
 }
 
+// Iterations enqueued before the host looks whether the solve has stopped: past
+// the one that stops it they are empty launches, so a large p (plain Jacobi
+// relaxation) must not put maxiter of them on the stream.
+constexpr int AAJ_RUN = 16;
+
 template <int M>
 void gram_go(sqg_ctx *c, int nb, size_t N)
 {
@@ -104,11 +109,11 @@ int poisson_aaj(sqg_ctx *c, const double *rhs, const double *guess, double tol, 
     int iter = 1;
     while (!ctl.done) {
         // the iterations up to the next Anderson step (every p-th, past the
-        // first) or the last one, then one wait for all of them: with a wait
-        // per iteration one took 36 us around kernels of 5 (an SCF step's
-        // Poisson, Vxc and energy on a 32^3 grid: 3.3 ms, now 1.9)
+        // first) or the last one, but at most AAJ_RUN, then one wait for all of
+        // them: with a wait per iteration one took 36 us around kernels of 5 (an
+        // SCF step's Poisson, Vxc and energy on a 32^3 grid: 3.3 ms, now 2.1)
         int step = 0;   // the iteration with the Anderson step
-        for (; !step && iter <= maxiter; ++iter) {
+        for (int run = 0; run < AAJ_RUN && !step && iter <= maxiter; ++run, ++iter) {
             AajArgs A{};
             A.n = n;
             A.ctl = c->pz_ctl.as<AajCtl>();
