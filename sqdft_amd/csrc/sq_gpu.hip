@@ -1727,8 +1727,11 @@ int sqg_tangent_veff(sqg_ctx *c, const double *dV, int fixed_n, double *drho)
 int sqg_poisson_aaj(sqg_ctx *c, const double *rhs, const double *phi_guess, double tol, int maxiter, double beta,
                     int m, int p, double *phi, int *iters, double *relres)
 {
-    // periodic stencil indices wrap once: the grid must span the stencil half-width
-    if (!c || !rhs || !phi_guess || !phi || m < 1 || m > 8 || p < 1 || maxiter < 1 || !(tol > 0) || c->p.n < FDN)
+    // periodic stencil indices wrap once: the grid must span the stencil half-width;
+    // a tolerance that every residual meets (infinite, or lost on tol + 1) asks for
+    // no iteration and is refused
+    if (!c || !rhs || !phi_guess || !phi || m < 1 || m > 8 || p < 1 || maxiter < 1 || !(tol > 0) || !(tol + 1 > tol) ||
+        c->p.n < FDN)
         return SQG_E_ARG;
     HIPCHK(hipSetDevice(c->p.device));
     return poisson_aaj(c, rhs, phi_guess, tol, maxiter, beta, m, p, phi, iters, relres);

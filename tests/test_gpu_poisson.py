@@ -87,3 +87,11 @@ def test_converged_start_does_not_pay_for_maxiter(al):
         print("converged start", t, flush=True)
         assert code == 0 and it == 1
     assert t < 0.1
+
+
+@pytest.mark.parametrize("tol", [0.0, -1.0, float("nan"), float("inf"), 1e17])
+def test_tolerances_that_ask_for_no_iteration_are_refused(al, tol):
+    S, scf, rhs = al
+    for maxiter in (1, 100):
+        code, phi, it, _ = solve(scf, rhs, np.ones(S.nn), tol, maxiter, 0.6, 7, 6)
+        assert code == -1 and it == 0 and not phi.any()   # SQG_E_ARG, nothing written
