@@ -152,8 +152,8 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     }
     hipLaunchKernelGGL((k_adj_center<T>), dim3((B + 127) / 128), dim3(128), 0, c->st, B, (int)M3, cidx,
                        (const T *)tb(1), G);
-    const int X = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : 128;   // threads along x
-    hipLaunchKernelGGL((k_adj_gather<T>), dim3(n * n), dim3(AGT), 0, c->st, n, c->p.nloc, z0, nz, X,
+    auto gather = n < c->M ? k_adj_gather<T, true> : k_adj_gather<T, false>;
+    hipLaunchKernelGGL(gather, dim3(n * n, (n + AGX - 1) / AGX), dim3(AGT), 0, c->st, n, c->p.nloc, z0, nz,
                        c->adj_slot.as<int>(), (const T *)G, c->zee_all.as<double>(), c->adj_out.as<double>());
     int ovf4[4] = {0, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(ovf4, c->flags.p, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));

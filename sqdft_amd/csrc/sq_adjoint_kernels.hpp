@@ -96,56 +96,62 @@ __global__ void k_adj_center(int B, int M3, int c, const T *tb1, T *G)
 
 // dL/dVeff(g) += sum over the batch's nodes i whose cube holds g of G_i(p)/zee_i.
 // The batch is the nodes of z-planes [z0, z0 + nz); slot_of gives the slot of
-// the node at ((z - z0) n + y) n + x.  One workgroup per grid row (gy, gz):
-// thread (x, sub) owns gx = x, x + X, ... and the cube offsets dz = sub mod S,
-// and walks the nodes of each row of nodes, so that neighbouring lanes read
-// neighbouring values of one node's vector (each value is read once: HBM
-// bound).  Every sum runs in a fixed order over its nodes and then over the
-// subs: deterministic, no atomics.  A thread per grid point walked all its
-// (2 nloc + 1)^3 offsets alone, with loads a cube apart between lanes: 24.5 ms
-// for 4,096 nodes with 35^3 cubes (16 workgroups); an adjoint product on the
-// 16^3 Al grid 266 -> 242 ms with this kernel.
-constexpr int AGT = 256;
-template <typename T>
-__global__ void __launch_bounds__(AGT) k_adj_gather(int n, int nloc, int z0, int nz, int X, const int *slot_of,
-                                                    const T *G, const double *zee, double *out)
+// the node at ((z - z0) n + y) n + x.  A workgroup owns AGX points of a grid row
+// (gy, gz): thread (x, sub) takes point x and the rows of cube offsets (dz, dy) =
+// sub mod AGT / AGX, and walks the nodes of that row of nodes whose cubes reach the
+// AGX points (all n of them, or M + AGX - 1), so that neighbouring lanes read
+// neighbouring values of one node's vector.  Every sum runs in a fixed order over
+// its rows and nodes and then over the subs: deterministic, no atomics.
+// MULTI: the grid is smaller than the cube, which then holds a point several
+// times.  Bound by the latency of the walks (slot, weight and value of a node, a
+// division each): 35^3 cubes on a 16^3 grid 2.10 ms (1.4 GB, 0.67 TB/s), on 32^3,
+// one batch, 4.75 ms; 9^3 on 36^3 0.21 ms; a batch of 13^3 on 48^3 0.52 ms, of 9^3
+// on 96^3 0.24 ms.  A walk of all n nodes of each row took 2.44, 7.74, 0.92, 2.33
+// and 2.10 ms, a thread per point that reads values a cube apart 24.4, 24.0, 0.42,
+// 1.42 and 0.44 ms.
+constexpr int AGT = 256, AGX = 16;
+template <typename T, bool MULTI>
+__global__ void __launch_bounds__(AGT) k_adj_gather(int n, int nloc, int z0, int nz, const int *slot_of, const T *G,
+                                                    const double *zee, double *out)
 {
     __shared__ double part[AGT];
-    const int gy = blockIdx.x % n, gz = blockIdx.x / n;
-    const int M = 2 * nloc + 1, M2 = M * M;
-    const size_t M3 = (size_t)M2 * M;
-    const int S = AGT / X, sub = threadIdx.x / X, tx = threadIdx.x - sub * X;
-    for (int x0 = 0; x0 < n; x0 += X) {
-        const int gx = x0 + tx;
-        double acc = 0.0;
-        if (sub < S && gx < n) {
-            for (int dz = -nloc + sub; dz <= nloc; dz += S) {
-                const int bz = wrapn(gz - dz, n), zs = bz - z0;
-                if (zs < 0 || zs >= nz) continue;
-                for (int dy = -nloc; dy <= nloc; ++dy) {
-                    const int by = wrapn(gy - dy, n);
-                    const int row = (zs * n + by) * n, zrow = (bz * n + by) * n;
-                    const T *g0 = G + ((dz + nloc) * M + (dy + nloc)) * M + nloc;
-                    for (int bx = 0; bx < n; ++bx) {
-                        const T *g = g0 + slot_of[row + bx] * M3;
-                        const double iz = 1.0 / zee[zrow + bx];
-                        // offsets dx = gx - bx modulo n inside the cube
-                        int dx = gx - bx;
-                        dx -= (dx + nloc) / n * n;
-                        if (dx < -nloc) dx += n;
-                        for (; dx <= nloc; dx += n) acc += (double)g[dx] * iz;
-                    }
-                }
+    const int gy = blockIdx.x % n, gz = blockIdx.x / n, x0 = blockIdx.y * AGX;
+    const int M = 2 * nloc + 1;
+    const size_t M3 = (size_t)M * M * M;
+    const int sub = threadIdx.x / AGX, tx = threadIdx.x % AGX, gx = x0 + tx;
+    // the nodes are bx = x0 - nloc + i modulo n; the point's offset in the cube of the
+    // first one (the smallest from -nloc on), one less in that of each next
+    const int cnt = min(n, M + AGX - 1), b0 = wrapn(x0 - nloc, n), d0 = (tx + 2 * nloc) % n - nloc;
+    double acc = 0.0;
+    for (int r = sub; r < M * M; r += AGT / AGX) {
+        const int dz = r / M - nloc, dy = r % M - nloc;
+        const int bz = wrapn(gz - dz, n), zs = bz - z0;
+        if (zs < 0 || zs >= nz) continue;
+        const int by = wrapn(gy - dy, n);
+        const int *sl = slot_of + (zs * n + by) * n;
+        const double *zr = zee + (bz * n + by) * n;
+        const T *g0 = G + (size_t)r * M + nloc;
+        int d = d0, bx = b0;
+#pragma unroll 4
+        for (int i = 0; i < cnt; ++i) {
+            const T *g = g0 + sl[bx] * M3;
+            const double z = zr[bx];
+            if constexpr (MULTI) {
+                for (int e = d; e <= nloc; e += n) acc += (double)g[e] / z;
+            } else {
+                const double v = (double)g[min(d, nloc)] / z;
+                acc += d <= nloc ? v : 0.0;
             }
+            if (--d < -nloc) d += n;
+            if (++bx == n) bx = 0;
         }
-        part[threadIdx.x] = acc;
-        __syncthreads();
-        if (sub == 0 && gx < n) {
-            double t = acc;
-            for (int k = 1; k < S; ++k) t += part[k * X + tx];
-            out[((size_t)gz * n + gy) * n + gx] += t;
-        }
-        __syncthreads();
+    }
+    part[threadIdx.x] = acc;
+    __syncthreads();
+    if (sub == 0 && gx < n) {
+        double t = acc;
+        for (int k = 1; k < AGT / AGX; ++k) t += part[k * AGX + tx];
+        out[((size_t)gz * n + gy) * n + gx] += t;
     }
 }
 
