@@ -242,15 +242,19 @@ int ensure_batch(sqg_ctx *c, int B)
     return SQG_OK;
 }
 
-int choose_batch(sqg_ctx *c, int want, int nvec = 2)
+// Nodes per batch: at most want, and what 0.6 of the free memory and of the batch
+// buffers held now takes.  nvec: see batch_node_bytes; node_lists: the pass builds
+// image lists per node.
+int choose_batch(sqg_ctx *c, int want, int nvec = 2, bool node_lists = false)
 {
     int B = c->p.batch_nodes > 0 ? c->p.batch_nodes : c->nn;
     B = std::min(B, want);
     size_t freeb = 0, totb = 0;
     if (hipMemGetInfo(&freeb, &totb) == hipSuccess && freeb > 0) {
-        const size_t per = (nvec + 3) * (size_t)c->M3 * c->real_size() + (size_t)std::max(c->n_ip, 1) * 8 +
-                           LCAP * 4 + GLCAP * 4 / NG + 4 * (MAXIT + 2) * 8 + 256;
-        const size_t cap = (size_t)(0.6 * (double)(freeb + (size_t)c->Bcap * per)) / per;
+        const size_t per = batch_node_bytes(c->dims(), c->real_size(), nvec);
+        const size_t held = (size_t)c->Bcap * per + c->glist.bytes + c->glist_cnt.bytes + c->gst.bytes +
+                            c->list.bytes + c->list_cnt.bytes;
+        const size_t cap = (size_t)(0.6 * (double)(freeb + held)) / (per + batch_list_bytes(node_lists));
         if ((size_t)B > cap) B = (int)std::max<size_t>(cap, 1);
     }
     return std::max(B, 1);
@@ -1556,7 +1560,7 @@ int sqg_forces_nonlocal(sqg_ctx *c, double *f)
     for (int i = 0; i < 3 * na; ++i) f[i] = 0.0;
     if (c->n_ip == 0) return SQG_OK;
     std::vector<double> rec;   // node, atom, fx, fy, fz per contributing image
-    const int cap = choose_batch(c, c->nn, 3);
+    const int cap = choose_batch(c, c->nn, 3, true);
     const std::vector<int> nodes = node_order(c->p.n);
     int done_n = 0;
     while (done_n < c->nn) {

@@ -26,7 +26,6 @@ namespace sqk {
 constexpr int FDN = 6;          // half FD order (12th-order stencil)
 constexpr int WIN = 2 * FDN + 1;
 constexpr int MAXM = 43;        // largest cube side one workgroup marches ((M+1)/2*M <= 1024)
-constexpr int MAXIT = 500;      // Lanczos max_iter (sq.cpp:967)
 
 __device__ __forceinline__ int wrapn(int a, int n)
 {

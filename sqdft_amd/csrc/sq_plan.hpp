@@ -14,6 +14,7 @@ constexpr int NG = 8;           // node cubes per workgroup of the grouped proje
 constexpr int SLW = 10;         // LDS row of k_nlapplyg: NG projections padded to 80 B (rows
                                 // r and r + 4 would share banks at 64 B)
 constexpr int GLCAP = 1024;     // max images meeting the cubes of one group
+constexpr int MAXIT = 500;      // Lanczos max_iter (sq.cpp:967)
 constexpr size_t LDS_MAX = 160 * 1024;
 
 // Image data that k_projs and k_projw read per image and plane, cached in LDS per group
@@ -192,6 +193,21 @@ inline size_t nlapplyg_lds(const ProjDims &d, int gl_max)
     const size_t head = ((size_t)std::max(d.n_ip, 1) * 4 + 15) / 16 * 16;
     return head + (size_t)std::max(gl_max * d.max_nproj, 1) * SLW * sizeof(double) +
            std::max((size_t)(d.M + 3) * (d.M + 3), (size_t)(d.M + 7) * d.M) * 4;
+}
+
+// Device bytes that a batch holds per node: nvec + 3 vectors of rs bytes per value
+// (the two Lanczos pairs and the nonlocal term, and what a pass adds), the
+// projections, the Lanczos tridiagonals with their scratch, and scalars ...
+inline size_t batch_node_bytes(const ProjDims &d, size_t rs, int nvec)
+{
+    return (nvec + 3) * (size_t)d.M * d.M * d.M * rs + (size_t)std::max(d.n_ip, 1) * 8 + 4 * (MAXIT + 2) * 8 + 256;
+}
+
+// ... and of image lists at most: those of a group, which may hold one node where
+// the nodes are far apart, and a node's own (the forces).
+constexpr size_t batch_list_bytes(bool node_lists)
+{
+    return (GLCAP + 2) * sizeof(int) + (node_lists ? (LCAP + 1) * sizeof(int) : 0);
 }
 
 // Per-call buffers of the allocation-free H v of nb nodes in ng groups, in

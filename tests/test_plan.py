@@ -32,6 +32,10 @@ long noalloc_cap(int M, int n_ip, int nb, int rs, int nn)
 {
     return (long)noalloc_limit({M, 1, n_ip, 9}, nb, rs, rs == 4, nn);
 }
+long node_bytes(int M, int n_ip, int rs, int nvec, int lists)
+{
+    return (long)(batch_node_bytes({M, 1, n_ip, 9}, rs, nvec) + batch_list_bytes(lists));
+}
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -49,6 +53,7 @@ def plan(tmp_path_factory):
     d = C.CDLL(str(lib))
     d.noalloc_need.restype = d.noalloc_cap.restype = C.c_long
     d.noalloc_need.argtypes = [C.c_int, C.c_int, C.c_int, C.c_long, C.c_int, C.c_int]
+    d.node_bytes.restype = C.c_long
     return d
 
 
@@ -131,3 +136,15 @@ def test_allocation_free_calls_split_only_where_they_must(plan, M, n_ip, rs):
         assert plan.noalloc_cap(M, n_ip, nb, rs, nn) == cap
         assert plan.noalloc_need(M, n_ip, nb, ng, rs, nn) <= cap
         assert plan.noalloc_need(M, n_ip, nb, ng + nb // 4, rs, nn) <= cap
+
+
+@pytest.mark.parametrize("M,n_ip", [(7, 62), (17, 900), (43, 20000)])
+@pytest.mark.parametrize("rs", [8, 4])
+def test_batches_budget_for_groups_of_one_node(plan, M, n_ip, rs):
+    """A batch is sized for everything it allocates per node: five vectors (one
+    more for the forces), projections, four rows of 502 tridiagonal entries, 22
+    doubles and 3 ints of scalars, and the lists of a group that holds one node."""
+    held = 5 * M ** 3 * rs + 8 * n_ip + 4 * 502 * 8 + 8 * (11 + 8 + 4 + 2) + 4 * 3
+    group = 4 * (1024 + 1 + 1)
+    assert plan.node_bytes(M, n_ip, rs, 2, 0) >= held + group
+    assert plan.node_bytes(M, n_ip, rs, 3, 1) >= held + M ** 3 * rs + group + 4 * (512 + 1)
