@@ -448,9 +448,8 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
     const size_t sa = images_lds(c->gl_max);
     // projector values are loaded and summed for npu of the mp slots
     const int npu = mp == 1 ? 1 : c->max_nproj == 3 ? 3 : 4;
-    P.pu = projs_pu(c->M);
     for (int sz : {D, D / 2, 1}) {
-        const size_t shs = sa + (size_t)P.pu * NG * sizeof(T) * sz;
+        const size_t shs = sa + (size_t)projs_pu(c->M) * NG * sizeof(T) * sz;
         if (shs > 160 * 1024) continue;
         if (sz == 4) projs_np<T, FORMED, 4>(c, shs, P, npu);
         else if (sz == 2) projs_np<T, FORMED, 2>(c, shs, P, npu);

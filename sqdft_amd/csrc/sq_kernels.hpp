@@ -589,7 +589,6 @@ struct PArgs {
     const T *V2;                  // LANCZOS: previous normalized vector
     double *s;                    // [B][n_ip] out
     int n_ip;
-    const int *list, *list_cnt;   // [B][LCAP], [B]
     const int *img_type, *img_nn, *ip_base;
     const long *udv_off;
     const T *udv;
@@ -598,7 +597,6 @@ struct PArgs {
     const double *ca, *ib;        // LANCZOS: projects v = (V - ca V2) * ib
     const int *gst;               // [groups + 1] first slot of each group
     const int *glist, *glist_cnt; // group image lists
-    int pu;                       // k_projs: LDS values per plane and member
     int sz;                       // k_projw: planes per slab
 };
 
@@ -856,7 +854,7 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
     }
     const int cnt = A.glist_cnt[q];
     if (nact == 0 || cnt == 0) return;
-    // LDS: image data [cnt] | staged slab [SZ][pu][NM]
+    // LDS: image data [cnt] | staged slab [SZ][union points][NM]
     __shared__ int sh_ncmax, sh_lo, sh_hi;
     if (tid == 0) sh_ncmax = 0;
     __syncthreads();
