@@ -81,7 +81,7 @@ struct sqg_ctx {
     DBuf gst, glist, glist_cnt;    // first slot of each group, group image lists
     int ng = 0;                    // groups of the current batch
     int gl_max = 0;                // longest group list of the current batch
-    int proj_shape = -1;           // compiled shape of k_projw for the batch (-1: k_projs instead)
+    ProjwPlan projw[2];            // k_projw on the batch's vectors of 4 and 8 bytes per value
     DBuf lred, aa, bb, dq, eq, lmin, lmax, lmin_prev, lmax_prev, lchg, cnt, done, ca, ib, bprev;
     DBuf chiB, zeeB, center, dots, htemp;
     // all-node state of the last density step
@@ -335,7 +335,7 @@ std::vector<int> groups_of(const sqg_ctx *c, const int *nodes, int B)
 }
 
 // Image lists of the B nodes in node_list on the groups gst, and per node where
-// node_lists asks for them (the forces); sets ng, gl_max and proj_shape.  Overflow
+// node_lists asks for them (the forces); sets ng, gl_max and projw.  Overflow
 // goes to flags[0].
 int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
 {
@@ -361,14 +361,11 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     size_t ts[2];
     const int nsh = stored_types(c, ts);
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)2, 0);
-    bool any_on = false, any_mfma = false;
     for (int i = 0; i < nsh; ++i) {
         const ProjwUse pw = projw_use(dm, ts[i]);
         if (!pw.on) continue;
         L.pr_need = c->flags.as<int>() + 4;
         L.pr_sz[L.pr_n++] = projw_sz(c->M, pw, ts[i]);
-        any_on = true;
-        any_mfma |= pw.mfma != 0;
     }
     hipLaunchKernelGGL(k_group_images, dim3(ng), dim3(64), 0, c->st, L);
     if (node_lists) hipLaunchKernelGGL(k_node_images, dim3(B), dim3(64), 0, c->st, L);
@@ -378,11 +375,11 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     HIPCHK(hipStreamSynchronize(c->st));
     c->gl_max = 0;
     for (int i = 0; i < ng; ++i) c->gl_max = std::max(c->gl_max, gc[i]);
-    // the sums are the same in every shape, so batches stay bitwise alike
-    c->proj_shape = -1;
-    const ProjShape *sh = any_mfma ? PROJM_SHAPES : PROJR_SHAPES;
-    for (int i = 0; any_on && i < (any_mfma ? 2 : 4); ++i)
-        if (gc[ng + (sh[i].nw == PROJ_NW[1])] <= sh[i].R) { c->proj_shape = i; break; }
+    const int need[2] = {gc[ng], gc[ng + 1]};
+    for (int i = 0; i < nsh; ++i) {
+        const ProjwUse pw = projw_use(dm, ts[i]);
+        c->projw[ts[i] == 8] = projw_plan(c->M, pw, ts[i], projw_sz(c->M, pw, ts[i]), c->gl_max, need);
+    }
     return SQG_OK;
 }
 
@@ -422,72 +419,62 @@ void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
 }
 
 template <typename T, int MAXP, int FORMED, int SZ, int NT, int NPU>
-void projs_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
+void projs_go(sqg_ctx *c, const ProjsPlan &pl, const PArgs<T> &P)
 {
     auto fn = k_projs<T, MAXP, FORMED, SZ, NT, NPU>;
-    if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(c->ng), dim3(NT), shm, c->st, P);
+    if (pl.lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
+    hipLaunchKernelGGL(fn, dim3(c->ng, pl.shares), dim3(NT), pl.lds, c->st, P);
 }
 
 template <typename T, int FORMED, int SZ>
-void projs_np(sqg_ctx *c, size_t shs, const PArgs<T> &P, int npu)
+void projs_np(sqg_ctx *c, const ProjsPlan &pl, const PArgs<T> &P, int npu)
 {
     constexpr int NT = 512;
-    if (npu == 1) projs_go<T, 1, FORMED, SZ, NT, 1>(c, shs, P);
-    else if (npu == 3) projs_go<T, 4, FORMED, SZ, NT, 3>(c, shs, P);
-    else projs_go<T, 4, FORMED, SZ, NT, 4>(c, shs, P);
+    if (npu == 1) projs_go<T, 1, FORMED, SZ, NT, 1>(c, pl, P);
+    else if (npu == 3) projs_go<T, 4, FORMED, SZ, NT, 3>(c, pl, P);
+    else projs_go<T, 4, FORMED, SZ, NT, 4>(c, pl, P);
 }
 
-// Staged projections (k_projs, all members of a group per workgroup) with the
-// deepest slab (planes staged at once) that fits the LDS.  Returns false when
-// not even a single union plane fits.
+// Staged projections (k_projs, all members of a group per workgroup).  Returns
+// false when not even a single union plane fits the LDS.
 template <typename T, int FORMED>
 bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
 {
-    constexpr int D = sizeof(T) == 4 ? 4 : 2;   // deep slab (planes)
-    const size_t sa = images_lds(c->gl_max);
+    const ProjsPlan pl = projs_plan(c->M, sizeof(T), sizeof(T) == 4 ? 4 : 2, c->gl_max);
     // projector values are loaded and summed for npu of the mp slots
     const int npu = mp == 1 ? 1 : c->max_nproj == 3 ? 3 : 4;
-    for (int sz : {D, D / 2, 1}) {
-        const size_t shs = sa + (size_t)projs_pu(c->M) * NG * sizeof(T) * sz;
-        if (shs > 160 * 1024) continue;
-        if (sz == 4) projs_np<T, FORMED, 4>(c, shs, P, npu);
-        else if (sz == 2) projs_np<T, FORMED, 2>(c, shs, P, npu);
-        else projs_np<T, FORMED, 1>(c, shs, P, npu);
-        return true;
-    }
-    return false;
+    if (pl.sz == 4) projs_np<T, FORMED, 4>(c, pl, P, npu);
+    else if (pl.sz == 2) projs_np<T, FORMED, 2>(c, pl, P, npu);
+    else if (pl.sz == 1) projs_np<T, FORMED, 1>(c, pl, P, npu);
+    return pl.sz > 0;
 }
 
 template <typename T, int FORMED, bool MFMA, int I>
-void projw_go(sqg_ctx *c, size_t shm, const PArgs<T> &P)
+void projw_go(sqg_ctx *c, const ProjwPlan &pl, const PArgs<T> &P)
 {
     constexpr ProjShape S = MFMA ? PROJM_SHAPES[MFMA ? I : 0] : PROJR_SHAPES[I];
     auto fn = k_projw<T, FORMED, S.nw * 64, S.R, PROJW_RPI, MFMA, MFMA ? 0 : sizeof(T) == 4 ? 2 : 1>;
-    if (shm > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL(fn, dim3(c->ng, projw_split(c->ng)), dim3(S.nw * 64), shm, c->st, P);
+    if (pl.lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
+    hipLaunchKernelGGL(fn, dim3(c->ng, std::max(pl.shares, projw_split(c->ng))), dim3(S.nw * 64), pl.lds, c->st, P);
 }
 
 template <typename T, int FORMED>
 bool launch_projw(sqg_ctx *c, PArgs<T> &P)
 {
-    const ProjwUse pw = projw_use(c->dims(), sizeof(T));
-    if (!pw.on) return false;
-    P.sz = projw_sz(c->M, pw, sizeof(T));
-    const size_t shm = projw_head(c->M, c->gl_max) + (size_t)projw_pu(c->M, pw) * NG * sizeof(T) * P.sz;
-    if (shm > 160 * 1024) return false;
+    const ProjwPlan &pl = c->projw[sizeof(T) == 8];
+    if (pl.shape < 0) return false;
+    P.sz = pl.sz; P.pad = pl.pad;
     if constexpr (sizeof(T) == 8) {
-        if (pw.mfma) {
-            if (c->proj_shape == 0) projw_go<T, FORMED, true, 0>(c, shm, P);
-            else projw_go<T, FORMED, true, 1>(c, shm, P);
+        if (projw_use(c->dims(), 8).mfma) {
+            if (pl.shape == 0) projw_go<T, FORMED, true, 0>(c, pl, P);
+            else projw_go<T, FORMED, true, 1>(c, pl, P);
             return true;
         }
     }
-    if (pw.mfma) return false;
-    if (c->proj_shape == 0) projw_go<T, FORMED, false, 0>(c, shm, P);
-    else if (c->proj_shape == 1) projw_go<T, FORMED, false, 1>(c, shm, P);
-    else if (c->proj_shape == 2) projw_go<T, FORMED, false, 2>(c, shm, P);
-    else projw_go<T, FORMED, false, 3>(c, shm, P);
+    if (pl.shape == 0) projw_go<T, FORMED, false, 0>(c, pl, P);
+    else if (pl.shape == 1) projw_go<T, FORMED, false, 1>(c, pl, P);
+    else if (pl.shape == 2) projw_go<T, FORMED, false, 2>(c, pl, P);
+    else projw_go<T, FORMED, false, 3>(c, pl, P);
     return true;
 }
 
@@ -505,7 +492,7 @@ void launch_proj(sqg_ctx *c, int B, const PArgs<T> &A, int which = -1, double al
     if (c->n_ip > 0) {
         PArgs<T> P = A;
         const dim3 grid(c->ng);
-        if (c->proj_shape >= 0 && launch_projw<T, FORMED>(c, P)) goto apply;
+        if (launch_projw<T, FORMED>(c, P)) goto apply;
         const int mp = c->max_nproj <= 1 ? 1 : c->max_nproj <= 4 ? 4 : 0;
         if (mp && launch_projs<T, FORMED>(c, P, mp)) goto apply;
         if (c->max_nproj <= 1)

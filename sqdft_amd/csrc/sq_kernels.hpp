@@ -597,7 +597,7 @@ struct PArgs {
     const double *ca, *ib;        // LANCZOS: projects v = (V - ca V2) * ib
     const int *gst;               // [groups + 1] first slot of each group
     const int *glist, *glist_cnt; // group image lists
-    int sz;                       // k_projw: planes per slab
+    int sz, pad;                  // k_projw: planes per slab, padded LDS rows
 };
 
 // Projections s[b][ip] = <U_ip, v_b>/Denom over the intersection of the
@@ -852,7 +852,9 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
             if (FORMED) { cab[m] = (T)A.ca[b0 + m]; ibb[m] = (T)A.ib[b0 + m]; }
         }
     }
-    const int cnt = A.glist_cnt[q];
+    // this workgroup's share of the group's images, consecutive in z
+    const int gcnt = A.glist_cnt[q];
+    const int l0 = (int)(gcnt * blockIdx.y / gridDim.y), cnt = (int)(gcnt * (blockIdx.y + 1) / gridDim.y) - l0;
     if (nact == 0 || cnt == 0) return;
     // LDS: image data [cnt] | staged slab [SZ][union points][NM]
     __shared__ int sh_ncmax, sh_lo, sh_hi;
@@ -862,7 +864,7 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
     ImgMeta *im = reinterpret_cast<ImgMeta *>(smem_raw);
     T *pl = reinterpret_cast<T *>(smem_raw + ((size_t)cnt * sizeof(ImgMeta) + 15) / 16 * 16);
     for (int li = tid; li < cnt; li += blockDim.x) {
-        const int J = A.glist[(size_t)q * GLCAP + li];
+        const int J = A.glist[(size_t)q * GLCAP + l0 + li];
         const int t = A.img_type[J], nc = A.nlocc[t];
         ImgMeta e;
         e.ox = A.img_nn[3 * J] - nc; e.oy = A.img_nn[3 * J + 1] - nc; e.oz = A.img_nn[3 * J + 2] - nc;
@@ -1042,7 +1044,7 @@ __global__ void __launch_bounds__(NT) k_projs(PArgs<T> A)
 // A[b][i][k] at lane 16k + 4b + i, B[b][k][j] at 16k + 4b + j, D[b][i][j] at
 // 16i + 4b + j.
 //
-// LDS rows are padded to a pitch congruent to the box side modulo 32 values, so
+// LDS rows are padded (A.pad) to a pitch congruent to the box side modulo 32 values, so
 // that the box rows one wave reads fall on disjoint banks; with MFMA the member
 // stride is congruent to 8, so that the 8 members of a point do.  Bound by the
 // vectors' HBM reads and, since one workgroup fills a CU's LDS, by what its
@@ -1130,7 +1132,7 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
     for (int m = 0; m < NM; ++m)
         kof[m] = member_offset(m, pad, M, M2, M3, ux0 - ni[m] + nloc, uy0 - nj[m] + nloc, uz0 - nk[m] + nloc) * (int)TS;
     const int wbox = __builtin_amdgcn_readfirstlane(im[0].w);
-    const int upx = ux + (((wbox - ux) % 32) + 32) % 32, up = upx * uy;
+    const int upx = ux + (A.pad ? (((wbox - ux) % 32) + 32) % 32 : 0), up = upx * uy;
     const int ms = MFMA ? up + (((8 - up) % 32) + 32) % 32 : up;
     // MFMA lane roles: K index, block (member quad, point phase), row/column
     const int kk = lane >> 4, bb = (lane >> 2) & 3, ii = lane & 3;

@@ -90,10 +90,14 @@ inline int projw_slab(const ProjwUse &pw, int ux, int uy)
     return pw.mfma ? u + (((8 - u) % 32) + 32) % 32 : u;
 }
 
-// Slab capacity per plane and member: the union plane of a 4x2 block of cubes
-// or one cube.
-inline int projw_pu(int M, const ProjwUse &pw)
+// k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
+inline int projs_pu(int M) { return (M + 3) * (M + 3); }
+
+// k_projw's slab capacity per plane and member: the union plane of a 4x2 block of
+// cubes or one cube; without padded rows any union that make_groups forms.
+inline int projw_pu(int M, const ProjwUse &pw, bool pad = true)
 {
+    if (!pad) return projs_pu(M) + (pw.mfma ? 31 : 0);
     return std::max(projw_slab(pw, M + 3, M + 1), projw_slab(pw, M, M));
 }
 
@@ -122,9 +126,6 @@ inline int projw_sz(int M, const ProjwUse &pw, size_t ts)
     if (!pw.mfma) return ts == 4 ? 2 : 1;
     return std::max(1, std::min({8, lds, 3072 / ((M + 3) * (M + 1))}));
 }
-
-// k_projs' slab capacity: the union plane of a 4x4 footprint of cubes.
-inline int projs_pu(int M) { return (M + 3) * (M + 3); }
 
 // Cuts B slots into groups of up to NG consecutive ones whose cubes the
 // staged projection kernels can walk together: the union plane fits the slab
@@ -184,6 +185,48 @@ inline int projw_split(int ng)
         if (ti < t) { t = ti; best = 1 << i; }
     }
     return best;
+}
+
+// How k_projw walks a batch: compiled shape (-1: not at all), planes per slab,
+// workgroups that a group's images are shared out to at least, padded rows, LDS
+// bytes of one workgroup.
+struct ProjwPlan { int shape = -1, sz = 0, shares = 1, pad = 1; size_t lds = 0; };
+
+// need: register slots that any group's walk takes with PROJ_NW[0] and PROJ_NW[1]
+// waves; gl_max: images of the longest group list.  The image data must fit beside
+// the slab and the column table; where only the table is too much, the images are
+// shared out (a share holds its own images' data alone), or the rows go unpadded.
+// The sums are the same in every plan, so batches stay bitwise alike.
+inline ProjwPlan projw_plan(int M, const ProjwUse &pw, size_t ts, int sz, int gl_max, const int (&need)[2])
+{
+    ProjwPlan p;
+    if (!pw.on) return p;
+    const ProjShape *sh = pw.mfma ? PROJM_SHAPES : PROJR_SHAPES;
+    int shape = -1;
+    for (int i = 0; i < (pw.mfma ? 2 : 4) && shape < 0; ++i)
+        if (need[sh[i].nw == PROJ_NW[1]] <= sh[i].R) shape = i;
+    if (shape < 0) return p;
+    auto slab = [&](bool pad) { return (size_t)projw_pu(M, pw, pad) * NG * ts * sz; };
+    const bool room = images_lds(gl_max) + slab(true) <= LDS_MAX;   // but for the table
+    for (int pad : {1, 0})
+        for (int shares : {1, 2, 4}) {
+            const size_t lds = projw_head(M, (gl_max + shares - 1) / shares) + slab(pad);
+            if (room && lds <= LDS_MAX) return {shape, sz, shares, pad, lds};
+        }
+    return p;
+}
+
+// k_projs: planes per slab (at most `deep`) and workgroups that share a group's
+// images, as few as hold the image data beside the deepest slab; sz 0: does not fit.
+struct ProjsPlan { int sz, shares; size_t lds; };
+inline ProjsPlan projs_plan(int M, size_t ts, int deep, int gl_max)
+{
+    for (int shares : {1, 2, 4})
+        for (int sz : {deep, deep / 2, 1}) {
+            const size_t lds = images_lds((gl_max + shares - 1) / shares) + (size_t)projs_pu(M) * NG * ts * sz;
+            if (lds <= LDS_MAX) return {sz, shares, lds};
+        }
+    return {0, 0, 0};
 }
 
 // LDS bytes of one k_nlapplyg workgroup (loc table, NG values per row, union

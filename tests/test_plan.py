@@ -36,6 +36,23 @@ long node_bytes(int M, int n_ip, int rs, int nvec, int lists)
 {
     return (long)(batch_node_bytes({M, 1, n_ip, 9}, rs, nvec) + batch_list_bytes(lists));
 }
+int walk(int M, int max_nproj, int w, int ts, int gl_max, int need12, int need8, long *out)
+{
+    const ProjDims d{M, max_nproj, 100, w};
+    const ProjwUse pw = projw_use(d, ts);
+    const int need[2] = {need12, need8};
+    const ProjwPlan p = projw_plan(M, pw, ts, projw_sz(M, pw, ts), gl_max, need);
+    const long v[8] = {p.shape, p.sz, p.shares, p.pad, (long)p.lds, pw.on ? projw_pu(M, pw, p.pad) : 0,
+                       pw.on ? projw_pu(M, pw) : 0, pw.mfma};
+    std::memcpy(out, v, sizeof v);
+    return pw.on;
+}
+int staged(int M, int ts, int deep, int gl_max, long *out)
+{
+    const ProjsPlan p = projs_plan(M, ts, deep, gl_max);
+    out[0] = p.sz; out[1] = p.shares; out[2] = (long)p.lds;
+    return 0;
+}
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -148,3 +165,54 @@ def test_batches_budget_for_groups_of_one_node(plan, M, n_ip, rs):
     group = 4 * (1024 + 1 + 1)
     assert plan.node_bytes(M, n_ip, rs, 2, 0) >= held + group
     assert plan.node_bytes(M, n_ip, rs, 3, 1) >= held + M ** 3 * rs + group + 4 * (512 + 1)
+
+
+LDS = 160 * 1024
+IMG = 40          # bytes of an image's data in LDS
+WIDTHS = {1: (1, 3, 5, 7, 9, 11, 13), 3: (1, 3, 5, 7, 9, 11, 13, 15)}
+
+
+def up16(b):
+    return -(-b // 16) * 16
+
+
+@pytest.mark.parametrize("np_,ts", [(1, 8), (1, 4), (3, 8)])
+def test_walks_whose_slab_and_images_fit_find_room_for_the_columns(plan, np_, ts):
+    """k_projw takes every table whose padded slab (one FP64, two FP32 planes) fits
+    the LDS beside the longest list's data, with LDS for what its plan stages."""
+    out = (C.c_long * 8)()
+    for w in WIDTHS[np_]:
+        for M in range(max(w, 3), MAXM + 1, 2):
+            for gl in list(range(1, 620, 3)) + [700, 1024]:
+                assert plan.walk(M, np_, w, ts, gl, 1, 1, out)
+                shape, sz, shares, pad, lds, cap, cap_pad, mfma = out
+                fits = up16(gl * IMG) + cap_pad * 8 * ts * (sz if shape >= 0 else 2 if ts == 4 else 1) <= LDS
+                if mfma and shape < 0:
+                    continue
+                assert (shape >= 0) == fits, (w, M, gl)
+                if shape < 0:
+                    continue
+                columns = up16(4 * (M + 3) ** 2)
+                assert up16(-(-gl // shares) * IMG) + columns + cap * 8 * ts * sz <= lds <= LDS
+                if up16(gl * IMG) + columns + cap_pad * 8 * ts * sz <= LDS - 4 * 49:
+                    assert shares == 1 and pad == 1   # shared or unpadded only where it must
+                # every union that a group may have fits the capacity
+                for dx in range(0, 10):
+                    for dy in range(0, 10):
+                        ux, uy = M + dx, M + dy
+                        if ux * uy > (M + 3) ** 2:
+                            continue
+                        if not pad:
+                            u = ux * uy
+                            assert u + (8 - u) % 32 * mfma <= cap
+
+
+@pytest.mark.parametrize("ts,deep", [(8, 2), (4, 4)])
+def test_staged_projections_take_every_list(plan, ts, deep):
+    out = (C.c_long * 3)()
+    for M in range(3, MAXM + 1, 2):
+        for gl in range(1, 1025, 7):
+            plan.staged(M, ts, deep, gl, out)
+            sz, shares, lds = out
+            assert sz in (1, 2, 4) and sz <= deep
+            assert up16(-(-gl // shares) * IMG) + (M + 3) ** 2 * 8 * ts * sz <= lds <= LDS, (M, gl)
