@@ -360,26 +360,27 @@ int image_lists(sqg_ctx *c, int B, const std::vector<int> &gst, bool node_lists)
     const ProjDims dm = c->dims();
     size_t ts[2];
     const int nsh = stored_types(c, ts);
-    hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + 4, (size_t)2, 0);
+    constexpr int NEED = 4, NNEED = 2 * PR_DEPTHS;   // where their words start among the flags
+    hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(64), 0, c->st, c->flags.as<int>() + NEED, (size_t)NNEED, 0);
+    int first[2] = {0, 0};   // of each stored type's depths
     for (int i = 0; i < nsh; ++i) {
-        const ProjwUse pw = projw_use(dm, ts[i]);
-        if (!pw.on) continue;
-        L.pr_need = c->flags.as<int>() + 4;
-        L.pr_sz[L.pr_n++] = projw_sz(c->M, pw, ts[i]);
+        const ProjwDepths dep = projw_depths(c->M, projw_use(dm, ts[i]), ts[i]);
+        first[i] = L.pr_n;
+        for (int k = 0; k < dep.n; ++k) L.pr_sz[L.pr_n++] = dep.sz[k];
     }
+    L.pr_need = c->flags.as<int>() + NEED;
     hipLaunchKernelGGL(k_group_images, dim3(ng), dim3(64), 0, c->st, L);
     if (node_lists) hipLaunchKernelGGL(k_node_images, dim3(B), dim3(64), 0, c->st, L);
-    std::vector<int> gc(ng + 2);
+    std::vector<int> gc(ng + NNEED);
     HIPCHK(hipMemcpyAsync(gc.data(), c->glist_cnt.p, (size_t)ng * sizeof(int), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(gc.data() + ng, c->flags.as<int>() + 4, 2 * sizeof(int), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipMemcpyAsync(gc.data() + ng, c->flags.as<int>() + NEED, NNEED * sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->gl_max = 0;
     for (int i = 0; i < ng; ++i) c->gl_max = std::max(c->gl_max, gc[i]);
-    const int need[2] = {gc[ng], gc[ng + 1]};
-    for (int i = 0; i < nsh; ++i) {
-        const ProjwUse pw = projw_use(dm, ts[i]);
-        c->projw[ts[i] == 8] = projw_plan(c->M, pw, ts[i], projw_sz(c->M, pw, ts[i]), c->gl_max, need);
-    }
+    int need[PR_DEPTHS][2];
+    for (int i = 0; i < NNEED; ++i) need[i / 2][i % 2] = gc[ng + i];
+    for (int i = 0; i < nsh; ++i)
+        c->projw[ts[i] == 8] = projw_plan(c->M, projw_use(dm, ts[i]), ts[i], c->gl_max, need + first[i]);
     return SQG_OK;
 }
 

@@ -1633,12 +1633,11 @@ struct LArgs {
     int *list, *list_cnt, *overflow;   // [B][LCAP], [B] (k_node_images)
     const int *gst;               // [groups + 1] first slot of each group
     int *glist, *glist_cnt;       // [groups][GLCAP], [groups]
-    // register slots k_projw needs for any group of the batch (a
-    // maximum; 99 when the list mixes box sizes) with PROJ_NW[0] and
-    // PROJ_NW[1] waves walking slabs of pr_sz planes, for each of the pr_n
-    // slab depths in use
+    // register slots k_projw needs for any group of the batch (a maximum; 99 when
+    // the list mixes box sizes) walking slabs of pr_sz planes, for each of the pr_n
+    // depths in question: [depth][wave count of PROJ_NW]
     int *pr_need;
-    int pr_n, pr_sz[2];
+    int pr_n, pr_sz[PR_DEPTHS];
 };
 
 // Images that meet the cube of a node of the block (one wave: gn nodes at
@@ -1739,12 +1738,13 @@ __global__ void __launch_bounds__(64) k_group_images(LArgs A)
         if (bad) atomicOr(A.overflow, 1);
         A.glist_cnt[q] = cnt;
     }
-    if (!A.pr_need || cnt == 0) return;
+    if (A.pr_n == 0 || cnt == 0) return;
     __syncthreads();   // the sorted list is read back below
     const int nc0 = A.nlocc[A.img_type[id[0]]];
-    int need[2] = {1, 1};
+    int need = 1;
     for (int i = lane; i < cnt; i += 64)
-        if (A.nlocc[A.img_type[id[i]]] != nc0) need[0] = need[1] = 99;
+        if (A.nlocc[A.img_type[id[i]]] != nc0) need = 99;
+    need = __ballot(need == 99) ? 99 : 1;
     // the k-th image of a wave that meets the walk's union takes slot k mod R,
     // so R must exceed k - j for every earlier one j still alive in the slab
     // where k enters (a walk with fewer members clamps to a smaller z-range
@@ -1771,14 +1771,12 @@ __global__ void __launch_bounds__(64) k_group_images(LArgs A)
             if (nl == WN) { nd = 99; break; }
             kk[nl] = k; ee[nl] = E; ++nl;
         }
-        need[nv] = max(need[nv], nd);
+        need = max(need, nd);
     }
+    // the quarter's maximum
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) need[i] = max(need[i], __shfl_xor(need[i], o, 64));
-        if (lane == 0) atomicMax(A.pr_need + i, need[i]);
-    }
+    for (int o = 8; o >= 1; o >>= 1) need = max(need, __shfl_xor(need, o, 64));
+    if (v < A.pr_n && wv == 0) atomicMax(A.pr_need + 2 * v + nv, need);
 }
 
 // ---------------------------------------------------------------- fills

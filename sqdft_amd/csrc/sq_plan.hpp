@@ -64,6 +64,7 @@ struct ProjShape { int nw, R; };
 constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
 constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // MFMA: two doubles per slot and lane
 constexpr int PROJ_NW[2] = {12, 8};
+constexpr int PR_DEPTHS = 2;    // slab depths in question on one batch at most
 
 // How k_projw runs on vectors of ts bytes per value: on = 0 when it does not
 // apply; the matrix cores for FP64 tables of several projectors.
@@ -113,18 +114,25 @@ inline size_t columns_lds(int M)
 // LDS bytes of k_projw beside the slab: image data and union columns.
 inline size_t projw_head(int M, int images) { return images_lds(images) + columns_lds(M); }
 
-// Planes per slab.  VALU: one FP64 or two FP32 planes (a deeper slab keeps more
-// images alive than the slots of twelve waves: 17^3 cubes with three planes
-// took 269 us a pass with ten slots in eight waves against 81).  MFMA, whose
-// slots are small: about four load rounds of a workgroup between two barriers,
-// at most eight planes, as far as the LDS holds them beside a list of 256
-// images (25^3 cubes, two planes: 373 against 496 us a pass).
-inline int projw_sz(int M, const ProjwUse &pw, size_t ts)
+// Depths (planes per slab) that k_projw may walk in, the preferred one first.
+// VALU: one FP64 or two FP32 planes (a deeper slab keeps more images alive than the
+// slots of twelve waves: 17^3 cubes with three planes took 269 us a pass with ten
+// slots in eight waves against 81).  MFMA, whose slots are small: about four load
+// rounds of a workgroup between two barriers, at most eight planes, as far as the
+// LDS holds them beside a list of 256 images (25^3 cubes, two planes: 373 against
+// 496 us a pass); or one plane, which never keeps more images alive than several do,
+// where a deep slab takes more slots than there are (4,096 nodes with 21^3 cubes and
+// 418 images a group: 537 us a pass, 675 in k_projs).  A list too long for the deep
+// slab alone is shared out instead (29^3 cubes, 402 images: 752 against 855 us).
+struct ProjwDepths { int n, sz[PR_DEPTHS]; };
+inline ProjwDepths projw_depths(int M, const ProjwUse &pw, size_t ts)
 {
+    if (!pw.on) return {0, {0, 0}};
+    if (!pw.mfma) return {1, {ts == 4 ? 2 : 1, 0}};
     const size_t plane = (size_t)projw_pu(M, pw) * NG * ts, head = projw_head(M, 256);
     const int lds = plane + head <= LDS_MAX ? (int)((LDS_MAX - head) / plane) : 1;
-    if (!pw.mfma) return ts == 4 ? 2 : 1;
-    return std::max(1, std::min({8, lds, 3072 / ((M + 3) * (M + 1))}));
+    const int deep = std::max(1, std::min({8, lds, 3072 / ((M + 3) * (M + 1))}));
+    return {deep > 1 ? 2 : 1, {deep, 1}};
 }
 
 // Cuts B slots into groups of up to NG consecutive ones whose cubes the
@@ -192,28 +200,31 @@ inline int projw_split(int ng)
 // bytes of one workgroup.
 struct ProjwPlan { int shape = -1, sz = 0, shares = 1, pad = 1; size_t lds = 0; };
 
-// need: register slots that any group's walk takes with PROJ_NW[0] and PROJ_NW[1]
-// waves; gl_max: images of the longest group list.  The image data must fit beside
-// the slab and the column table; where only the table is too much, the images are
-// shared out (a share holds its own images' data alone), or the rows go unpadded.
-// The sums are the same in every plan, so batches stay bitwise alike.
-inline ProjwPlan projw_plan(int M, const ProjwUse &pw, size_t ts, int sz, int gl_max, const int (&need)[2])
+// need[k]: register slots that any group's walk in the k-th depth takes with
+// PROJ_NW[0] and PROJ_NW[1] waves; gl_max: images of the longest group list.  The
+// image data must fit beside the slab and the column table; where only the table is
+// too much, the images are shared out (a share holds its own images' data alone), or
+// the rows go unpadded.  The sums are the same in every plan, so batches stay
+// bitwise alike.
+inline ProjwPlan projw_plan(int M, const ProjwUse &pw, size_t ts, int gl_max, const int (*need)[2])
 {
-    ProjwPlan p;
-    if (!pw.on) return p;
+    const ProjwDepths dep = projw_depths(M, pw, ts);
     const ProjShape *sh = pw.mfma ? PROJM_SHAPES : PROJR_SHAPES;
-    int shape = -1;
-    for (int i = 0; i < (pw.mfma ? 2 : 4) && shape < 0; ++i)
-        if (need[sh[i].nw == PROJ_NW[1]] <= sh[i].R) shape = i;
-    if (shape < 0) return p;
-    auto slab = [&](bool pad) { return (size_t)projw_pu(M, pw, pad) * NG * ts * sz; };
-    const bool room = images_lds(gl_max) + slab(true) <= LDS_MAX;   // but for the table
-    for (int pad : {1, 0})
-        for (int shares : {1, 2, 4}) {
-            const size_t lds = projw_head(M, (gl_max + shares - 1) / shares) + slab(pad);
-            if (room && lds <= LDS_MAX) return {shape, sz, shares, pad, lds};
-        }
-    return p;
+    int shape[PR_DEPTHS] = {-1, -1};
+    for (int k = 0; k < dep.n; ++k)
+        for (int i = 0; i < (pw.mfma ? 2 : 4) && shape[k] < 0; ++i)
+            if (need[k][sh[i].nw == PROJ_NW[1]] <= sh[i].R) shape[k] = i;
+    auto slab = [&](int sz, bool pad) { return (size_t)projw_pu(M, pw, pad) * NG * ts * sz; };
+    for (int k = 0; k < dep.n; ++k) {
+        const bool room = images_lds(gl_max) + slab(dep.sz[k], true) <= LDS_MAX;   // but for the table
+        if (shape[k] < 0 || !room) continue;
+        for (int pad : {1, 0})
+            for (int shares : {1, 2, 4}) {
+                const size_t lds = projw_head(M, (gl_max + shares - 1) / shares) + slab(dep.sz[k], pad);
+                if (lds <= LDS_MAX) return {shape[k], dep.sz[k], shares, pad, lds};
+            }
+    }
+    return {};
 }
 
 // k_projs: planes per slab (at most `deep`) and workgroups that share a group's

@@ -36,14 +36,14 @@ long node_bytes(int M, int n_ip, int rs, int nvec, int lists)
 {
     return (long)(batch_node_bytes({M, 1, n_ip, 9}, rs, nvec) + batch_list_bytes(lists));
 }
-int walk(int M, int max_nproj, int w, int ts, int gl_max, int need12, int need8, long *out)
+int walk(int M, int max_nproj, int w, int ts, int gl_max, int deep12, int deep8, int one12, int one8, long *out)
 {
     const ProjDims d{M, max_nproj, 100, w};
     const ProjwUse pw = projw_use(d, ts);
-    const int need[2] = {need12, need8};
-    const ProjwPlan p = projw_plan(M, pw, ts, projw_sz(M, pw, ts), gl_max, need);
-    const long v[8] = {p.shape, p.sz, p.shares, p.pad, (long)p.lds, pw.on ? projw_pu(M, pw, p.pad) : 0,
-                       pw.on ? projw_pu(M, pw) : 0, pw.mfma};
+    const int need[2][2] = {{deep12, deep8}, {one12, one8}};
+    const ProjwPlan p = projw_plan(M, pw, ts, gl_max, need);
+    const long v[9] = {p.shape, p.sz, p.shares, p.pad, (long)p.lds, pw.on ? projw_pu(M, pw, p.pad) : 0,
+                       pw.on ? projw_pu(M, pw) : 0, pw.mfma, projw_depths(M, pw, ts).sz[0]};
     std::memcpy(out, v, sizeof v);
     return pw.on;
 }
@@ -180,18 +180,17 @@ def up16(b):
 def test_walks_whose_slab_and_images_fit_find_room_for_the_columns(plan, np_, ts):
     """k_projw takes every table whose padded slab (one FP64, two FP32 planes) fits
     the LDS beside the longest list's data, with LDS for what its plan stages."""
-    out = (C.c_long * 8)()
+    out = (C.c_long * 9)()
     for w in WIDTHS[np_]:
         for M in range(max(w, 3), MAXM + 1, 2):
             for gl in list(range(1, 620, 3)) + [700, 1024]:
-                assert plan.walk(M, np_, w, ts, gl, 1, 1, out)
-                shape, sz, shares, pad, lds, cap, cap_pad, mfma = out
-                fits = up16(gl * IMG) + cap_pad * 8 * ts * (sz if shape >= 0 else 2 if ts == 4 else 1) <= LDS
-                if mfma and shape < 0:
-                    continue
-                assert (shape >= 0) == fits, (w, M, gl)
+                assert plan.walk(M, np_, w, ts, gl, 1, 1, 1, 1, out)
+                shape, sz, shares, pad, lds, cap, cap_pad, mfma, deep = out
+                # the shallowest slab that may be walked
+                assert (shape >= 0) == (up16(gl * IMG) + cap_pad * 8 * ts * (1 if mfma else deep) <= LDS), (w, M, gl)
                 if shape < 0:
                     continue
+                assert sz == deep or up16(gl * IMG) + cap_pad * 8 * ts * deep > LDS
                 columns = up16(4 * (M + 3) ** 2)
                 assert up16(-(-gl // shares) * IMG) + columns + cap * 8 * ts * sz <= lds <= LDS
                 if up16(gl * IMG) + columns + cap_pad * 8 * ts * sz <= LDS - 4 * 49:
@@ -216,3 +215,16 @@ def test_staged_projections_take_every_list(plan, ts, deep):
             sz, shares, lds = out
             assert sz in (1, 2, 4) and sz <= deep
             assert up16(-(-gl // shares) * IMG) + (M + 3) ** 2 * 8 * ts * sz <= lds <= LDS, (M, gl)
+
+
+def test_a_deep_slab_short_of_slots_gives_way_to_one_plane(plan):
+    """Matrix-core walks: slots are planned for the deep slab and for one plane."""
+    out = (C.c_long * 9)()
+    for M, w in ((7, 5), (17, 9), (21, 7), (25, 9)):
+        plan.walk(M, 3, w, 8, 200, 12, 18, 12, 18, out)
+        deep = out[8]
+        assert deep > 1 and (out[0], out[1]) == (0, deep)
+        plan.walk(M, 3, w, 8, 200, 13, 19, 12, 18, out)
+        assert (out[0], out[1]) == (0, 1)
+        plan.walk(M, 3, w, 8, 200, 99, 99, 99, 99, out)
+        assert out[0] == -1
