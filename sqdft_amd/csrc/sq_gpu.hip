@@ -397,20 +397,21 @@ int node_images(sqg_ctx *c, const int *nodes, int B, bool node_lists = false)
 template <typename T, int K>
 void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
 {
-    const size_t shg = nlapplyg_lds(c->dims(), c->gl_max);
-    if (shg <= 160 * 1024) {
+    const NlapplyPlan pl = nlapply_plan(c->dims(), c->gl_max);
+    if (pl.fits) {
         NGArgs<T> N{};
         N.g = A.g; N.nl = A.nl; N.nlv = A.nlv;
         N.gst = c->gst.as<int>(); N.glist = c->glist.as<int>(); N.glist_cnt = c->glist_cnt.as<int>();
         N.img_type = c->img_type.as<int>(); N.nproj = c->nproj.as<int>(); N.ip_base = c->ip_base.as<int>();
         N.mp = std::max(c->max_nproj, 1);
-        auto fn = N.nl.ip16 ? k_nlapplyg<T, true> : k_nlapplyg<T, false>;
-        if (shg > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shg);
+        auto fn = pl.columns ? (N.nl.ip16 ? k_nlapplyg<T, true, true> : k_nlapplyg<T, false, true>)
+                             : (N.nl.ip16 ? k_nlapplyg<T, true, false> : k_nlapplyg<T, false, false>);
+        if (pl.lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
         // three workgroups share a CU: about eight rounds of them, so that the
         // last one costs little, with at least four points a thread each
         const int pts = (c->M + 3) * (c->M + 1) * c->M;
         const int split = std::max(1, std::min(6144 / std::max(c->ng, 1), pts / (4 * 512)));
-        hipLaunchKernelGGL(fn, dim3(c->ng, split), dim3(512), shg, c->st, N);
+        hipLaunchKernelGGL(fn, dim3(c->ng, split), dim3(512), pl.lds, c->st, N);
         return;
     }
     const size_t shm = (size_t)std::max(c->n_ip, 1) * sizeof(double);

@@ -1365,8 +1365,10 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
 // a CU (four at a time: 892 against 867 us; the next point's entries fetched
 // early as well: 128 VGPRs, spills, 1147 us).  Where a point sits and which
 // members hold it comes from a table of the union's columns, its place in a
-// member's cube is a scalar offset.  Several workgroups share a group, each with
-// a run of planes (shares that alternate point by point split cache lines:
+// member's cube is a scalar offset.  COLS = false, where the table does not fit the
+// LDS beside the rows: worked out per point (512 nodes with 43^3 cubes and 520 images
+// of three projectors a group: 446 us, 604 in k_nlapply).  Several workgroups share a group,
+// each with a run of planes (shares that alternate point by point split cache lines:
 // 879 us).  Before these changes against now, us a pass: 8,192 nodes with FP64
 // 35^3 cubes 888 and 732 (2.8 GB: 3.8 TB/s), 4,096 with FP32 ones 285 and 213,
 // 1,000 with FP64 17^3 cubes 34 and 24; 4,096 with 31^3 LiH ones (eight entries
@@ -1382,7 +1384,7 @@ struct NGArgs {
     int mp;                       // projectors of an image at most: rows per image
 };
 
-template <typename T, bool IP16>
+template <typename T, bool IP16, bool COLS>
 __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
 {
     constexpr unsigned TS = sizeof(T);
@@ -1427,7 +1429,7 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     if (cnt == 0 && threadIdx.x < SLW) sl[threadIdx.x] = 0.0;
     // union column -> x, y (12 bits each) and the members whose cube holds it
     const int ux = ex1 - ex0 + 1, uy = ey1 - ey0 + 1, uz = ez1 - ez0 + 1, np_ = ux * uy;
-    for (int p = threadIdx.x; p < np_; p += blockDim.x) {
+    auto column = [&](int p) {
         const int yy = p / ux, xx = p - yy * ux;
         unsigned v = (unsigned)xx | (unsigned)yy << 12;
 #pragma unroll
@@ -1435,8 +1437,10 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
             if (((onmask >> m) & 1u) && (unsigned)(ex0 + xx - ni[m]) < (unsigned)M &&
                 (unsigned)(ey0 + yy - nj[m]) < (unsigned)M)
                 v |= 1u << (24 + m);
-        xyt[p] = v;
-    }
+        return v;
+    };
+    if constexpr (COLS)
+        for (int p = threadIdx.x; p < np_; p += blockDim.x) xyt[p] = column(p);
     __syncthreads();
     const int E3 = (int)A.nl.E3;
     const int KA = A.nl.k_alloc;
@@ -1469,7 +1473,7 @@ __global__ void __launch_bounds__(512, 4) k_nlapplyg(NGArgs<T> A)
     };
     auto load = [&](Pt &P) {
         const bool on = P.z < zb;
-        P.cv = on ? xyt[P.p] : 0u;
+        P.cv = !on ? 0u : COLS ? xyt[P.p] : column(P.p);
         P.g = ((ez0 + P.z) * E + ey0 + (int)((P.cv >> 12) & 4095)) * E + ex0 + (int)(P.cv & 4095);
         P.cn = bload_u8(rEC, on ? (unsigned)P.g : OOB);
         entries(P.g, 0, on, P.u, P.ip);

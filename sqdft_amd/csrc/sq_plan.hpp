@@ -240,13 +240,16 @@ inline ProjsPlan projs_plan(int M, size_t ts, int deep, int gl_max)
     return {0, 0, 0};
 }
 
-// LDS bytes of one k_nlapplyg workgroup (loc table, NG values per row, union
-// columns)
-inline size_t nlapplyg_lds(const ProjDims &d, int gl_max)
+// LDS bytes of one k_nlapplyg workgroup: loc table, NG values per row and, where
+// they fit as well, the union columns (else worked out point by point).
+struct NlapplyPlan { bool fits, columns; size_t lds; };
+inline NlapplyPlan nlapply_plan(const ProjDims &d, int gl_max)
 {
-    const size_t head = ((size_t)std::max(d.n_ip, 1) * 4 + 15) / 16 * 16;
-    return head + (size_t)std::max(gl_max * d.max_nproj, 1) * SLW * sizeof(double) +
-           std::max((size_t)(d.M + 3) * (d.M + 3), (size_t)(d.M + 7) * d.M) * 4;
+    const size_t base = ((size_t)std::max(d.n_ip, 1) * 4 + 15) / 16 * 16 +
+                        (size_t)std::max(gl_max * d.max_nproj, 1) * SLW * sizeof(double);
+    const size_t all = base + std::max((size_t)(d.M + 3) * (d.M + 3), (size_t)(d.M + 7) * d.M) * 4;
+    if (all <= LDS_MAX) return {true, true, all};
+    return {base <= LDS_MAX, false, base};
 }
 
 // Device bytes that a batch holds per node: nvec + 3 vectors of rs bytes per value

@@ -116,3 +116,15 @@ def test_dense_tables_of_several_projectors(n, h, nloc, natom):
     assert list_length(S, nodes) == {14: 402, 3: 151, 10: 418}[nloc]
     print("dense", S.info["nloc"], flush=True)
     check(S, Rcut, T, nodes, precs=("fp64", "mixed_lanczos"), moments=True)
+
+
+def test_nonlocal_apply_without_the_column_table():
+    """43^3 cubes of a dense p-channel table: the nonlocal apply's rows fill the LDS."""
+    S, Rcut, T = system("li", 40, 1.2, 21, scattered(250, 7))
+    nodes = block(40, 0, 3, 10)
+    gl = list_length(S, nodes)
+    rows = 4 * 3 * S.images()["type"].size + gl * 3 * 80
+    print("columns", gl, rows, flush=True)
+    assert rows <= 160 * 1024 < rows + 4 * 46 ** 2
+    assert max(list_length(S, nodes[i:i + 1]) for i in range(8)) <= 512
+    check(S, Rcut, T, nodes, precs=("fp64", "mixed"), moments=False)

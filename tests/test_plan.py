@@ -53,6 +53,12 @@ int staged(int M, int ts, int deep, int gl_max, long *out)
     out[0] = p.sz; out[1] = p.shares; out[2] = (long)p.lds;
     return 0;
 }
+int nlapply(int M, int max_nproj, int n_ip, int gl_max, long *out)
+{
+    const NlapplyPlan p = nlapply_plan({M, max_nproj, n_ip, 9}, gl_max);
+    out[0] = p.fits; out[1] = p.columns; out[2] = (long)p.lds;
+    return 0;
+}
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -228,3 +234,20 @@ def test_a_deep_slab_short_of_slots_gives_way_to_one_plane(plan):
         assert (out[0], out[1]) == (0, 1)
         plan.walk(M, 3, w, 8, 200, 99, 99, 99, 99, out)
         assert out[0] == -1
+
+
+@pytest.mark.parametrize("np_", [1, 3, 4, 9])
+def test_nonlocal_rows_need_no_room_for_the_columns(plan, np_):
+    """k_nlapplyg takes every batch whose loc table and rows fit the LDS, and keeps
+    the column table where that fits too."""
+    out = (C.c_long * 3)()
+    for M in (7, 17, 25, 31, 35, 43):
+        for gl in range(1, 1025, 9):
+            for n_ip in (1, 900, 3000, 8000, 20000, 40000):
+                rows = up16(4 * n_ip) + gl * np_ * 80
+                cols = 4 * (M + 3) ** 2
+                plan.nlapply(M, np_, n_ip, gl, out)
+                assert bool(out[0]) == (rows <= LDS)
+                if out[0]:
+                    assert rows + cols * out[1] <= out[2] <= LDS
+                    assert out[1] or rows + cols + 4 * 49 > LDS
