@@ -454,7 +454,7 @@ bool launch_projs(sqg_ctx *c, PArgs<T> &P, int mp)
 template <typename T, int FORMED, bool MFMA, int I>
 void projw_go(sqg_ctx *c, const ProjwPlan &pl, const PArgs<T> &P)
 {
-    constexpr ProjShape S = MFMA ? PROJM_SHAPES[MFMA ? I : 0] : PROJR_SHAPES[I];
+    constexpr ProjShape S = MFMA ? PROJM_SHAPES[0] : PROJR_SHAPES[I];
     auto fn = k_projw<T, FORMED, S.nw * 64, S.R, PROJW_RPI, MFMA, MFMA ? 0 : sizeof(T) == 4 ? 2 : 1>;
     if (pl.lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
     hipLaunchKernelGGL(fn, dim3(c->ng, std::max(pl.shares, projw_split(c->ng))), dim3(S.nw * 64), pl.lds, c->st, P);
@@ -468,15 +468,13 @@ bool launch_projw(sqg_ctx *c, PArgs<T> &P)
     P.sz = pl.sz; P.pad = pl.pad;
     if constexpr (sizeof(T) == 8) {
         if (projw_use(c->dims(), 8).mfma) {
-            if (pl.shape == 0) projw_go<T, FORMED, true, 0>(c, pl, P);
-            else projw_go<T, FORMED, true, 1>(c, pl, P);
+            projw_go<T, FORMED, true, 0>(c, pl, P);
             return true;
         }
     }
     if (pl.shape == 0) projw_go<T, FORMED, false, 0>(c, pl, P);
     else if (pl.shape == 1) projw_go<T, FORMED, false, 1>(c, pl, P);
-    else if (pl.shape == 2) projw_go<T, FORMED, false, 2>(c, pl, P);
-    else projw_go<T, FORMED, false, 3>(c, pl, P);
+    else projw_go<T, FORMED, false, 2>(c, pl, P);
     return true;
 }
 

@@ -59,10 +59,13 @@ constexpr int member_offset(int m, int pad, int M, int M2, int M3, int dx, int d
 // with FP32 ones 468 and 402 against 542 and 488; MFMA, 4,096 nodes with 31^3
 // cubes, 875 and 862 against 1142 and 1166.  With the union columns worked out
 // once per walk the twelve-wave ones take 1192, 863, 459, 358, 838 and 760.
+// Eight waves help only with more slots in all: a walk that R slots in twelve waves
+// do not hold has 12 R + 1 consecutive images alive, so one of eight waves needs
+// 3 R / 2 + 1 slots at least.
 constexpr int PROJW_RPI = 3;
 struct ProjShape { int nw, R; };
-constexpr ProjShape PROJR_SHAPES[4] = {{12, 4}, {8, 5}, {8, 10}, {8, 16}};
-constexpr ProjShape PROJM_SHAPES[2] = {{12, 12}, {8, 16}};   // MFMA: two doubles per slot and lane
+constexpr ProjShape PROJR_SHAPES[3] = {{12, 4}, {8, 10}, {8, 16}};
+constexpr ProjShape PROJM_SHAPES[1] = {{12, 12}};   // MFMA: two doubles per slot and lane
 constexpr int PROJ_NW[2] = {12, 8};
 constexpr int PR_DEPTHS = 2;    // slab depths in question on one batch at most
 
@@ -210,9 +213,10 @@ inline ProjwPlan projw_plan(int M, const ProjwUse &pw, size_t ts, int gl_max, co
 {
     const ProjwDepths dep = projw_depths(M, pw, ts);
     const ProjShape *sh = pw.mfma ? PROJM_SHAPES : PROJR_SHAPES;
+    const int nsh = pw.mfma ? 1 : 3;
     int shape[PR_DEPTHS] = {-1, -1};
     for (int k = 0; k < dep.n; ++k)
-        for (int i = 0; i < (pw.mfma ? 2 : 4) && shape[k] < 0; ++i)
+        for (int i = 0; i < nsh && shape[k] < 0; ++i)
             if (need[k][sh[i].nw == PROJ_NW[1]] <= sh[i].R) shape[k] = i;
     auto slab = [&](int sz, bool pad) { return (size_t)projw_pu(M, pw, pad) * NG * ts * sz; };
     for (int k = 0; k < dep.n; ++k) {

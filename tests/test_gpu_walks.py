@@ -50,6 +50,19 @@ def list_length(S, nodes):
     return int(np.sum(hit & has))
 
 
+def slots(S, nodes, planes, waves):
+    """Register slots a walk of the nodes' images takes: image li of the z-sorted list
+    is wave li mod waves', and holds a slot from the slab where it enters the union of
+    the cubes to the one where it leaves."""
+    n, im, nloc = S.n, S.images(), S.info["nloc"]
+    c = S.type_info(0)["nlocc"]
+    r = np.array([[nd % n, (nd // n) % n, nd // (n * n)] for nd in nodes])
+    lo, hi = r.min(axis=0) - nloc, r.max(axis=0) + nloc
+    z = np.sort(im["nn"][np.all((im["nn"] + c >= lo) & (im["nn"] - c <= hi), axis=1), 2])
+    enter, leave = np.maximum(z - c, lo[2]) // planes, np.minimum(z + c, hi[2]) // planes
+    return max(int(np.sum(leave[w:i:waves] >= enter[i])) + 1 for i in range(z.size) for w in [i % waves])
+
+
 def block(n, x, y, z, dx=4, dy=2):
     return np.array([(z * n + y + j) * n + x + i for j in range(dy) for i in range(dx)], dtype=np.int32)
 
@@ -128,3 +141,16 @@ def test_nonlocal_apply_without_the_column_table():
     assert rows <= 160 * 1024 < rows + 4 * 46 ** 2
     assert max(list_length(S, nodes[i:i + 1]) for i in range(8)) <= 512
     check(S, Rcut, T, nodes, precs=("fp64", "mixed"), moments=False)
+
+
+@pytest.mark.parametrize("n,h,nloc,natom,waves,need", [(16, 0.8, 8, 20, 12, range(1, 5)), (12, 1.2, 7, 20, 8, range(6, 11)),
+                                                       (12, 1.2, 7, 40, 8, range(11, 17))])
+def test_every_compiled_slot_count(n, h, nloc, natom, waves, need):
+    """s-channel walks of twelve waves with 4 slots and of eight with 10 and 16, for
+    slabs of one FP64 and two FP32 planes."""
+    S, Rcut, T = system("al", n, h, nloc, scattered(natom, 5))
+    nodes = block(n, 4, 4, 4)
+    assert all(slots(S, nodes, planes, waves) in need for planes in (1, 2))
+    assert waves == 12 or slots(S, nodes, 1, 12) > 4
+    print("slots", slots(S, nodes, 1, waves), slots(S, nodes, 2, waves), flush=True)
+    check(S, Rcut, T, nodes, precs=("fp64", "mixed", "mixed_lanczos"))
