@@ -78,9 +78,8 @@ int adjoint_batch(sqg_ctx *c, int z0, int nz, const AdjPlan &P)
     const int cidx = (c->p.nloc * c->M + c->p.nloc) * c->M + c->p.nloc;
     int st = ensure_batch(c, B);
     if (st) return st;
-    std::vector<int> nodes(B), slot_of(B);
-    for (int i = 0; i < B; ++i) nodes[i] = z0 * n * n + i;
-    NodeOrder(n).sort(nodes);   // brick order: full projection groups
+    const std::vector<int> nodes = NodeOrder(n).planes(z0, nz);   // brick order: full projection groups
+    std::vector<int> slot_of(B);
     for (int i = 0; i < B; ++i) slot_of[nodes[i] - z0 * n * n] = i;
     HIPCHK(c->adj_slot.ensure((size_t)B * sizeof(int)));
     HIPCHK(hipMemcpyAsync(c->adj_slot.p, slot_of.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->st));

@@ -169,52 +169,6 @@ Geo make_geo(const sqg_ctx *c, const int *dnodes, const int *ddone)
 // half of the cube's rows (two workgroups per node cube).
 int zmarch_threads(int M) { return (zhalf_rows(M, 0) * M + 63) / 64 * 64; }
 
-// Visiting order of the FD nodes: bricks of up to 4x4x2 nodes, so that
-// workgroups that run at the same time (consecutive batch slots) march
-// overlapping cubes and share Veff, projector tables and ELL entries in the
-// caches.  Each axis is cut into near-equal runs (of up to 4, 2 and 2 nodes in
-// x, y and z; a brick is two y runs), so a grid side that 4 does not divide
-// has no thin last brick.  The nodes of one (x run, y run, z) are consecutive:
-// the up to 4x2x1 block that one projection workgroup takes.
-struct NodeOrder {
-    int n;
-    std::vector<int> rx, ry, rz;   // run of each coordinate
-    explicit NodeOrder(int n_) : n(n_), rx(runs(n_, 4)), ry(runs(n_, 2)), rz(runs(n_, 2)) {}
-    static std::vector<int> runs(int n, int len)
-    {
-        const int m = (n + len - 1) / len;
-        std::vector<int> r(n);
-        for (int c = 0; c < m; ++c)
-            for (int i = (int)((long)c * n / m); i < (int)((long)(c + 1) * n / m); ++i) r[i] = c;
-        return r;
-    }
-    // sort key: brick z, y, x; then z, the brick's y run, y, x
-    unsigned long key(int node) const
-    {
-        const int x = node % n, y = (node / n) % n, z = node / (n * n);
-        const unsigned long m = (unsigned long)n + 1;
-        unsigned long k = rz[z];
-        for (unsigned long f : {(unsigned long)(ry[y] / 2), (unsigned long)rx[x], (unsigned long)z}) k = k * m + f;
-        return (k * 2 + (ry[y] & 1)) * (m * m) + (unsigned long)y * m + x;
-    }
-    void sort(std::vector<int> &nodes) const
-    {
-        std::vector<std::pair<unsigned long, int>> k(nodes.size());
-        for (size_t i = 0; i < nodes.size(); ++i) k[i] = {key(nodes[i]), nodes[i]};
-        if (std::is_sorted(k.begin(), k.end())) return;
-        std::sort(k.begin(), k.end());
-        for (size_t i = 0; i < nodes.size(); ++i) nodes[i] = k[i].second;
-    }
-};
-
-std::vector<int> node_order(int n)
-{
-    std::vector<int> seq((size_t)n * n * n);
-    for (size_t i = 0; i < seq.size(); ++i) seq[i] = (int)i;
-    NodeOrder(n).sort(seq);
-    return seq;
-}
-
 // Allocates per-batch buffers for up to B nodes.
 int ensure_batch(sqg_ctx *c, int B)
 {
@@ -828,12 +782,9 @@ int moments_for_nodes(sqg_ctx *c, const int *nodes, int count, long *passes, int
     return SQG_OK;
 }
 
-int moments_dispatch(sqg_ctx *c, const int *list, int count, long *passes, int cap = 0, bool lanczos = true)
+// nodes: in the order of NodeOrder (results are kept by node).
+int moments_dispatch(sqg_ctx *c, const int *nodes, int count, long *passes, int cap = 0, bool lanczos = true)
 {
-    // results are kept by node, so the list is visited in brick order
-    std::vector<int> order(list, list + count);
-    NodeOrder(c->p.n).sort(order);
-    const int *nodes = order.data();
     if (cap <= 0) cap = choose_batch(c, count);
     if (c->p.precision == SQG_MIXED) return moments_for_nodes<float, float>(c, nodes, count, passes, cap, lanczos);
     if (c->split()) return moments_for_nodes<float, double>(c, nodes, count, passes, cap, lanczos);
@@ -1265,7 +1216,9 @@ int sqg_node_moments(sqg_ctx *c, const double *veff, const int *nodes, int nb, d
     c->have_state = false;
     timing_reset(c);
     long passes = 0;
-    st = moments_dispatch(c, nodes, nb, &passes);
+    std::vector<int> order(nodes, nodes + nb);
+    NodeOrder(c->p.n).sort(order);
+    st = moments_dispatch(c, order.data(), nb, &passes);
     if (st) return st;
     timing_sum(c);
     if (nb == 0) return SQG_OK;
@@ -1309,7 +1262,7 @@ int sqg_density(sqg_ctx *c, const double *veff, int scf_iter, double ncharge, do
     timing_reset(c);
     HIPCHK(hipEventRecord(t0, c->st));
     const int cap = choose_batch(c, c->nn);
-    const std::vector<int> all = node_order(c->p.n);
+    const std::vector<int> all = NodeOrder(c->p.n).planes(0, c->p.n);
     long passes = 0;
     st = moments_dispatch(c, all.data(), c->nn, &passes, cap);
     if (st) return st;
@@ -1547,7 +1500,7 @@ int sqg_forces_nonlocal(sqg_ctx *c, double *f)
     if (c->n_ip == 0) return SQG_OK;
     std::vector<double> rec;   // node, atom, fx, fy, fz per contributing image
     const int cap = choose_batch(c, c->nn, 3, true);
-    const std::vector<int> nodes = node_order(c->p.n);
+    const std::vector<int> nodes = NodeOrder(c->p.n).planes(0, c->p.n);
     int done_n = 0;
     while (done_n < c->nn) {
         const int B = std::min(cap, c->nn - done_n);
@@ -1616,7 +1569,7 @@ int sqg_density_fixed(sqg_ctx *c, const double *veff, double ncharge, double lf_
     if (st) return st;
     c->have_state = false;
     const int cap = choose_batch(c, c->nn);
-    const std::vector<int> all = node_order(c->p.n);
+    const std::vector<int> all = NodeOrder(c->p.n).planes(0, c->p.n);
     long passes = 0;
     timing_reset(c);
     st = moments_dispatch(c, all.data(), c->nn, &passes, cap, false);
@@ -1694,7 +1647,7 @@ int sqg_tangent_veff(sqg_ctx *c, const double *dV, int fixed_n, double *drho)
     const int cap = std::min(choose_batch_adj(c, nn, 6 * (size_t)c->M3 * c->real_size() +
                                                      (size_t)(c->p.npl / 2 + 1) * 3 * sizeof(double)),
                              65535);
-    const std::vector<int> all = node_order(c->p.n);
+    const std::vector<int> all = NodeOrder(c->p.n).planes(0, c->p.n);
     for (int s0 = 0; s0 < nn; s0 += cap) {
         const std::vector<int> nodes(all.begin() + s0, all.begin() + std::min(s0 + cap, nn));
         st = c->p.precision == SQG_MIXED ? tangent_batch<float>(c, nodes) : tangent_batch<double>(c, nodes);

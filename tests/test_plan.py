@@ -14,6 +14,7 @@ MAXM = 43   # largest cube side the kernels take
 
 SRC = r"""
 #include "sq_plan.hpp"
+#include <chrono>
 #include <cstring>
 using namespace sqk;
 extern "C" {
@@ -59,6 +60,32 @@ int nlapply(int M, int max_nproj, int n_ip, int gl_max, long *out)
     out[0] = p.fits; out[1] = p.columns; out[2] = (long)p.lds;
     return 0;
 }
+int planes(int n, int z0, int nz, int *out)
+{
+    const std::vector<int> v = NodeOrder(n).planes(z0, nz);
+    std::memcpy(out, v.data(), v.size() * sizeof(int));
+    return (int)v.size();
+}
+void order(int n, int *nodes, int cnt)
+{
+    std::vector<int> v(nodes, nodes + cnt);
+    NodeOrder(n).sort(v);
+    std::memcpy(nodes, v.data(), v.size() * sizeof(int));
+}
+// seconds to order the whole grid, and to sort it by key
+void order_time(int n, double *out)
+{
+    auto now = [] { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); };
+    double t = now();
+    const std::vector<int> v = NodeOrder(n).planes(0, n);
+    out[0] = now() - t;
+    t = now();
+    const NodeOrder o(n);
+    std::vector<std::pair<unsigned long, int>> k(v.size());
+    for (size_t i = 0; i < k.size(); ++i) k[i] = {o.key((int)i), (int)i};
+    std::sort(k.begin(), k.end());
+    out[1] = now() - t;
+}
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -71,7 +98,7 @@ def plan(tmp_path_factory):
     d = tmp_path_factory.mktemp("plan")
     src, lib = d / "plan.cpp", d / "libplan.so"
     src.write_text(SRC)
-    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC, str(src), "-o",
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-fPIC", "-shared", "-I", CSRC, str(src), "-o",
                     str(lib)], check=True)
     d = C.CDLL(str(lib))
     d.noalloc_need.restype = d.noalloc_cap.restype = C.c_long
@@ -251,3 +278,43 @@ def test_nonlocal_rows_need_no_room_for_the_columns(plan, np_):
                 if out[0]:
                     assert rows + cols * out[1] <= out[2] <= LDS
                     assert out[1] or rows + cols + 4 * 49 > LDS
+
+
+def runs(n, length):
+    m = -(-n // length)
+    r = np.zeros(n, dtype=int)
+    for c in range(m):
+        r[c * n // m:(c + 1) * n // m] = c
+    return r
+
+
+def brick_key(n, nodes):
+    """Brick z, y, x of the even runs of up to 2, 4 and 4 nodes, then z, y, x."""
+    rx, ry, rz = runs(n, 4), runs(n, 2), runs(n, 2)
+    x, y, z = nodes % n, (nodes // n) % n, nodes // (n * n)
+    return np.lexsort((x, y, z, rx[x], ry[y] // 2, rz[z]))
+
+
+@pytest.mark.parametrize("n", list(range(1, 20)) + [25, 32])
+def test_nodes_are_visited_brick_by_brick(plan, n):
+    rng = np.random.Generator(np.random.PCG64(n))
+    for z0, nz in {(0, n), (0, 1), (n // 2, n - n // 2), (max(n - 2, 0), min(n, 2)), (n // 3, 1)}:
+        out = np.zeros(n ** 3, dtype=np.int32)
+        cnt = plan.planes(n, z0, nz, iptr(out))
+        ref = np.arange(z0 * n * n, (z0 + nz) * n * n)
+        assert cnt == ref.size and np.array_equal(out[:cnt], ref[brick_key(n, ref)])
+    for cnt in (0, 1, 2, n ** 3 // 20, n ** 3 // 2, 2 * n ** 3):     # with repeats
+        v = rng.integers(0, n ** 3, cnt).astype(np.int32)
+        ref = v[brick_key(n, v)]
+        plan.order(n, iptr(v), v.size)
+        assert np.array_equal(v, ref)
+
+
+def test_ordering_a_whole_grid_takes_no_sort(plan):
+    """96^3 nodes are ordered at every density step, while the GPU waits."""
+    t = (C.c_double * 2)()
+    best = [1e9, 1e9]
+    for _ in range(3):
+        plan.order_time(96, t)
+        best = [min(a, b) for a, b in zip(best, t)]
+    assert 3 * best[0] < best[1], best
