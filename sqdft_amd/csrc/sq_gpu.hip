@@ -361,11 +361,7 @@ void nlapply_go(sqg_ctx *c, int B, const NArgs<T> &A)
         auto fn = pl.columns ? (N.nl.ip16 ? k_nlapplyg<T, true, true> : k_nlapplyg<T, false, true>)
                              : (N.nl.ip16 ? k_nlapplyg<T, true, false> : k_nlapplyg<T, false, false>);
         if (pl.lds > 64 * 1024) (void)hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds);
-        // three workgroups share a CU: about eight rounds of them, so that the
-        // last one costs little, with at least four points a thread each
-        const int pts = (c->M + 3) * (c->M + 1) * c->M;
-        const int split = std::max(1, std::min(6144 / std::max(c->ng, 1), pts / (4 * 512)));
-        hipLaunchKernelGGL(fn, dim3(c->ng, split), dim3(512), pl.lds, c->st, N);
+        hipLaunchKernelGGL(fn, dim3(c->ng, nlapply_split(c->dims(), c->ng)), dim3(512), pl.lds, c->st, N);
         return;
     }
     const size_t shm = (size_t)std::max(c->n_ip, 1) * sizeof(double);

@@ -330,6 +330,18 @@ inline NlapplyPlan nlapply_plan(const ProjDims &d, int gl_max)
     return {base <= LDS_MAX, false, base};
 }
 
+// Workgroups that share a group's planes in k_nlapplyg, with at least four points a
+// thread each.  Three of them share a CU: about eight rounds for tables of one
+// projector, so that the last one costs little, four for several, whose rows every
+// share fills again.  us a pass with 8 and 4 rounds: 8,192 nodes with 35^3 Al cubes
+// 735 and 775; with 31^3 LiH cubes 912 and 858 (FP32 623 and 590), 4,096 of them 388
+// and 373.
+inline int nlapply_split(const ProjDims &d, int ng)
+{
+    const int pts = (d.M + 3) * (d.M + 1) * d.M, wgs = d.max_nproj > 1 ? 3072 : 6144;
+    return std::max(1, std::min(wgs / std::max(ng, 1), pts / (4 * 512)));
+}
+
 // Device bytes that a batch holds per node: nvec + 3 vectors of rs bytes per value
 // (the two Lanczos pairs and the nonlocal term, and what a pass adds), the
 // projections, the Lanczos tridiagonals with their scratch, and scalars ...

@@ -86,6 +86,7 @@ void order_time(int n, double *out)
     std::sort(k.begin(), k.end());
     out[1] = now() - t;
 }
+int nlapply_shares(int M, int max_nproj, int ng) { return nlapply_split({M, max_nproj, 100, 9}, ng); }
 int pad(int M) { return group_pad(M); }
 int range(int M) { return group_range(M); }
 int offset(int m, int M, int dx, int dy, int dz) { return member_offset(m, group_pad(M), M, M * M, M * M * M, dx, dy, dz); }
@@ -318,3 +319,14 @@ def test_ordering_a_whole_grid_takes_no_sort(plan):
         plan.order_time(96, t)
         best = [min(a, b) for a, b in zip(best, t)]
     assert 3 * best[0] < best[1], best
+
+
+def test_shares_of_the_nonlocal_apply(plan):
+    """Every share fills the rows again, three times as many for p projectors: fewer
+    shares there; at least four points a thread, at least one share."""
+    for M in range(3, MAXM + 1, 2):
+        for ng in (1, 7, 64, 480, 512, 1024, 4096, 100000):
+            s, p = plan.nlapply_shares(M, 1, ng), plan.nlapply_shares(M, 3, ng)
+            assert 1 <= p <= s <= max(1, (M + 3) * (M + 1) * M // 2048)
+            assert p * ng <= max(3072, ng) and s * ng <= max(6144, ng)
+    assert plan.nlapply_shares(35, 1, 1024) == 6 and plan.nlapply_shares(31, 3, 1024) == 3
