@@ -17,6 +17,7 @@
 #pragma once
 
 #include "sq_plan.hpp"
+#include "sq_sturm.hpp"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -1882,55 +1883,15 @@ __device__ int ql_extremes(double *d, double *e, int n, double *lmin, double *lm
 
 // 1/q to within an ulp or so: the hardware estimate and two Newton steps (a
 // correctly rounded division is a chain three times as long, and the Sturm
-// recurrences below are nothing but such chains).
-__device__ __forceinline__ double recip(double q)
-{
-    double r = __builtin_amdgcn_rcp(q);
-    r = fma(fma(-q, r, 1.0), r, r);
-    return fma(fma(-q, r, 1.0), r, r);
-}
-
-// Largest eigenvalue of the symmetric tridiagonal sg T (T: diagonal d(0..n-1),
-// off-diagonal e(0..n-2) through the accessors) by Newton's method on
-// det(xI - sg T).  With q_i = p_i/p_{i-1} (Sturm ratios) and r_i = q_i'/q_i,
-// p'/p = sum_i q_i'/q_i; past the largest root the characteristic polynomial
-// is monotone and convex, so iterates started outside the spectrum move
-// monotonically onto the root; the iteration stops at the first step that is
-// no longer inward by more than rounding.  A start x is outside iff every
-// q_i(x) > 0.  It first tries the near start b + g (just past the previous
-// pass's extreme, which the new one can only exceed), widening the gap 16-fold
-// per failed sweep, and falls back to the far start f (a Weyl bound, always
-// outside).  Returns false after 200 sweeps.
-template <typename D, typename E>
-__device__ bool tridiag_largest(D d, E e, int n, double sg, double f, double b, double g, double *out)
-{
-    bool probe = b + g < f;
-    double x = probe ? b + g : f;
-    for (int it = 0; it < 200; ++it) {
-        double q = x - sg * d(0), dq = 1.0, iq = recip(q), s = iq;
-        bool outside = q > 0.0;
-#pragma unroll 4
-        for (int i = 1; i < n; ++i) {
-            const double ei = e(i - 1), r = ei * ei * iq;
-            dq = 1.0 + r * dq * iq;
-            q = (x - sg * d(i)) - r;
-            outside = outside && q > 0.0;
-            iq = recip(q);
-            s += dq * iq;
-        }
-        if (probe && !outside) {
-            g *= 16.0;           // inside: widen, or take the far start
-            x = b + g;
-            if (!(x < f)) { x = f; probe = false; }
-            continue;
-        }
-        probe = false;
-        const double xn = x - recip(s);
-        if (!(xn < x - 2.0e-16 * fabs(x))) { *out = x; return true; }
-        x = xn;
+// recurrences of tridiag_largest are nothing but such chains).
+struct Recip {
+    __device__ __forceinline__ double operator()(double q) const
+    {
+        double r = __builtin_amdgcn_rcp(q);
+        r = fma(fma(-q, r, 1.0), r, r);
+        return fma(fma(-q, r, 1.0), r, r);
     }
-    return false;
-}
+};
 
 // Alpha and beta of a Lanczos pass and the extremes of the grown tridiagonal.
 // Two lanes per node, one per extreme, 32 nodes per wave; the tridiagonals'
@@ -1999,10 +1960,10 @@ __global__ void __launch_bounds__(2 * LQN) k_lanczos_scalars(QArgs A)
     bool ok;
     if (p < LQR) {
         sd[p][nb] = al;
-        ok = tridiag_largest([&](int i) { return sd[i][nb]; }, [&](int i) { return se[i][nb]; }, nq, sg, far, bx,
-                             gap, &x);
+        ok = tridiag_largest([&](int i) { return sd[i][nb]; }, [&](int i) { return se[i][nb]; }, Recip(), nq, sg,
+                             far, bx, gap, &x);
     } else {
-        ok = tridiag_largest(d, e, nq, sg, far, bx, gap, &x);
+        ok = tridiag_largest(d, e, Recip(), nq, sg, far, bx, gap, &x);
     }
     // lane pairs: (largest, smallest) to both
     const double mine = sg * x, other = __shfl_xor(mine, 1, 64);
