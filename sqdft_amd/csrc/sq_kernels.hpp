@@ -1384,7 +1384,7 @@ __global__ void __launch_bounds__(NT) k_projw(PArgs<T> A)
 // 879 us).  Before these changes against now, us a pass: 8,192 nodes with FP64
 // 35^3 cubes 888 and 732 (2.8 GB: 3.8 TB/s), 4,096 with FP32 ones 285 and 213,
 // 1,000 with FP64 17^3 cubes 34 and 24; 4,096 with 31^3 LiH ones (eight entries
-// a point: LDS rows) 386 and 387.
+// a point: LDS rows) 386 and 373.
 template <typename T>
 struct NGArgs {
     Geo g;

@@ -74,7 +74,7 @@ def lib(tmp_path_factory):
     src = d / "sturm.cpp"
     src.write_text(SRC)
     so = d / "libsturm.so"
-    subprocess.run(["g++", "-std=c++17", "-O2", "-mfma", "-ffp-contract=off", "-shared", "-fPIC", "-I", CSRC,
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-shared", "-fPIC", "-I", CSRC,
                     str(src), "-o", str(so)], check=True)
     L = C.CDLL(str(so))
     P, D, I = C.POINTER(C.c_double), C.c_double, C.c_int
